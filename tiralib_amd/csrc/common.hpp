@@ -49,6 +49,8 @@ enum Slot {
     WS_TABLE3, WS_PAY2, WS_PIPE0, WS_PIPE1, WS_SPEC0, WS_SPEC1, WS_THIN0, WS_THIN1,
     WS_NB2,  // the 2D neighbour table of the last stick/plate vote (kept while unchanged)
     WS_TABLE4,  // offset table of the tabulated-network vote
+    WS_TABLE5,  // offset tables of the listed plate gather
+    WS_LIST,    // its voter list, segment starts and tile flags
     WS_NSLOTS
 };
 int ws_get(int slot, size_t bytes, void** p);

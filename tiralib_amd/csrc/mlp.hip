@@ -817,6 +817,7 @@ static int mlp_build_vote_table(PlateMlp* m, hipStream_t st) {
         }
     } while (0);
     hipFree(drho); hipFree(X);
+    if (rc == TIRA_OK) m->vtab_custom = false;
     return rc;
 }
 
@@ -1218,6 +1219,7 @@ int tira_plate_mlp_set_vote_table(void* handle, const float* tab, size_t nfloats
     TH_ARG(nfloats == n, "vote table has %zu floats (got %zu)", n, nfloats);
     TH_HIP(hipStreamSynchronize(stream()));
     TH_HIP(hipMemcpy(m->vtab, tab, n * 4, hipMemcpyHostToDevice));
+    m->vtab_custom = true;
     m->version++;
     return TIRA_OK;
 }

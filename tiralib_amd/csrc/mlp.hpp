@@ -133,6 +133,7 @@ struct PlateMlp {
                                     // network evaluated per pair, then the tabulated network
     float4* vtab = nullptr;         // tabulated network, vtab_rows x kMlpTabM x 2 float4
     int vtab_rows = 0;
+    bool vtab_custom = false;       // the caller's table: its cell differences need not be those of its values
     std::vector<int> shells;        // squared distances of rows 1..K (mlp_shells)
     MlpAffine aff = {{0, 0, 0, 0, 0, 0}, {1, 1, 1, 1, 1, 1}};
     unsigned adam_t = 0;

@@ -25,7 +25,9 @@
 #include "common.hpp"
 #include "eig_device.hpp"
 #include "mlp.hpp"
+#include "plate_sparse.hpp"
 #include "vote3.hpp"
+#include "vote3_acc.hpp"
 #include "voxel_payload.hpp"
 
 #include <cmath>
@@ -64,7 +66,7 @@ float sticknorm3_host(float s1, float s2, unsigned p) {
 
 // Offset direction and attenuations exactly as cpu::build_neighbors3d
 // (tensorvote.h:1411-1436) computes them in float.
-static void offset_geometry(int du, int dv, int dw, float s1, float s2, float d[3], float& c1, float& c2) {
+void offset_geometry(int du, int dv, int dw, float s1, float s2, float d[3], float& c1, float& c2) {
     const float is1 = (s1 > 0) ? 1.0f / (s1 * s1) : 0.0f;
     const float is2 = (s2 > 0) ? 1.0f / (s2 * s2) : 0.0f;
     const float l2 = (float)(du * du + dv * dv + dw * dw);
@@ -217,10 +219,6 @@ void build_atv3_table(int w, float sigma, std::vector<float>& tab) {
 }
 
 // ---------------------------------------------------------------- device pair kernels
-struct Acc {
-    float xx, xy, xz, yy, yz, zz, ii;
-};
-
 template <int N>
 __device__ __forceinline__ float ipow(float x) {
     float r = x;
@@ -375,20 +373,6 @@ __device__ __forceinline__ void stick_pair_rt(Acc& a, const float4 S, const floa
     const float f0 = f * r0, f1 = f * r1, f2 = f * r2;
     a.xx = fmaf(f0, r0, a.xx); a.xy = fmaf(f0, r1, a.xy); a.xz = fmaf(f0, r2, a.xz);
     a.yy = fmaf(f1, r1, a.yy); a.yz = fmaf(f1, r2, a.yz); a.zz = fmaf(f2, r2, a.zz);
-}
-
-__device__ __forceinline__ void write_out(float* __restrict__ out, int layout, size_t v, const Acc& a,
-                                          bool add = false) {
-    const float xx = a.xx + a.ii, yy = a.yy + a.ii, zz = a.zz + a.ii;
-    if (layout == TIRA_LAYOUT_MAT9) {
-        float* o = out + v * 9;
-        const float t[9] = {xx, a.xy, a.xz, a.xy, yy, a.yz, a.xz, a.yz, zz};
-        for (int k = 0; k < 9; k++) o[k] = add ? o[k] + t[k] : t[k];
-    } else {
-        float* o = out + v * 6;
-        const float t[6] = {xx, a.xy, a.xz, yy, a.yz, zz};
-        for (int k = 0; k < 6; k++) o[k] = add ? o[k] + t[k] : t[k];
-    }
 }
 
 __device__ __forceinline__ void tile_coords(const VoteGeom& g, int bz_tile, unsigned& bx, unsigned& by,
@@ -685,15 +669,19 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
 // surrogate's error check -- their plate votes come from the integrator (the
 // closed form of the N-sample sum). Without pay_u (the tabulated network)
 // a flagged voter gets plate scale 0 in pay_n and its (n, scale) in pay_f,
-// which is zero for every other voter.
+// which is zero for every other voter. n_wild (optional) counts the voters
+// whose stick an FFT would spread beyond its window: not finite, or of a scale
+// whose sums could overflow.
+constexpr float kWildScale = 1e30f;
 __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict__ in, int layout, VoteGeom g,
                                                         float4* __restrict__ pay_s, float4* __restrict__ pay_n,
                                                         float4* __restrict__ pay_u, float4* __restrict__ pay_f,
                                                         const float* __restrict__ bin_err, float tol,
-                                                        unsigned long long* __restrict__ n_fallback) {
+                                                        unsigned long long* __restrict__ n_fallback,
+                                                        unsigned long long* __restrict__ n_wild) {
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
-    unsigned nf = 0;
+    unsigned nf = 0, wild = 0;
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
         const int px = (int)(p % g.P2), py = (int)((p / g.P2) % g.P1), pz = (int)(p / ((size_t)g.P1 * g.P2));
         const int x = px - g.r, y = py - g.r, z = pz - g.r;
@@ -707,7 +695,9 @@ __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict_
         const size_t v = ((size_t)z * g.s1 + y) * g.s2 + x;
         float l0, l1, l2, e0[3], e2[3];
         voxel_eig(in, layout, v, l0, l1, l2, e0, e2);
-        if (pay_s) pay_s[p] = make_float4(e2[0], e2[1], e2[2], copysignf(fabsf(l2) - fabsf(l1), l2));
+        const float ss = copysignf(fabsf(l2) - fabsf(l1), l2);
+        if (pay_s) pay_s[p] = make_float4(e2[0], e2[1], e2[2], ss);
+        wild += !(fabsf(ss) < kWildScale) || !isfinite(e2[0] + e2[1] + e2[2]) ? 1u : 0u;
         float n[3] = {e0[0], e0[1], e0[2]};
         const float nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
         float sp = copysignf(fabsf(l1) - fabsf(l0), l1);
@@ -728,6 +718,7 @@ __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict_
         }
     }
     if (n_fallback && nf) atomicAdd(n_fallback, (unsigned long long)nf);
+    if (n_wild && wild) atomicAdd(n_wild, (unsigned long long)wild);
 }
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -956,19 +947,22 @@ __global__ __launch_bounds__(kThreads) void k_vote3_mlp(const float4* __restrict
 // the offset's c1 / pi), so every pair reads its row from LDS. tab:
 // kMlpTabStride floats per offset (build_mlptab_table). Voters flagged by the
 // error check carry plate scale 0 here; their plates come from the
-// integrator's pass.
+// integrator's pass. listed (optional): tiles with a nonzero flag are left to
+// the listed gather (plate_sparse.hip); accumulate: add the votes to `out`.
 template <int P, bool STICK, int BZ>
 __global__ __launch_bounds__(kThreads) void k_vote3_mlptab(const float4* __restrict__ pay_s,
                                                            const float4* __restrict__ pay_p,
                                                            const float* __restrict__ tab,
                                                            const float4* __restrict__ vtab, int nrows,
-                                                           VoteGeom g, float* __restrict__ out, int out_layout) {
+                                                           VoteGeom g, float* __restrict__ out, int out_layout,
+                                                           const unsigned char* __restrict__ listed, int accumulate) {
     constexpr int STRIDE = kMlpTabStride;
     constexpr int C1PI = 8, ROW = 9;
     constexpr int CELLS2 = 2 * kMlpTabPad;  // float4 per staged row
     extern __shared__ float4 s_rows[];
     unsigned bx, by, bz;
     tile_coords_zfast(g, bx, by, bz);
+    if (listed && listed[(bz * g.nby + by) * g.nbx + bx]) return;
     const int x = (int)bx * kTileX + (int)(threadIdx.x % kTileX);
     const int y = (int)by * kTileY + (int)(threadIdx.x / kTileX);
     const int z0 = (int)bz * BZ;
@@ -1025,7 +1019,7 @@ __global__ __launch_bounds__(kThreads) void k_vote3_mlptab(const float4* __restr
 #pragma unroll
         for (int j = 0; j < BZ; j++) {
             const int z = z0 + j;
-            if (z < g.s0) write_out(out, out_layout, ((size_t)z * g.s1 + y) * g.s2 + x, acc[j]);
+            if (z < g.s0) write_out(out, out_layout, ((size_t)z * g.s1 + y) * g.s2 + x, acc[j], accumulate != 0);
         }
     }
 }
@@ -1530,13 +1524,15 @@ static int mlptab_lds_attr(size_t lds) {
 
 template <int P>
 static int launch_mlptab(bool stick, unsigned grid, size_t lds, hipStream_t st, const float4* ps, const float4* pn,
-                         const float* t, const float4* vt, int nrows, const VoteGeom& g, float* out, int layout) {
+                         const float* t, const float4* vt, int nrows, const VoteGeom& g, float* out, int layout,
+                         const unsigned char* listed, bool accumulate) {
+    const int acc = accumulate ? 1 : 0;
     if (stick) {
         TH_TRY((mlptab_lds_attr<P, true>(lds)));
-        k_vote3_mlptab<P, true, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout);
+        k_vote3_mlptab<P, true, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout, listed, acc);
     } else {
         TH_TRY((mlptab_lds_attr<P, false>(lds)));
-        k_vote3_mlptab<P, false, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout);
+        k_vote3_mlptab<P, false, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout, listed, acc);
     }
     return TIRA_OK;
 }
@@ -1566,16 +1562,17 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
     if (stick) TH_TRY(ws_get(WS_PAY0, ptotal * 16, (void**)&ps));
     TH_TRY(ws_get(WS_PAY1, ptotal * 16, (void**)&pn));
     TH_TRY(ws_get(WS_PAY2, ptotal * 16, table ? (void**)&pf : (void**)&pu));
-    unsigned long long* cnt = nullptr;
+    unsigned long long* cnt = nullptr;  // voters of the fallback, voters whose stick must stay local
     if (n_fallback || table) {
-        TH_TRY(ws_get(WS_COUNTER, 8, (void**)&cnt));
-        k_fill_zero<<<1, 64, 0, st>>>((float*)cnt, 2);
+        TH_TRY(ws_get(WS_COUNTER, 16, (void**)&cnt));
+        k_fill_zero<<<1, 64, 0, st>>>((float*)cnt, 4);
     }
     const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), 65536);
     {
         ProfScope prof("vote3_prep_mlp", st);
         k_vote3_prep_mlp<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pn, pu, pf,
-                                                table ? m->bin_err + kMlpBins : m->bin_err, tol, cnt);
+                                                table ? m->bin_err + kMlpBins : m->bin_err, tol, cnt,
+                                                table ? cnt + 1 : nullptr);
     }
     TH_HIP(hipGetLastError());
     const TableKey key{0, (int)w, m->sigma1, m->sigma2, m->power, 0u};
@@ -1590,13 +1587,39 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
         const size_t lds = (size_t)(w / 2 + 1) * 2 * kMlpTabPad * sizeof(float4);
         const float4* vt = m->vtab;
         const int nr = m->vtab_rows;
+        // The sticks, where the spectral vote serves them: they leave the
+        // window gather 36 of its 57 VALU instructions per pair, and the plates
+        // can then take the listed gather. Both add to the spectral output. A
+        // stick that is not finite stays within its window: the gather of the
+        // sticks overwrites the spectral ones if any voter is such.
+        bool spectral = false;
+        if (stick && spectral_preferred(s0, s1, s2, w, m->power, true, false, 0)) {
+            const int rc = vote3_spectral_run(tensors, in_layout, nullptr, nullptr, nullptr, out, out_layout, s0, s1, s2,
+                                              m->sigma1, m->sigma2, w, m->power, true, false, 0, false, st);
+            if (rc != TIRA_OK && rc != kSpectralNotApplicable) return rc;
+            spectral = rc == TIRA_OK;
+        }
+        if (spectral) {
+            ProfScope prof("vote3_mlp_wild", st);
+            switch (P) {
+                case 1: k_vote3_closed<1, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
+                case 2: k_vote3_closed<2, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
+                case 3: k_vote3_closed<3, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
+                default: k_vote3_closed<4, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
+            }
+            TH_HIP(hipGetLastError());
+        }
+        const bool gather_stick = stick && !spectral;
+        const unsigned char* listed = nullptr;
+        if (!gather_stick && !m->vtab_custom)
+            TH_TRY(plate_sparse_run(pn, vt, nr, m->sigma1, g, kBZMlp, out, out_layout, spectral, st, &listed));
         {
             ProfScope prof("vote3_mlptab", st);
             switch (P) {
-                case 1: TH_TRY(launch_mlptab<1>(stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout)); break;
-                case 2: TH_TRY(launch_mlptab<2>(stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout)); break;
-                case 3: TH_TRY(launch_mlptab<3>(stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout)); break;
-                default: TH_TRY(launch_mlptab<4>(stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout)); break;
+                case 1: TH_TRY(launch_mlptab<1>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
+                case 2: TH_TRY(launch_mlptab<2>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
+                case 3: TH_TRY(launch_mlptab<3>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
+                default: TH_TRY(launch_mlptab<4>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
             }
         }
         TH_HIP(hipGetLastError());
