@@ -48,14 +48,16 @@ typedef enum tira_status {
 
 /* Plate-vote evaluation for the 3D vote (samples > 0 is the reference's
  * numerically integrated plate, tensorvote.h:1651-1695 / 2457-2485). */
-#define TIRA_PLATE_AUTO    0   /* the spectral vote when it applies (power 1, samples 0 or >= 3, w >= 5, at
-                                  least 32^3 voxels, memory within 80% of the device); else the closed
+#define TIRA_PLATE_AUTO    0   /* the spectral vote when it applies (power 1 and w >= 5, 2 or 3 and
+                                  w >= 9, or 4 and w >= 11; samples 0 or >= power + 2; at least 32^3
+                                  voxels; memory within 80% of the device); else the closed
                                   form when samples >= power+2 (the Riemann sum is then exact), else the
                                   literal sum */
 #define TIRA_PLATE_SUM     1   /* literal N-sample Riemann sum, the reference's algorithm, any N */
 #define TIRA_PLATE_CLOSED  2   /* closed form of the same integral (exact for N >= p+2 and for samples == 0) */
 #define TIRA_PLATE_MLP     3   /* learned surrogate with per-voxel integrator fallback: served by tira_tensorvote3_mlp */
-#define TIRA_VOTE_SPECTRAL 4   /* stick + exact (closed-form) plate vote as an FFT convolution: power 1 and
+#define TIRA_VOTE_SPECTRAL 4   /* stick + exact (closed-form) plate vote as an FFT convolution (above power 1
+                                  where TIRA_PLATE_AUTO takes it): power 1 and
                                   samples == 0 or >= 3; other requests take the direct gather (AUTO) */
 
 /* eig3 flags */

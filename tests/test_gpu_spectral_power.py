@@ -1,0 +1,128 @@
+"""The spectral vote of powers 2 to 4 (28, 45, 66 features) against the window
+gather and, at one receiver set, the FP64 oracle: every combination of stick,
+plate, input and layout, sizes that are odd, ragged and larger than one row
+block, and the voters that have to be voted by window instead."""
+import numpy as np
+import pytest
+
+from tiralib_amd import _lib, api, synth
+
+pytestmark = pytest.mark.gpu
+SLOTS = [0, 1, 2, 4, 5, 8]
+
+
+def _field(shape, seed):
+    f = synth.tubes_sheets_volume(shape, n_straight=3, n_helix=2, n_sheets=2, seed=seed).reshape(shape + (9,))
+    rng = np.random.default_rng(seed)
+    a = rng.normal(size=shape + (3, 3)) * (rng.random(shape) < 0.05)[..., None, None]  # signed, all three eigenvalues
+    return np.ascontiguousarray(f + (a + a.swapaxes(-1, -2)).reshape(shape + (9,)), np.float32)
+
+
+def _run(f, shape, mode, sigma, sigma2, w, power, stick=True, plate=True, samples=20, out_layout=_lib.LAYOUT_MAT9):
+    d, o = _lib.DeviceArray.from_host(f), _lib.DeviceArray(shape + (9 if out_layout == _lib.LAYOUT_MAT9 else 6,))
+    try:
+        _lib.call("tira_hip_profile_begin")
+        api.tensorvote3_async(d, o, shape, sigma, sigma2, w, power, stick=stick, plate=plate, samples=samples,
+                              plate_mode=mode, out_layout=out_layout)
+        _lib.call("tira_hip_synchronize")
+        _lib.call("tira_hip_profile_end")
+        return o.to_host(), _lib.profile_get("spec_mul")[1]
+    finally:
+        d.free()
+        o.free()
+
+
+def _rel(a, b):
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("power", [2, 3, 4])
+@pytest.mark.parametrize("shape,w,stick,plate,samples,layout", [
+    ((32, 32, 32), 11, True, True, 20, _lib.LAYOUT_MAT9),
+    ((33, 41, 37), 11, True, False, 0, _lib.LAYOUT_PACKED6),
+    ((19, 50, 71), 13, False, True, 6, _lib.LAYOUT_MAT9),
+    ((3, 90, 129), 13, True, True, 0, _lib.LAYOUT_PACKED6),
+])
+def test_spectral_power_equals_gather(hip, power, shape, w, stick, plate, samples, layout):
+    f = _field(shape, seed=power)
+    got, n = _run(f, shape, _lib.PLATE_AUTO, 2.0, 1.0, w, power, stick, plate, samples, layout)
+    ref, m = _run(f, shape, _lib.PLATE_CLOSED, 2.0, 1.0, w, power, stick, plate, samples, layout)
+    assert (n, m) == (1, 0)
+    # either is within 1e-6 of 64 bits at these windows (5e-7 .. 1e-6 measured)
+    assert _rel(got, ref) <= 2e-6
+
+
+@pytest.mark.parametrize("power", [2, 3, 4])
+def test_spectral_power_vs_oracle(hip, oracle, power):
+    shape, w = (34, 32, 35), 11
+    f = _field(shape, seed=11)
+    rng = np.random.default_rng(1)
+    recv = np.sort(rng.choice(int(np.prod(shape)), 200, replace=False))
+    ref = oracle.tensorvote3_f64(f, 1.75, 0.5, power, w, samples=20, recv=recv, nthreads=8)[:, SLOTS]
+    got, n = _run(f, shape, _lib.PLATE_AUTO, 1.75, 0.5, w, power)
+    assert n == 1
+    assert _rel(got.reshape(-1, 9)[recv][:, SLOTS], ref) <= 4e-6  # sampled: four times the whole field's 1e-6
+
+
+@pytest.mark.parametrize("power,w,spectral", [(2, 7, 0), (2, 9, 1), (3, 9, 1), (4, 9, 0), (4, 11, 1), (5, 13, 0)])
+def test_spectral_power_rule(hip, power, w, spectral):
+    shape = (32, 32, 32)
+    f = _field(shape, seed=2)
+    for mode in (_lib.PLATE_AUTO, _lib.VOTE_SPECTRAL):
+        assert _run(f, shape, mode, 1.5, 0.0, w, power)[1] == spectral
+    assert _run(f, shape, _lib.PLATE_AUTO, 1.5, 0.0, w, power, samples=power + 1)[1] == 0  # not the exact integral
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 3e37])
+def test_wild_voter_is_voted_by_window(hip, bad):
+    """A voter that the transforms would spread or overflow leaves the gather's result."""
+    shape = (32, 36, 40)
+    f = _field(shape, seed=4)
+    f[12, 20, 17] = 0
+    f[12, 20, 17, 0] = bad
+    got, n = _run(f, shape, _lib.PLATE_AUTO, 1.5, 0.0, 9, 2)
+    ref, _ = _run(f, shape, _lib.PLATE_CLOSED, 1.5, 0.0, 9, 2)
+    assert n == 1
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+    inside = np.zeros(shape, bool)
+    inside[8:17, 16:25, 13:22] = True
+    assert np.isfinite(got[~inside]).all()
+    assert np.abs(got[~inside] - ref[~inside]).max() <= 1e-5 * np.abs(ref[~inside]).max()
+    a, b = got[inside], ref[inside]
+    ok = np.isfinite(b)
+    assert ok.sum() == 0 or np.abs(a[ok] - b[ok]).max() <= 1e-5 * np.abs(b[ok]).max()
+
+
+def test_stick_of_other_length_is_voted_by_window(hip):
+    """Eigenvectors handed in need not be of unit length: the vote takes them as they are."""
+    shape = (32, 33, 34)
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(5)
+    e = np.linalg.qr(rng.normal(size=(n, 3, 3)))[0].astype(np.float32)
+    lam = np.sort(rng.random((n, 3)), axis=1).astype(np.float32)
+    e2, e0 = np.ascontiguousarray(e[:, :, 0]), np.ascontiguousarray(e[:, :, 1])
+    out = {}
+    for name, scale in (("unit", 1.0), ("long", 1.5)):
+        for power in (2,):
+            out[name] = api.tensorvote3_tk(lam, e2 * np.float32(scale), e0, shape, 1.5, 0.0, power, 9, True, False, 20)
+    # (1 - t^2)^p of a longer vector is no multiple of the unit one's: check against one receiver in 64 bits
+    at, h = (16, 17, 18), 4
+    for name, scale in (("unit", 1.0), ("long", 1.5)):
+        V = np.zeros((3, 3))
+        q3 = (e2.reshape(shape + (3,)) * scale).astype(np.float64)
+        l3 = lam.reshape(shape + (3,)).astype(np.float64)
+        sn = 1 / (np.pi ** 1.5 / 2 * 1.5 ** 3 * 2 ** 5 * 4 / 120)
+        for dw in range(-h, h + 1):
+            for dv in range(-h, h + 1):
+                for du in range(-h, h + 1):
+                    l2 = du * du + dv * dv + dw * dw
+                    d = np.array([du, dv, dw]) / np.sqrt(l2) if l2 else np.zeros(3)
+                    i = (at[0] + dw, at[1] + dv, at[2] + du)
+                    q, s = q3[i], l3[i][2] - l3[i][1]
+                    t = q @ d
+                    eta = np.exp(-l2 / 1.5 ** 2) * (1 - t * t) ** 2 + (t ** 4 if l2 == 0 else 0)
+                    r = q - 2 * t * d
+                    V += sn * s * eta * np.outer(r, r)
+        g = out[name].reshape(shape + (3, 3))[at]
+        assert np.abs(g - V).max() <= 1e-5 * np.abs(V).max(), name

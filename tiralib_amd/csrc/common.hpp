@@ -50,7 +50,8 @@ enum Slot {
     WS_NB2,  // the 2D neighbour table of the last stick/plate vote (kept while unchanged)
     WS_TABLE4,  // offset table of the tabulated-network vote
     WS_TABLE5,  // offset tables of the listed plate gather
-    WS_LIST,    // its voter list, segment starts and tile flags
+    WS_WILD,    // flag of a spectral vote that has to be voted by window
+    WS_LIST,    // the listed gather's voter list, segment starts and tile flags
     WS_NSLOTS
 };
 int ws_get(int slot, size_t bytes, void** p);

@@ -20,6 +20,11 @@
 // The whole field's vote is a 15-in / 6-out correlation with a w^3 window:
 // O(N log N) through FFTs instead of O(N w^3) pair evaluations.
 //
+// Powers 2 to 4 are the same with degree g = 2 p + 2 (eta has degree 2 p):
+// (g + 1)(g + 2) / 2 = 28, 45 or 66 monomials. Their circle averages are
+// evaluated as the mean over p + 2 equispaced directions of the half circle,
+// which is exact for a trigonometric polynomial of degree g.
+//
 // Pipeline of one call (device buffers, zero padding to L >= n + w/2 per axis
 // so the circular convolution equals the reference's bounded window):
 //  1. payload: eigen-decomposition of every voxel, for eigenpair input only
@@ -64,17 +69,22 @@ constexpr size_t kColsLds = 40960;
 constexpr int kMaxL = 1024;    // longest transform
 constexpr int kMaxStages = 16;
 constexpr int kMono = 15;      // quartic monomials
+constexpr unsigned kSpecMaxPower = 4;
+constexpr float kSpecWild = 1e30f;  // features from here on could overflow the transforms
+// Monomials of the degree 2 p + 2 of a power-p vote.
+__host__ __device__ constexpr int mono_count(int power) { return (2 * power + 3) * (power + 2); }
+constexpr int kMaxMono = mono_count((int)kSpecMaxPower);
 
-// Exponents (a, b, c) of monomial m: a = 4..0, b = 4-a..0, c = 4-a-b.
-__host__ __device__ constexpr int mono_a(int m) {
-    return m < 1 ? 4 : m < 3 ? 3 : m < 6 ? 2 : m < 10 ? 1 : 0;
+// Exponents (a, b, c) of monomial m of degree g: a = g..0, b = g-a..0, c = g-a-b.
+__host__ __device__ constexpr int mono_k(int m) {  // g - a: the k with k (k + 1) / 2 <= m < (k + 1)(k + 2) / 2
+    int k = 0;
+    while ((k + 1) * (k + 2) / 2 <= m) k++;
+    return k;
 }
-__host__ __device__ constexpr int mono_b(int m) {
-    const int a = mono_a(m);
-    const int first = (4 - a) * (5 - a) / 2;  // index of (a, 4-a, 0)
-    return (4 - a) - (m - first);
-}
-__host__ __device__ constexpr int mono_c(int m) { return 4 - mono_a(m) - mono_b(m); }
+__host__ __device__ constexpr int mono_a(int m, int g = 4) { return g - mono_k(m); }
+__host__ __device__ constexpr int mono_c(int m) { return m - mono_k(m) * (mono_k(m) + 1) / 2; }
+__host__ __device__ constexpr int mono_b(int m) { return mono_k(m) - mono_c(m); }
+static_assert(mono_count(1) == kMono && mono_a(14) == 0 && mono_b(13) == 1 && mono_c(13) == 3, "monomial order");
 // Number of x / y / z indices in output component c (xx, xy, xz, yy, yz, zz).
 __host__ __device__ constexpr int comp_nx(int c) { return c == 0 ? 2 : (c == 1 || c == 2) ? 1 : 0; }
 __host__ __device__ constexpr int comp_ny(int c) { return c == 3 ? 2 : (c == 1 || c == 4) ? 1 : 0; }
@@ -722,13 +732,18 @@ struct SpecGeom {
     int n0, n1, n2;       // field (n2 fastest)
     int L0, L1, L2;       // FFT lengths
     int h0, h1, h2;       // octant extents L/2 + 1
-    int nf, nz;           // real features of the product (the 15 combined quartic features), complex channels
+    int nf, nz;           // real features of the product (the combined features), complex channels
+    int power;
     int stick, plate;     // which votes the features carry
     int atv;              // analytical tensor voting: s1 m(e2) + 2 s2 circle(e0) + 3 s3 sphere
     float alpha;          // scale of the plate part: sticknorm3 (vote) or 2 (ATV)
     int P2;               // row stride in complex values (L2 rounded up to 16)
     size_t cs;            // complex values per channel volume
     size_t ocs;           // kernel-spectrum values per channel (octant)
+    // parities of feature f along x and y: bit f, and bit f - 64 of the second word (held in
+    // scalar registers: a table read per feature made the product 2.5 us slower at 128^3)
+    unsigned long long odd_x, odd_y;
+    unsigned odd_x1, odd_y1;
 };
 
 // The 15 quartic monomials of (x, y, z) in the order of mono_a / mono_b,
@@ -772,6 +787,62 @@ __device__ __forceinline__ void add_circle_average(const float4 N, float* __rest
     for (int i = 0; i < 42; i++) A[t[i].f] = fmaf(t[i].a, B[t[i].g], A[t[i].f]);
 }
 
+// The monomials of degree 2 P + 2 of (x, y, z) times w, added to A.
+template <int P>
+__device__ __forceinline__ void add_mono(float x, float y, float z, float w, float* __restrict__ A) {
+    constexpr int G = 2 * P + 2;
+    float px[G + 1], py[G + 1], pz[G + 1];
+    px[0] = w;
+    py[0] = pz[0] = 1.0f;
+#pragma unroll
+    for (int i = 1; i <= G; i++) {
+        px[i] = px[i - 1] * x;
+        py[i] = py[i - 1] * y;
+        pz[i] = pz[i - 1] * z;
+    }
+    int m = 0;
+#pragma unroll
+    for (int k = 0; k <= G; k++)
+#pragma unroll
+        for (int c = 0; c <= k; c++, m++) A[m] = fmaf(px[G - k], py[k - c] * pz[c], A[m]);
+}
+
+// Features of a power-P voter: the stick's monomials, and the plate's as the
+// mean of the stick's over the half circle perpendicular to n (P + 2
+// equispaced directions; N.w carries the plate's scale and sticknorm3).
+template <int P>
+__device__ __forceinline__ void voter_features(const float4 S, const float4 N, bool stick, bool plate,
+                                               float* __restrict__ A) {
+#pragma unroll
+    for (int m = 0; m < mono_count(P); m++) A[m] = 0.0f;
+    if (stick) add_mono<P>(S.x, S.y, S.z, S.w, A);
+    if (plate) {
+        // u, v span the plane: u = a x n for the axis a of the smaller |n_a|
+        const bool ax = fabsf(N.x) < fabsf(N.z);
+        float u0 = ax ? 0.0f : N.y, u1 = ax ? -N.z : -N.x, u2 = ax ? N.y : 0.0f;
+        const float il = rsqrtf(fmaf(u0, u0, fmaf(u1, u1, u2 * u2)));
+        const bool ok = N.w != 0.0f;  // a voter without a plate may carry no normal
+        u0 = ok ? u0 * il : 0.0f;
+        u1 = ok ? u1 * il : 0.0f;
+        u2 = ok ? u2 * il : 0.0f;
+        const float v0 = N.y * u2 - N.z * u1, v1 = N.z * u0 - N.x * u2, v2 = N.x * u1 - N.y * u0;
+        const float w = N.w * (1.0f / (P + 2));
+        constexpr float cs[3][6] = {{1.0f, 0.707106781186547524f, 0.0f, -0.707106781186547524f, 0.0f, 0.0f},
+                                    {1.0f, 0.809016994374947424f, 0.309016994374947424f, -0.309016994374947424f,
+                                     -0.809016994374947424f, 0.0f},
+                                    {1.0f, 0.866025403784438647f, 0.5f, 0.0f, -0.5f, -0.866025403784438647f}};
+        constexpr float sn[3][6] = {{0.0f, 0.707106781186547524f, 1.0f, 0.707106781186547524f, 0.0f, 0.0f},
+                                    {0.0f, 0.587785252292473129f, 0.951056516295153572f, 0.951056516295153572f,
+                                     0.587785252292473129f, 0.0f},
+                                    {0.0f, 0.5f, 0.866025403784438647f, 1.0f, 0.866025403784438647f, 0.5f}};
+#pragma unroll
+        for (int i = 0; i < P + 2; i++) {
+            const float c = cs[P - 2][i], t = sn[P - 2][i];
+            add_mono<P>(fmaf(c, u0, t * v0), fmaf(c, u1, t * v1), fmaf(c, u2, t * v2), w, A);
+        }
+    }
+}
+
 // Forward x pass fused with the features. A block takes B rows (z, y) of the
 // field and the complex channels in groups of C (all of them unless a row's
 // lines exceed 64 KB of LDS): every element computes all features of its
@@ -784,11 +855,14 @@ __device__ __forceinline__ void add_circle_average(const float4 N, float* __rest
 // voxel).
 // Four waves per SIMD (at most 128 VGPRs): unbounded, the eigen-solve and the
 // features take 136 and three waves; bounded, they fit in 120 without a spill.
-template <bool FROM_TENSORS>
-__global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__ ps, const float4* __restrict__ pp,
-                                                   const float* __restrict__ tensors, int layout, SpecGeom g, int B,
-                                                   int C, int FG, FftPlan pl, const float2* __restrict__ twg,
-                                                   float2* __restrict__ Z) {
+// wild (power above 1): set when a feature is not finite or so large that the
+// transforms' sums could overflow, for the caller to vote by window instead.
+template <bool FROM_TENSORS, int P>
+__global__ __launch_bounds__(kFT, P == 1 ? 4 : 2) void k_spec_xfwd(
+    const float4* __restrict__ ps, const float4* __restrict__ pp, const float* __restrict__ tensors, int layout,
+    SpecGeom g, int B, int C, int FG, FftPlan pl, const float2* __restrict__ twg, float2* __restrict__ Z,
+    unsigned long long* __restrict__ wild) {
+    constexpr int NF = mono_count(P);
     extern __shared__ float2 xs_dyn[];  // C B L staged values, then L twiddles
     const int L = pl.L;
     float2* s = xs_dyn;
@@ -817,8 +891,7 @@ __global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__
             // part); the stick features are written first, zero when the vote
             // has no stick part (zeroing A ahead of the eigen-solve kept 15
             // registers live through it and spilled 80 bytes per lane)
-            float A[kMono + 1];
-            A[kMono] = 0.0f;
+            float A[(NF + 2) & ~1];
             {
                 const size_t vox = (size_t)(row0 + b) * g.n2 + e;
                 float4 S = make_float4(0.0f, 0.0f, 0.0f, 0.0f), N = S;
@@ -837,9 +910,25 @@ __global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__
                     if (g.stick) S = ps[vox];
                     if (g.plate) N = pp[vox];
                 }
-                mono15(g.stick ? S : make_float4(0.0f, 0.0f, 0.0f, 0.0f), A);
-                if (g.plate) add_circle_average(make_float4(N.x, N.y, N.z, N.w * g.alpha), A);
-                if (g.atv) {  // three times the sphere averages: 1/5 for x^4, 1/15 for x^2 y^2
+                if (P > 1) {
+                    voter_features<(P > 1 ? P : 2)>(S, make_float4(N.x, N.y, N.z, N.w * g.alpha), g.stick != 0,
+                                                    g.plate != 0, A);
+                    if (NF & 1) A[NF] = 0.0f;
+                    float big = 0.0f;
+#pragma unroll
+                    for (int m = 0; m < NF; m++) big = fmaxf(big, fabsf(A[m]));
+                    // fmaxf drops NaN: a NaN feature shows in the sum of squares of the voter
+                    const float nan = fmaf(S.w, S.x + S.y + S.z, N.w * (N.x + N.y + N.z));
+                    // the features take a stick of unit length (a caller's eigenvectors need not be)
+                    const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
+                    const bool odd = g.stick && S.w != 0.0f && !(fabsf(q2 - 1.0f) < 2e-6f);
+                    if (wild && (!(big < kSpecWild) || nan != nan || odd)) atomicAdd(wild, 1ull);
+                } else {
+                    mono15(g.stick ? S : make_float4(0.0f, 0.0f, 0.0f, 0.0f), A);
+                    A[NF] = 0.0f;
+                    if (g.plate) add_circle_average(make_float4(N.x, N.y, N.z, N.w * g.alpha), A);
+                }
+                if (P == 1 && g.atv) {  // three times the sphere averages: 1/5 for x^4, 1/15 for x^2 y^2
                     A[0] = fmaf(0.6f, s3, A[0]);
                     A[3] = fmaf(0.2f, s3, A[3]);
                     A[5] = fmaf(0.2f, s3, A[5]);
@@ -849,7 +938,7 @@ __global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__
                 }
             }
 #pragma unroll
-            for (int j = 0; j < (kMono + 1) / 2; j++)
+            for (int j = 0; j < (NF + 1) / 2; j++)
                 if (j >= j0 && j < j0 + Cv) s[((j - j0) * Bv + b) * L + e] = make_float2(A[2 * j], A[2 * j + 1]);
         }
         __syncthreads();
@@ -913,8 +1002,8 @@ __global__ __launch_bounds__(256) void k_spec_mul(float2* __restrict__ Z, const 
         for (int h = 0; h < 2; h++) {
             const int f = 2 * j + h;
             if (f >= g.nf) break;
-            const int m = f % kMono;  // the constant feature (ATV) shares x^4's parities (all even)
-            const int am = mono_a(m), bm = mono_b(m);
+            const int odx = f < 64 ? (int)(g.odd_x >> f) : (int)(g.odd_x1 >> (f - 64));
+            const int ody = f < 64 ? (int)(g.odd_y >> f) : (int)(g.odd_y1 >> (f - 64));
             float2 F[4];
 #pragma unroll
             for (int sl = 0; sl < 4; sl++) {
@@ -924,7 +1013,7 @@ __global__ __launch_bounds__(256) void k_spec_mul(float2* __restrict__ Z, const 
 #pragma unroll
             for (int c = 0; c < 6; c++) {
                 const float k = Kh[(size_t)(c * g.nf + f) * g.ocs + gid];
-                const bool ox = ((comp_nx(c) + am) & 1) != 0, oy = ((comp_ny(c) + bm) & 1) != 0;
+                const bool ox = ((comp_nx(c) + odx) & 1) != 0, oy = ((comp_ny(c) + ody) & 1) != 0;
                 const float k1 = ox ? -k : k, k2 = oy ? -k : k, k3 = (ox != oy) ? -k : k;
                 Y[0][c].x = fmaf(k, F[0].x, Y[0][c].x);  Y[0][c].y = fmaf(k, F[0].y, Y[0][c].y);
                 Y[1][c].x = fmaf(k1, F[1].x, Y[1][c].x); Y[1][c].y = fmaf(k1, F[1].y, Y[1][c].y);
@@ -1047,9 +1136,9 @@ __global__ __launch_bounds__(256) void k_khat_z(const double* __restrict__ T2, c
     }
 }
 
-// ---------------------------------------------------------------- host: offset kernels
+// ---------------------------------------------------------------- offset kernels
 // Fibonacci points on the unit sphere; the monomial matrix at these points
-// has full rank 15 (even polynomials of degree <= 4 restricted to the sphere).
+// has full rank (even polynomials of degree <= g restricted to the sphere).
 static void fit_points(std::vector<double>& Q, int npts) {
     Q.resize((size_t)npts * 3);
     const double ga = M_PI * (3.0 - std::sqrt(5.0));
@@ -1062,15 +1151,16 @@ static void fit_points(std::vector<double>& Q, int npts) {
     }
 }
 
-static double mono_eval(const double* q, int m) {
-    return std::pow(q[0], mono_a(m)) * std::pow(q[1], mono_b(m)) * std::pow(q[2], mono_c(m));
+static double mono_eval(const double* q, int m, int g) {
+    return std::pow(q[0], mono_a(m, g)) * std::pow(q[1], mono_b(m)) * std::pow(q[2], mono_c(m));
 }
 
-// Least-squares projector P (15 x npts): coefficients = P * values.
-static bool fit_projector(const std::vector<double>& Q, int npts, std::vector<double>& P) {
+// Least-squares projector P (mono_count(power) x npts): coefficients = P * values.
+static bool fit_projector(const std::vector<double>& Q, int npts, std::vector<double>& P, int power = 1) {
+    const int kMono = mono_count(power), g = 2 * power + 2;
     std::vector<double> A((size_t)npts * kMono), N(kMono * 2 * kMono, 0.0);
     for (int i = 0; i < npts; i++)
-        for (int m = 0; m < kMono; m++) A[(size_t)i * kMono + m] = mono_eval(&Q[i * 3], m);
+        for (int m = 0; m < kMono; m++) A[(size_t)i * kMono + m] = mono_eval(&Q[i * 3], m, g);
     // [A^T A | I] -> [I | (A^T A)^-1], Gauss-Jordan with partial pivoting.
     for (int r = 0; r < kMono; r++) {
         for (int c = 0; c < kMono; c++) {
@@ -1106,7 +1196,7 @@ static bool fit_projector(const std::vector<double>& Q, int npts, std::vector<do
     return true;
 }
 
-static void sym_add(double V[6], double f, const double a[3], const double b[3]) {  // f (a b^T + b a^T) / 2
+__host__ __device__ static inline void sym_add(double V[6], double f, const double a[3], const double b[3]) {  // f (a b^T + b a^T) / 2
     V[0] += f * a[0] * b[0];
     V[1] += 0.5 * f * (a[0] * b[1] + a[1] * b[0]);
     V[2] += 0.5 * f * (a[0] * b[2] + a[2] * b[0]);
@@ -1116,11 +1206,14 @@ static void sym_add(double V[6], double f, const double a[3], const double b[3])
 }
 
 // Pair votes (FP64) of a unit voter vector q at unit offset d (d = 0 at the
-// voter itself), attenuations c1, c2, power 1, normalised as the gather path
+// voter itself), attenuations c1, c2, normalised as the gather path
 // normalises them (1 / sticknorm3, 1 / pi).
-static void stick_vote64(const double q[3], const double d[3], double c1, double c2, double sn, double V[6]) {
+__host__ __device__ static inline void stick_vote64(const double q[3], const double d[3], double c1, double c2,
+                                                    double sn, double V[6], int power = 1) {
     const double t = q[0] * d[0] + q[1] * d[1] + q[2] * d[2];
-    const double eta = c1 * (1.0 - t * t) + c2 * t * t;
+    double e1 = 1.0 - t * t, e2 = t * t;
+    for (int i = 1; i < power; i++) { e1 *= 1.0 - t * t; e2 *= t * t; }
+    const double eta = c1 * e1 + c2 * e2;
     const double r[3] = {q[0] - 2 * t * d[0], q[1] - 2 * t * d[1], q[2] - 2 * t * d[2]};
     for (int k = 0; k < 6; k++) V[k] = 0.0;
     sym_add(V, eta * sn, r, r);
@@ -1152,7 +1245,7 @@ static void plate_vote64(const double n[3], const double d[3], bool self, const 
 // (l2 - l1, l1 - l0, l0), eigenvectors e0, e2, unit offset v (rho = 1) or the
 // voter itself (v = 0, rho = 0), attenuation c:
 //   KI I + K00 e0 e0^T + K22 e2 e2^T + Kvv v v^T + K0 (v e0^T + e0 v^T) + K2 (v e2^T + e2 v^T).
-static void atv_vote64(const double e0[3], const double e2[3], const double v[3], double rho, double c, double s1,
+__host__ __device__ static inline void atv_vote64(const double e0[3], const double e2[3], const double v[3], double rho, double c, double s1,
                        double s2, double s3, double V[6]) {
     const double a = e2[0] * v[0] + e2[1] * v[1] + e2[2] * v[2];
     const double b = e0[0] * v[0] + e0[1] * v[1] + e0[2] * v[2];
@@ -1172,7 +1265,40 @@ static void atv_vote64(const double e0[3], const double e2[3], const double v[3]
     sym_add(V, 2.0 * K2, v, e2);
 }
 
-// K[ch][dw][dv][du], ch = c * nf + f (see tira_spectral_offset_kernels). With
+// The offset kernels of the combined features on the device: coefficients of
+// the stick vote (ATV: of its e2 part) of every offset, K[c nf + f][dw][dv][du],
+// from its values at the fit points Q by the projector P (nf x npts). One
+// thread per (offset, feature); the votes are evaluated again by each feature,
+// which costs less than keeping them. 2197 offsets of the 15 quartic features:
+// 18 us, 29 us for the 28 of power 2 (the loop on the host grows with the
+// square of the features: 0.3 s for power 4 at w = 13).
+__global__ __launch_bounds__(256) void k_offset_kernels(int r, double s1, double s2, int power, int atv, double sn,
+                                                        const double* __restrict__ Q, const double* __restrict__ P,
+                                                        int npts, int nf, double* __restrict__ K) {
+    const int W = 2 * r + 1;
+    const size_t noff = (size_t)W * W * W, i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= noff * nf) return;
+    const int f = (int)(i / noff);
+    const size_t o = i - (size_t)f * noff;
+    const int du = (int)(o % W) - r, dv = (int)((o / W) % W) - r, dw = (int)(o / ((size_t)W * W)) - r;
+    const double l2 = (double)du * du + (double)dv * dv + (double)dw * dw;
+    double d[3] = {0.0, 0.0, 0.0};
+    if (l2 > 0) { const double L = sqrt(l2); d[0] = du / L; d[1] = dv / L; d[2] = dw / L; }
+    const double c1 = s1 > 0 ? exp(-l2 / (s1 * s1)) : (l2 > 0 ? 0.0 : 1.0);
+    const double c2 = s2 > 0 ? exp(-l2 / (s2 * s2)) : (l2 > 0 ? 0.0 : 1.0);
+    const double zero[3] = {0.0, 0.0, 0.0};
+    double acc[6] = {0, 0, 0, 0, 0, 0};
+    for (int k = 0; k < npts; k++) {
+        double V[6];
+        if (atv) atv_vote64(zero, Q + 3 * k, d, l2 > 0 ? 1.0 : 0.0, c1, 1.0, 0.0, 0.0, V);
+        else stick_vote64(Q + 3 * k, d, c1, c2, sn, V, power);
+        const double p = P[(size_t)f * npts + k];
+        for (int c = 0; c < 6; c++) acc[c] = fma(p, V[c], acc[c]);
+    }
+    for (int c = 0; c < 6; c++) K[((size_t)c * nf + f) * noff + o] = acc[c];
+}
+
+// K[ch][dw][dv][du], ch = c * nf + f (see tira_spectral_offset_kernels), on the host. With
 // `atv`, the features are s1 m(e2) (15), s2 m(e0) (15) and s3 (1), the window
 // half-width w / 2 and the attenuation exp(-|d|^2 / s1^2) of ATV.
 static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate, bool atv, std::vector<double>& K,
@@ -1247,10 +1373,10 @@ static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate
 struct SpecKey {
     int L0, L1, L2, w;
     float s1, s2;
-    int stick, plate, atv;
+    int power, atv;
     bool operator==(const SpecKey& o) const {
         return L0 == o.L0 && L1 == o.L1 && L2 == o.L2 && w == o.w && s1 == o.s1 && s2 == o.s2 &&
-               stick == o.stick && plate == o.plate && atv == o.atv;
+               power == o.power && atv == o.atv;
     }
 };
 
@@ -1258,7 +1384,7 @@ struct SpecKey {
 // caller alternating between shapes or scales rebuilds nothing), evicted
 // least recently used beyond kSpecEntries or 1/8 of the device's memory.
 struct SpecEntry {
-    SpecKey key{0, 0, 0, 0, 0, 0, 0, 0, 0};
+    SpecKey key{0, 0, 0, 0, 0, 0, 0, 0};
     int device = -1;
     void* buf = nullptr;  // twiddles (3 axes) then the octant spectra
     size_t bytes = 0;
@@ -1383,29 +1509,23 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
         twiddles(key.L2, t.data() + (tw_bytes(key.L0) + tw_bytes(key.L1)) / 8);
         TH_HIP(hipMemcpy(ent.buf, t.data(), tb, hipMemcpyHostToDevice));
     }
-    // offset kernels, parities and trig tables
-    std::vector<double> K;
-    int nf = 0;
-    // the stick (ATV: e2) part only: the plate part, and the ATV's e0 and
-    // constant parts, are linear maps of it and fold into the features
-    TH_TRY(offset_kernels((unsigned)key.w, key.s1, key.s2, true, false, key.atv != 0, K, nf));
-    if (nf > kMono) {  // ATV: keep the first 15 features of every component
-        const size_t noff = K.size() / ((size_t)6 * nf);
-        std::vector<double> K15((size_t)6 * kMono * noff);
-        for (int c = 0; c < 6; c++)
-            std::copy(K.begin() + (size_t)c * nf * noff, K.begin() + ((size_t)c * nf + kMono) * noff,
-                      K15.begin() + (size_t)c * kMono * noff);
-        K.swap(K15);
-        nf = kMono;
+    // offset kernels (the stick's, or the ATV's e2 part, only: the plate part,
+    // and the ATV's e0 and constant parts, are linear maps of it and fold into
+    // the features), parities and trig tables
+    const int w = 2 * (key.w / 2) + 1, r = key.w / 2, nf = g.nf;
+    const int nch = 6 * nf, npts = std::max(32, 3 * nf);
+    std::vector<double> Q, P;
+    fit_points(Q, npts);
+    if (!fit_projector(Q, npts, P, key.power)) {
+        set_error("spectral vote: degenerate fitting points (internal error)");
+        return TIRA_ERR_INVALID_ARG;
     }
-    const int w = 2 * (key.w / 2) + 1, r = key.w / 2;
-    const int nch = 6 * nf;
     std::vector<unsigned char> par(nch);
     for (int c = 0; c < 6; c++)
         for (int f = 0; f < nf; f++) {
-            const int m = f % kMono;
-            par[c * nf + f] = (unsigned char)(((comp_nx(c) + mono_a(m)) & 1) | (((comp_ny(c) + mono_b(m)) & 1) << 1) |
-                                              (((comp_nz(c) + mono_c(m)) & 1) << 2));
+            const int ga = 2 * key.power + 2;
+            par[c * nf + f] = (unsigned char)(((comp_nx(c) + mono_a(f, ga)) & 1) | (((comp_ny(c) + mono_b(f)) & 1) << 1) |
+                                              (((comp_nz(c) + mono_c(f)) & 1) << 2));
         }
     const int hs[3] = {g.h0, g.h1, g.h2}, Ls[3] = {g.L0, g.L1, g.L2};
     std::vector<double> trig[3];
@@ -1420,7 +1540,8 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
     }
     const size_t t1n = (size_t)nch * w * w * g.h2, t2n = (size_t)nch * w * g.h1 * g.h2;
     const size_t trig_n = trig[0].size() + trig[1].size() + trig[2].size();
-    const size_t tmp_bytes = (K.size() + t1n + t2n + trig_n) * 8 + nch + 256;
+    const size_t noff = (size_t)w * w * w, kn = (size_t)nch * noff;
+    const size_t tmp_bytes = (kn + t1n + t2n + trig_n + Q.size() + P.size()) * 8 + nch + 256;
     char* tmp = nullptr;
     if (hipMalloc((void**)&tmp, tmp_bytes) != hipSuccess) {
         (void)hipGetLastError();
@@ -1428,22 +1549,27 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
         return TIRA_ERR_OUT_OF_MEMORY;
     }
     double* dK = (double*)tmp;
-    double* dT1 = dK + K.size();
+    double* dT1 = dK + kn;
     double* dT2 = dT1 + t1n;
     double* dtr[3];
     dtr[0] = dT2 + t2n;
     dtr[1] = dtr[0] + trig[0].size();
     dtr[2] = dtr[1] + trig[1].size();
-    unsigned char* dpar = (unsigned char*)(dtr[2] + trig[2].size());
+    double* dQ = dtr[2] + trig[2].size();
+    double* dP = dQ + Q.size();
+    unsigned char* dpar = (unsigned char*)(dP + P.size());
     int rc = TIRA_OK;
     do {
-        if (hipMemcpy(dK, K.data(), K.size() * 8, hipMemcpyHostToDevice) != hipSuccess) { rc = -2; break; }
-        bool ok = true;
+        bool ok = hipMemcpy(dQ, Q.data(), Q.size() * 8, hipMemcpyHostToDevice) == hipSuccess &&
+                  hipMemcpy(dP, P.data(), P.size() * 8, hipMemcpyHostToDevice) == hipSuccess;
         for (int a = 0; a < 3; a++)
             ok = ok && hipMemcpy(dtr[a], trig[a].data(), trig[a].size() * 8, hipMemcpyHostToDevice) == hipSuccess;
         ok = ok && hipMemcpy(dpar, par.data(), nch, hipMemcpyHostToDevice) == hipSuccess;
         if (!ok) { rc = -2; break; }
         auto grid = [](size_t n) { return (unsigned)std::min<size_t>(ceil_div(n, 256), 65536); };
+        const double sn = key.atv ? 1.0 : 1.0 / (double)sticknorm3_host(key.s1, key.s2, (unsigned)key.power);
+        k_offset_kernels<<<ceil_div(noff * nf, 256), 256, 0, st>>>(r, key.s1, key.s2, key.power, key.atv, sn, dQ, dP,
+                                                                   npts, nf, dK);
         k_khat_x<<<grid(t1n), 256, 0, st>>>(dK, dtr[2], dpar, dT1, w, g.h2, nch);
         k_khat_y<<<grid(t2n), 256, 0, st>>>(dT1, dtr[1], dpar, dT2, w, g.h1, g.h2, nch);
         const double scale = 0.5 / ((double)g.L0 * g.L1 * g.L2);
@@ -1512,21 +1638,35 @@ static LineGeom strided_geom(size_t cs, int nchan, int L, size_t estride, int na
     return g;
 }
 
-// Whether TIRA_PLATE_AUTO takes the spectral vote: power 1, an exact plate
-// (samples 0 or >= 3), FFT lengths within range, a window of at least 5 and
-// a volume of at least 32^3 voxels (below that the gather costs microseconds
-// and the first call's spectra build would dominate), and device memory for
-// the spectra, their build and the feature volumes within 80% of the device.
-// With `atv`: analytical tensor voting (31 features, 16 complex channels),
-// whose features come from the input tensors in the x pass only.
+// Powers and plates the spectral vote serves: power 1 to 4, a plate that is
+// the exact circle integral (samples 0 or >= power + 2).
+static bool spectral_serves(unsigned p, bool plate, unsigned samples) {
+    return p <= kSpecMaxPower && !(plate && samples > 0 && samples < p + 2);
+}
+
+// Whether TIRA_PLATE_AUTO takes the spectral vote: a power and a plate that it
+// serves, FFT lengths within range, a window of at least 5 (power 1), 9 (2 and
+// 3) or 11 (4) and a volume of at least 32^3 voxels (below that the gather
+// costs microseconds and the first call's spectra build would dominate), and
+// device memory for the spectra, their build and the feature volumes within
+// 80% of the device.
+// Above power 1 the features are more (28, 45, 66 for 15) and the line lies
+// where neither time nor error against 64 bits is worse than the gather's,
+// measured from 32^3 to 128^3: power 2 at w = 9 takes 69 us for 718 us (32^3)
+// and 555 for 2296 (128^3) at 5e-7 for 4.6e-7, power 3 931 for 2575 (128^3) at
+// 4.8e-7 for 5e-7; power 2 at w = 13 549 for 6598 us (128^3) at 5.2e-7 for
+// 6.3e-7, power 4 1329 for 7195 us at 7.3e-7 for 7.7e-7. At w = 7 the gather's
+// error is the smaller (3.3e-7 for 5e-7), at w = 5 its time too.
+// With `atv`: analytical tensor voting, whose features come from the input
+// tensors in the x pass only.
 bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsigned power, bool stick, bool plate,
                         unsigned samples, bool atv) {
-    const unsigned p = power < 1 ? 1 : power;
-    if (!atv && (p != 1 || (plate && samples > 0 && samples < 3))) return false;
-    if (w < 5 || (size_t)s0 * s1 * s2 < 32768) return false;
+    const unsigned p = power < 1 || atv ? 1 : power;
+    if (!atv && !spectral_serves(p, plate, samples)) return false;
+    if (w < (p == 1 ? 5u : p < 4 ? 9u : 11u) || (size_t)s0 * s1 * s2 < 32768) return false;
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);
     if (!L0 || !L1 || !L2 || 3 * L2 > (unsigned)kFftBL) return false;
-    const size_t nf = kMono, nz = (nf + 1) / 2;  // the combined features
+    const size_t nf = (size_t)mono_count((int)p), nz = (nf + 1) / 2;  // the combined features
     const size_t W = 2 * (w / 2) + 1;
     const size_t h0 = L0 / 2 + 1, h1 = L1 / 2 + 1, h2 = L2 / 2 + 1;
     const size_t need = nz * (size_t)L0 * L1 * L2 * 8 + 6 * nf * h0 * h1 * h2 * 4 + 6 * nf * W * h1 * h2 * 8 +
@@ -1543,16 +1683,28 @@ bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsig
     return need <= total_b / 10 * 8 && need <= (free_b + held) / 10 * 9;
 }
 
+template <bool FROM_TENSORS>
+static void launch_xfwd(int power, unsigned grid, size_t lds, hipStream_t st, const float4* ps, const float4* pp,
+                        const float* tensors, int layout, const SpecGeom& g, int B, int C, int FG, const FftPlan& pl,
+                        const float2* tw, float2* Z, unsigned long long* wild) {
+    switch (power) {
+        case 1: k_spec_xfwd<FROM_TENSORS, 1><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
+        case 2: k_spec_xfwd<FROM_TENSORS, 2><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
+        case 3: k_spec_xfwd<FROM_TENSORS, 3><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
+        default: k_spec_xfwd<FROM_TENSORS, 4><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
+    }
+}
+
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        float* out, int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1,
                        float sigma2, unsigned w, unsigned power, bool stick, bool plate, unsigned samples,
-                       bool atv, hipStream_t st, EigOut* eig) {
-    const unsigned p = power < 1 ? 1 : power;
+                       bool atv, hipStream_t st, EigOut* eig, unsigned long long* wild) {
+    const unsigned p = power < 1 || atv ? 1 : power;
     if (atv) {  // sigma2, power, stick, plate and samples do not apply to ATV
         stick = plate = true;
         sigma2 = 0.0f;
         if (!tensors) return kSpectralNotApplicable;
-    } else if (p != 1 || (plate && samples > 0 && samples < 3)) {
+    } else if (!spectral_serves(p, plate, samples)) {
         return kSpectralNotApplicable;
     }
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);
@@ -1566,12 +1718,23 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     g.n0 = (int)s0; g.n1 = (int)s1; g.n2 = (int)s2;
     g.L0 = (int)L0; g.L1 = (int)L1; g.L2 = (int)L2;
     g.h0 = g.L0 / 2 + 1; g.h1 = g.L1 / 2 + 1; g.h2 = g.L2 / 2 + 1;
-    g.nf = kMono;  // stick, plate and ATV parts combined into 15 quartic features
+    g.power = (int)p;
+    g.nf = mono_count((int)p);  // stick, plate and ATV parts combined
+    for (int f = 0; f < g.nf; f++) {
+        const unsigned ox = (unsigned)mono_a(f, 2 * (int)p + 2) & 1u, oy = (unsigned)mono_b(f) & 1u;
+        if (f < 64) {
+            g.odd_x |= (unsigned long long)ox << f;
+            g.odd_y |= (unsigned long long)oy << f;
+        } else {
+            g.odd_x1 |= ox << (f - 64);
+            g.odd_y1 |= oy << (f - 64);
+        }
+    }
     g.nz = (g.nf + 1) / 2;
     g.stick = stick ? 1 : 0;
     g.plate = plate ? 1 : 0;
     g.atv = atv ? 1 : 0;
-    g.alpha = atv ? 2.0f : sticknorm3_host(sigma1, sigma2, 1);
+    g.alpha = atv ? 2.0f : sticknorm3_host(sigma1, sigma2, p);
     g.P2 = ((int)L2 + 15) & ~15;  // rows start on 128-byte lines
     g.cs = (size_t)L0 * L1 * g.P2;
     g.ocs = (size_t)g.h0 * g.h1 * g.h2;
@@ -1627,7 +1790,7 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     if ((rc = alloc(ws_get(WS_SPEC0, (size_t)g.nz * g.cs * 8, (void**)&Z))) != TIRA_OK)
         return rc == TIRA_ERR_OUT_OF_MEMORY ? kSpectralNotApplicable : rc;
     // the spectra are those of the stick part whatever the stick / plate selection
-    const SpecKey key{g.L0, g.L1, g.L2, (int)w, sigma1, sigma2, 1, 1, atv ? 1 : 0};
+    const SpecKey key{g.L0, g.L1, g.L2, (int)w, sigma1, sigma2, (int)p, atv ? 1 : 0};
     const float2 *tw0, *tw1, *tw2;
     const float* kh;
     if ((rc = alloc(spectra_for(key, g, st, &tw0, &tw1, &tw2, &kh))) != TIRA_OK)
@@ -1644,9 +1807,9 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
         const size_t nblk = ceil_div(nrows, (size_t)B);
         TH_ARG(nblk < (1ull << 31), "spectral vote: volume too large");
         if (fused)
-            k_spec_xfwd<true><<<(unsigned)nblk, kFT, xlds, st>>>(ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z);
+            launch_xfwd<true>(g.power, (unsigned)nblk, xlds, st, ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z, wild);
         else
-            k_spec_xfwd<false><<<(unsigned)nblk, kFT, xlds, st>>>(ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z);
+            launch_xfwd<false>(g.power, (unsigned)nblk, xlds, st, ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z, wild);
         TH_HIP(hipGetLastError());
     }
     {

@@ -616,10 +616,12 @@ __device__ __forceinline__ void write_payload(const VoteGeom& g, size_t pidx, fl
 }
 
 // Grid-stride over the padded payload volume: voxels outside the field get a
-// zero payload.
+// zero payload. gate (optional): the launch does nothing while *gate == 0.
 __global__ __launch_bounds__(256) void k_vote3_prep(const float* __restrict__ in, int layout, VoteGeom g,
                                                     float4* __restrict__ pay_s, float4* __restrict__ pay_p,
-                                                    float4* __restrict__ pay_v, float sum_inv_n) {
+                                                    float4* __restrict__ pay_v, float sum_inv_n,
+                                                    const unsigned long long* __restrict__ gate) {
+    if (gate && *gate == 0ull) return;
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
@@ -642,7 +644,9 @@ __global__ __launch_bounds__(256) void k_vote3_prep(const float* __restrict__ in
 __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__ lam, const float* __restrict__ ev2,
                                                        const float* __restrict__ ev0, VoteGeom g,
                                                        float4* __restrict__ pay_s, float4* __restrict__ pay_p,
-                                                       float4* __restrict__ pay_v, float sum_inv_n) {
+                                                       float4* __restrict__ pay_v, float sum_inv_n,
+                                                       const unsigned long long* __restrict__ gate) {
+    if (gate && *gate == 0ull) return;
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
@@ -1205,8 +1209,8 @@ int vote3_payload_flat(const float* tensors, int in_layout, const float* lam, co
     g.P0 = (int)s0; g.P1 = (int)s1; g.P2 = (int)s2;
     const size_t n = (size_t)s0 * s1 * s2;
     const unsigned grid = (unsigned)std::min<size_t>(ceil_div(n, 256), 65536);
-    if (tensors) k_vote3_prep<<<grid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, nullptr, 1.0f);
-    else k_vote3_prep_tk<<<grid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, nullptr, 1.0f);
+    if (tensors) k_vote3_prep<<<grid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, nullptr, 1.0f, nullptr);
+    else k_vote3_prep_tk<<<grid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, nullptr, 1.0f, nullptr);
     TH_HIP(hipGetLastError());
     return TIRA_OK;
 }
@@ -1289,14 +1293,16 @@ constexpr int kBZMlp = 8;  // the tabulated-network gather (its LDS rows are sta
 
 template <int P>
 static void launch_closed(bool stick, bool plate, unsigned grid, hipStream_t st, const float4* ps, const float4* pp,
-                          const float* tab, const VoteGeom& g, float* out, int layout) {
+                          const float* tab, const VoteGeom& g, float* out, int layout,
+                          const unsigned long long* gate) {
     // voters staged in LDS: 3% faster than reading them through L1 at 256^3, w 25;
-    // windows above 449 (more than 64 KB of segments per block) read them through L1
+    // windows above 449 (more than 64 KB of segments per block) and the gated
+    // launch (empty but for voters no spectral vote serves) read them through L1
     const size_t sh = (size_t)kTileY * 2 * (kTileX + 2 * g.r) * sizeof(float4);
-    if (sh > 65536) {
-        if (stick && plate) k_vote3_closed<P, true, true, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, tab, g, out, layout, nullptr, 0);
-        else if (stick) k_vote3_closed<P, true, false, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, tab, g, out, layout, nullptr, 0);
-        else k_vote3_closed<P, false, true, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, tab, g, out, layout, nullptr, 0);
+    if (sh > 65536 || gate) {
+        if (stick && plate) k_vote3_closed<P, true, true, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, tab, g, out, layout, gate, 0);
+        else if (stick) k_vote3_closed<P, true, false, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, tab, g, out, layout, gate, 0);
+        else k_vote3_closed<P, false, true, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, tab, g, out, layout, gate, 0);
         return;
     }
     if (stick && plate) k_vote3_closed_lds<P, true, true, kBZ><<<grid, kThreads, sh, st>>>(ps, pp, tab, g, out, layout);
@@ -1318,15 +1324,34 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
         TH_HIP(hipGetLastError());
         return TIRA_OK;
     }
-    if (plate_mode == TIRA_PLATE_AUTO && spectral_preferred(s0, s1, s2, w, power, stick, plate, samples))
-        plate_mode = TIRA_VOTE_SPECTRAL;
+    // (a request for the spectral vote above power 1 is served where AUTO takes it)
+    if (plate_mode == TIRA_PLATE_AUTO || (plate_mode == TIRA_VOTE_SPECTRAL && power > 1))
+        plate_mode = spectral_preferred(s0, s1, s2, w, power, stick, plate, samples) ? TIRA_VOTE_SPECTRAL
+                                                                                     : TIRA_PLATE_AUTO;
+    const unsigned p = power < 1 ? 1 : power;
+    // Above power 1 a spectral vote met by a voter that an FFT would spread
+    // beyond its window (not finite, a scale whose sums could overflow, a
+    // caller's stick that is not of unit length) is voted again by window: the
+    // launches below do nothing while *gate is 0.
+    unsigned long long* gate = nullptr;
     if (plate_mode == TIRA_VOTE_SPECTRAL) {
-        const int rc = vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0, s1, s2, sigma1,
-                                          sigma2, w, power, stick, plate, samples, false, st, eig);
-        if (rc != kSpectralNotApplicable) return rc;
+        const size_t ob = nvox * (out_layout == TIRA_LAYOUT_MAT9 ? 36 : 24),
+                     ib = nvox * (in_layout == TIRA_LAYOUT_MAT9 ? 36 : 24);
+        const bool aliased = tensors && (const char*)out < (const char*)tensors + ib &&
+                             (const char*)tensors < (const char*)out + ob;
+        if (p > 1 && !aliased) {
+            TH_TRY(ws_get(WS_WILD, 8, (void**)&gate));
+            k_fill_zero<<<1, 64, 0, st>>>((float*)gate, 2);
+        }
+        // (in place, the windows could not be voted again)
+        const int rc = p > 1 && aliased ? kSpectralNotApplicable
+                                        : vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0,
+                                                             s1, s2, sigma1, sigma2, w, power, stick, plate, samples,
+                                                             false, st, p > 1 ? nullptr : eig, gate);
+        if (rc != kSpectralNotApplicable && (rc != TIRA_OK || p == 1)) return rc;
+        if (rc == kSpectralNotApplicable) gate = nullptr;
         plate_mode = TIRA_PLATE_AUTO;  // power, samples or size outside the spectral method: direct gather
     }
-    const unsigned p = power < 1 ? 1 : power;
     const int mode = plate ? resolve_plate_mode(plate_mode, power, samples) : TIRA_PLATE_CLOSED;
     if (mode == TIRA_PLATE_MLP) {
         set_error("plate_mode MLP is served by tira_tensorvote3_mlp");
@@ -1342,11 +1367,11 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     const unsigned nsamp = samples == 0 ? p + 2 : samples;  // samples == 0 (analytic) equals the exact integral
     if (sum) TH_TRY(ws_get(WS_SCRATCH0, ptotal * 16, (void**)&pv));
     const float inv_n = sum ? 1.0f / (float)nsamp : 1.0f;
-    const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), 65536);
+    const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), gate ? 4096 : 65536);
     {
-        ProfScope prof("vote3_prep", st);
-        if (tensors) k_vote3_prep<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, pv, inv_n);
-        else k_vote3_prep_tk<<<pgrid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, pv, inv_n);
+        ProfScope prof(gate ? "vote3_prep_gated" : "vote3_prep", st);
+        if (tensors) k_vote3_prep<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, pv, inv_n, gate);
+        else k_vote3_prep_tk<<<pgrid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, pv, inv_n, gate);
     }
     TH_HIP(hipGetLastError());
 
@@ -1360,17 +1385,17 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     TH_TRY(table_for(key, P, st, &dtab, &dcs));
     const unsigned grid = g.nbx * g.nby * g.nbz;
     const float* t = (const float*)dtab;
-    ProfScope prof_vote(sum ? "vote3_sum" : "vote3_closed", st);
+    ProfScope prof_vote(gate ? "vote3_closed_gated" : sum ? "vote3_sum" : "vote3_closed", st);
     if (sum) {
         if (stick && plate) k_vote3_sum<true, true, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, pv, t, dcs, nsamp, p, g, out, out_layout);
         else if (stick) k_vote3_sum<true, false, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, pv, t, dcs, nsamp, p, g, out, out_layout);
         else k_vote3_sum<false, true, kBZ><<<grid, kThreads, 0, st>>>(ps, pp, pv, t, dcs, nsamp, p, g, out, out_layout);
     } else {
         switch (P) {
-            case 1: launch_closed<1>(stick, plate, grid, st, ps, pp, t, g, out, out_layout); break;
-            case 2: launch_closed<2>(stick, plate, grid, st, ps, pp, t, g, out, out_layout); break;
-            case 3: launch_closed<3>(stick, plate, grid, st, ps, pp, t, g, out, out_layout); break;
-            default: launch_closed<4>(stick, plate, grid, st, ps, pp, t, g, out, out_layout); break;
+            case 1: launch_closed<1>(stick, plate, grid, st, ps, pp, t, g, out, out_layout, gate); break;
+            case 2: launch_closed<2>(stick, plate, grid, st, ps, pp, t, g, out, out_layout, gate); break;
+            case 3: launch_closed<3>(stick, plate, grid, st, ps, pp, t, g, out, out_layout, gate); break;
+            default: launch_closed<4>(stick, plate, grid, st, ps, pp, t, g, out, out_layout, gate); break;
         }
     }
     TH_HIP(hipGetLastError());

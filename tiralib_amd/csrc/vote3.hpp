@@ -36,10 +36,12 @@ struct EigOut {
 };
 // Status of vote3_spectral_run when the request is outside the spectral method.
 constexpr int kSpectralNotApplicable = -1;
+// wild (optional, device): raised when a power above 1 met a feature that is not
+// finite or could overflow; such a voter spoils the whole spectral output.
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        float* out, int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1,
                        float sigma2, unsigned w, unsigned power, bool stick, bool plate, unsigned samples,
-                       bool atv, hipStream_t st, EigOut* eig = nullptr);
+                       bool atv, hipStream_t st, EigOut* eig = nullptr, unsigned long long* wild = nullptr);
 int resolve_plate_mode(int plate_mode, unsigned power, unsigned samples);
 int vote3_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0, float* out,
               int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1, float sigma2, unsigned w,
