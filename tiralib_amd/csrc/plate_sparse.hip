@@ -20,6 +20,7 @@
 // from LDS.
 #include "common.hpp"
 #include "plate_sparse.hpp"
+#include "seg_list.hpp"
 #include "vote3_acc.hpp"
 
 #include <algorithm>
@@ -30,7 +31,6 @@ namespace th {
 
 constexpr int kCube = 4;                     // receivers per cube edge, 4^3 = one wave
 constexpr int kSparseThreads = 1024;         // one block per CU (its LDS holds the table)
-constexpr int kScanSegs = 1024;              // segments per scan block
 constexpr int kSparseCells = kMlpTabM + 2;   // staged cells of a row: x_j, j = -1 .. kMlpTabM
 constexpr size_t kSparseLds = 160 * 1024 - 1024;
 
@@ -51,60 +51,6 @@ __global__ __launch_bounds__(256) void k_plate_count(const float4* __restrict__ 
     if (x < (unsigned)g.s2) on = pay[((size_t)(z + g.r) * g.P1 + y + g.r) * g.P2 + x + g.r].w != 0.0f;
     const unsigned long long m = __ballot(on);
     if (lane == 0) cnt[seg] = (unsigned)__popcll(m);
-}
-
-// Exclusive sums of 1024 consecutive counts in place, their total to tot[block].
-__global__ __launch_bounds__(256) void k_plate_scan(unsigned* __restrict__ cnt, unsigned n, unsigned* __restrict__ tot) {
-    __shared__ unsigned s[256];
-    const unsigned i0 = blockIdx.x * kScanSegs + threadIdx.x * 4;
-    unsigned v[4], sum = 0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        v[k] = i0 + k < n ? cnt[i0 + k] : 0u;
-        sum += v[k];
-    }
-    s[threadIdx.x] = sum;
-    __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-        const unsigned a = (int)threadIdx.x >= d ? s[threadIdx.x - d] : 0u;
-        __syncthreads();
-        s[threadIdx.x] += a;
-        __syncthreads();
-    }
-    unsigned run = s[threadIdx.x] - sum;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        if (i0 + k < n) cnt[i0 + k] = run;
-        run += v[k];
-    }
-    if (threadIdx.x == 255) tot[blockIdx.x] = s[255];
-}
-
-// Exclusive sums of the block totals (one block), and the work counter's start.
-__global__ __launch_bounds__(1024) void k_plate_scan_top(unsigned* __restrict__ tot, unsigned n,
-                                                         unsigned* __restrict__ next) {
-    __shared__ unsigned s[1024];
-    unsigned carry = 0;
-    for (unsigned b = 0; b < n; b += 1024) {
-        const unsigned i = b + threadIdx.x, v = i < n ? tot[i] : 0u;
-        s[threadIdx.x] = v;
-        __syncthreads();
-        for (int d = 1; d < 1024; d <<= 1) {
-            const unsigned a = (int)threadIdx.x >= d ? s[threadIdx.x - d] : 0u;
-            __syncthreads();
-            s[threadIdx.x] += a;
-            __syncthreads();
-        }
-        if (i < n) tot[i] = carry + s[threadIdx.x] - v;
-        carry += s[1023];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *next = 0u;
-}
-
-__device__ __forceinline__ unsigned seg_start(const unsigned* __restrict__ cnt, const unsigned* __restrict__ tot,
-                                              unsigned seg) {
-    return cnt[seg] + tot[seg / kScanSegs];
 }
 
 // The list: voter (n, scale) and position (x + (y << 16), z).
@@ -153,10 +99,6 @@ __global__ __launch_bounds__(256) void k_plate_tiles(VoteGeom g, int bz, const u
         const float wc = (float)(2 * g.r + kCube), ww = (float)(2 * g.r + 1);
         sparse[t] = (float)c * wc * wc * wc * ratio < box * ww * ww * ww ? 1 : 0;
     }
-}
-
-__device__ __forceinline__ float lane_f(float v, int j) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
 }
 
 // One offset's entry: unit direction d and c1 / pi, and the byte offset of
@@ -401,8 +343,8 @@ int plate_sparse_run(const float4* pay, const float4* vtab, int vtab_rows, float
     unsigned char* flags = (unsigned char*)next + 256;
     ProfScope prof("plate_sparse", st);
     k_plate_count<<<nseg / 4 + 1, 256, 0, st>>>(pay, g, nseg, cnt);
-    k_plate_scan<<<nscan, 256, 0, st>>>(cnt, nseg + 1, tot);
-    k_plate_scan_top<<<1, 1024, 0, st>>>(tot, nscan, next);
+    k_seg_scan<<<nscan, 256, 0, st>>>(cnt, nseg + 1, tot);
+    k_seg_scan_top<<<1, 1024, 0, st>>>(tot, nscan, next);
     k_plate_list<<<ceil_div(nseg, 4), 256, 0, st>>>(pay, g, nseg, cnt, tot, lv, lp);
     k_plate_tiles<<<ceil_div(ntile, 4), 256, 0, st>>>(g, bz, cnt, tot, kSparseRatio, flags);
     const size_t lds = (size_t)nrows * kSparseCells * sizeof(float4);
