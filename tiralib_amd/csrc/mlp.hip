@@ -522,24 +522,341 @@ __global__ __launch_bounds__(256) void k_sum_partials(const float* __restrict__ 
     }
 }
 
+// ---------------------------------------------------------------- fused step
+// One training update as two launches instead of twenty: the launches of 3 to
+// 6 us each were what a batch of 4096 (0.2 GFLOP) waited for. 80 us an update
+// before, 12 + 5 us now.
+//
+// k_mlp_step: a wave takes 32 samples through forward, loss gradient and
+// backward in registers. A
+// 32 x 32 x 16 MFMA takes the same lane layout for both operands, so each
+// product of activations and weights is formed in both orders: with the
+// weights first, the result has units in its registers and the sample in its
+// lane, which is (after one exchange between the half waves) the next layer's
+// operand; with the activations first, samples in its registers and the unit
+// in its lane, which is the weight gradients' operand.
+// The products and their order are those of k_gemm_nt and k_gemm_tn, so an
+// update gives the same bits.
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ unsigned pk_bf16(float a, float b) {
+    const bf16x2 h = __builtin_convertvector((f32x2){a, b}, bf16x2);
+    return __builtin_bit_cast(unsigned, h);
+}
+__device__ __forceinline__ float bf_lo(unsigned p) { return __uint_as_float(p << 16); }
+__device__ __forceinline__ float bf_hi(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
+
+// Accumulator rows of lane half h are 8 q + 4 h + (0 .. 3), two packed words
+// (p[2q], p[2q + 1]) per q. An operand's half h takes rows 16 s + 8 h + (0 ..
+// 7): the halves exchange the words of odd q of the lower for those of even q
+// of the upper half.
+__device__ __forceinline__ bf16x8 half_swap(unsigned p0, unsigned p1, unsigned p2, unsigned p3) {
+    const auto a = __builtin_amdgcn_permlane32_swap(p0, p2, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(p1, p3, false, false);
+    return __builtin_bit_cast(bf16x8, make_uint4(a[0], b[0], a[1], b[1]));
+}
+
+// Operands (K steps s = 0, 1 of a 32-row tile) of packed words p[0..7].
+__device__ __forceinline__ void tile_operands(const unsigned p[8], bf16x8 o[2]) {
+    o[0] = half_swap(p[0], p[1], p[2], p[3]);
+    o[1] = half_swap(p[4], p[5], p[6], p[7]);
+}
+
+// ReLU of an accumulator tile as BF16 high parts and residuals.
+__device__ __forceinline__ void relu_split(const f32x16& c, unsigned hi[8], unsigned lo[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const float a = fmaxf(c[2 * i], 0.0f), b = fmaxf(c[2 * i + 1], 0.0f);
+        hi[i] = pk_bf16(a, b);
+        lo[i] = pk_bf16(a - bf_lo(hi[i]), b - bf_hi(hi[i]));
+    }
+}
+
+// Where the high parts of a tile are positive: bit i for element i.
+__device__ __forceinline__ unsigned positive_bits(const unsigned h[8]) {
+    unsigned b = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        b |= (short)(h[i] & 0xffffu) > 0 ? 1u << (2 * i) : 0u;
+        b |= (short)(h[i] >> 16) > 0 ? 2u << (2 * i) : 0u;
+    }
+    return b;
+}
+
+// BF16 of an accumulator tile where the activation's high part is positive.
+__device__ __forceinline__ void relu_mask(const f32x16& c, unsigned bits, unsigned o[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const unsigned v = pk_bf16(c[2 * i], c[2 * i + 1]);
+        o[i] = v & ((bits & (1u << (2 * i)) ? 0xffffu : 0u) | (bits & (2u << (2 * i)) ? 0xffff0000u : 0u));
+    }
+}
+__device__ __forceinline__ void relu_mask(const f32x16& c, const unsigned h[8], unsigned o[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const unsigned v = pk_bf16(c[2 * i], c[2 * i + 1]);
+        o[i] = ((short)(h[i] & 0xffffu) > 0 ? v & 0xffffu : 0u) | ((short)(h[i] >> 16) > 0 ? v & 0xffff0000u : 0u);
+    }
+}
+
+__device__ __forceinline__ f32x16 mma(bf16x8 a, bf16x8 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// Weight operand: rows 32 t + (lane % 32) of a row-major [.. x ld] matrix, K step s.
+__device__ __forceinline__ bf16x8 w_op(const u16* __restrict__ w, int ld, int t, int s, int m, int h) {
+    return *reinterpret_cast<const bf16x8*>(w + (size_t)(32 * t + m) * ld + 16 * s + 8 * h);
+}
+
+// A hidden layer of the forward pass for the 32-sample tiles u < U: the next
+// layer's operands hi / lo [u][K step] and, for training, where they are
+// positive (sample lanes, pos[u][t]) and the packed high parts with the unit in
+// the lane (hu[t][u]).
+template <int U, int K, bool SPLIT, bool TRAIN>
+__device__ __forceinline__ void step_layer(const u16* __restrict__ W, const bf16x8 (&xh)[U][K / 16],
+                                           const bf16x8 (&xl)[U][K / 16], int m, int h, bf16x8 (&oh)[U][4],
+                                           bf16x8 (&ol)[U][4], unsigned (&pos)[U][2], unsigned (&hu)[2][U][8]) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        bf16x8 w[K / 16];
+#pragma unroll
+        for (int s = 0; s < K / 16; s++) w[s] = w_op(W, K, t, s, m, h);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            f32x16 a = {}, b = {};
+#pragma unroll
+            for (int s = 0; s < K / 16; s++) {
+                a = mma(w[s], xh[u][s], a);
+                if (TRAIN) b = mma(xh[u][s], w[s], b);
+                if (SPLIT) {
+                    a = mma(w[s], xl[u][s], a);
+                    if (TRAIN) b = mma(xl[u][s], w[s], b);
+                }
+            }
+            unsigned hi[8], lo[8];
+            relu_split(a, hi, lo);
+            if (TRAIN) pos[u][t] = positive_bits(hi);
+            bf16x8 o[2];
+            tile_operands(hi, o);
+            oh[u][2 * t] = o[0]; oh[u][2 * t + 1] = o[1];
+            tile_operands(lo, o);
+            ol[u][2 * t] = o[0]; ol[u][2 * t + 1] = o[1];
+            if (TRAIN) relu_split(b, hu[t][u], lo);
+        }
+    }
+}
+
+// Forward pass alone, 64 samples a wave in registers (rows a multiple of 32):
+// the products of mlp_forward in its order, without its activations' round
+// trips through memory. Validation, vote table and error table of a sigma-2
+// network (2.1M samples): 0.23 ms, where mlp_forward's launches took 1.4 ms and
+// its activations 1.2 GB.
+__global__ __launch_bounds__(64) void k_mlp_infer(const u16* __restrict__ X, int rows, const u16* __restrict__ W,
+                                                  float* __restrict__ Y) {
+    const int l = (int)threadIdx.x, m = l & 31, h = l >> 5;
+    const int r0 = (int)blockIdx.x * 64;
+    const bool both = r0 + 32 < rows;
+    bf16x8 x[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int s = 0; s < 2; s++) x[u][s] = w_op(X + (size_t)r0 * kMlpIn, kMlpIn, both ? u : 0, s, m, h);
+    unsigned pos[2][2], hu[2][2][8];
+    bf16x8 ah[2][4], al[2][4], bh[2][4], bl[2][4];
+    step_layer<2, kMlpIn, false, false>(W + kMlpW1, x, x, m, h, ah, al, pos, hu);
+    step_layer<2, kMlpHid, true, false>(W + kMlpW2, ah, al, m, h, bh, bl, pos, hu);
+    step_layer<2, kMlpHid, true, false>(W + kMlpW3, bh, bl, m, h, ah, al, pos, hu);
+    bf16x8 w[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) w[s] = w_op(W + kMlpW4, kMlpHid, 0, s, m, h);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        f32x16 a = {};
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            a = mma(w[s], ah[u][s], a);
+            a = mma(w[s], al[u][s], a);
+        }
+        if (u == 0 || both) {
+            float* y = Y + (size_t)(r0 + 32 * u + m) * kMlpOutPad + 4 * h;
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *reinterpret_cast<float4*>(y + 8 * q) = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
+        }
+    }
+}
+
+// A layer of the backward pass of one 32-sample tile: [H > 0] (dZ W) from the
+// operands dz[K step] and the transposed weights; the next operands (if
+// wanted) and the weight gradients' operand z[t][sample step].
+template <int K, bool NEXT>
+__device__ __forceinline__ void step_back(const u16* __restrict__ WT, const bf16x8 (&dz)[K / 16], int m, int h,
+                                          const unsigned (&pos)[2], const unsigned (&hu)[2][1][8], bf16x8 (&o)[4],
+                                          bf16x8 (&z)[2][2]) {
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        f32x16 a = {}, b = {};
+#pragma unroll
+        for (int s = 0; s < K / 16; s++) {
+            const bf16x8 w = w_op(WT, K, t, s, m, h);
+            if (NEXT) a = mma(w, dz[s], a);
+            b = mma(dz[s], w, b);
+        }
+        unsigned p[8];
+        if (NEXT) {
+            relu_mask(a, pos[t], p);
+            bf16x8 q[2];
+            tile_operands(p, q);
+            o[2 * t] = q[0]; o[2 * t + 1] = q[1];
+        }
+        relu_mask(b, hu[t][0], p);
+        tile_operands(p, z[t]);
+    }
+}
+
+__device__ __forceinline__ void store_tile(float* __restrict__ dst, int ld, const f32x16& c, int m, int h) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) dst[(size_t)(8 * (r >> 2) + 4 * h + (r & 3)) * ld + m] = c[r];
+}
+
+// Block i takes samples 64 i .. 64 i + 63, the rows of wave i % 4 of split i / 4
+// of k_gemm_tn (one chunk per split: up to 16384 samples), a wave per 32 of
+// them; part: one kMlpNParam block of partial gradients per block. The two
+// waves hand their weight-gradient operands over through LDS and each forms
+// half of the gradient tiles over all 64 samples. Bound by its own latency:
+// 64 blocks at batch 4096, and about 5000 VALU instructions of conversions a
+// wave. One wave per 64 samples took 20 us.
+enum { kOpY = 0, kOpZ3 = 2, kOpZ2 = 6, kOpZ1 = 10, kOpH3 = 14, kOpH2 = 18, kOpH1 = 22, kOps = 26 };
+__global__ __launch_bounds__(128) void k_mlp_step(const u16* __restrict__ X, const float* __restrict__ T,
+                                                  const u16* __restrict__ W, const u16* __restrict__ WT, float gscale,
+                                                  MlpAffine aff, float* __restrict__ part) {
+    __shared__ bf16x8 ops[2][kOps][64];
+    const int u = (int)threadIdx.x >> 6, l = (int)threadIdx.x & 63, m = l & 31, h = l >> 5;
+    float* P = part + (size_t)blockIdx.x * kMlpNParam;
+    const int r0 = (int)blockIdx.x * (kTnChunk / 4), ru = r0 + 32 * u;
+    {
+        bf16x8 x[1][2];
+#pragma unroll
+        for (int s = 0; s < 2; s++) x[0][s] = w_op(X + (size_t)ru * kMlpIn, kMlpIn, 0, s, m, h);
+        unsigned s1[1][2], u1[2][1][8], s2[1][2], u2[2][1][8], s3[1][2], u3[2][1][8];
+        bf16x8 ah[1][4], al[1][4], bh[1][4], bl[1][4];
+        step_layer<1, kMlpIn, false, true>(W + kMlpW1, x, x, m, h, ah, al, s1, u1);
+        step_layer<1, kMlpHid, true, true>(W + kMlpW2, ah, al, m, h, bh, bl, s2, u2);
+        step_layer<1, kMlpHid, true, true>(W + kMlpW3, bh, bl, m, h, ah, al, s3, u3);
+        auto put = [&](int at, const bf16x8 (&q)[2]) {
+            ops[u][at][l] = q[0];
+            ops[u][at + 1][l] = q[1];
+        };
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            bf16x8 q[2];
+            tile_operands(u1[t][0], q);
+            put(kOpH1 + 2 * t, q);
+            tile_operands(u2[t][0], q);
+            put(kOpH2 + 2 * t, q);
+            tile_operands(u3[t][0], q);
+            put(kOpH3 + 2 * t, q);
+        }
+        // outputs and dY: components o = 4 h + r of a sample (sample lanes), sample rows of
+        // component m (unit lanes)
+        bf16x8 dy[2], q[2];
+        f32x16 a = {}, b = {};
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const bf16x8 w = w_op(W + kMlpW4, kMlpHid, 0, s, m, h);
+            a = mma(w, ah[0][s], a);
+            b = mma(ah[0][s], w, b);
+            a = mma(w, al[0][s], a);
+            b = mma(al[0][s], w, b);
+        }
+        const float* t = T + (size_t)ru * 8;
+        float d[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int o = 4 * h + r;
+            const float sd = h == 0 ? aff.sd[r] : aff.sd[r < 2 ? 4 + r : 4];
+            const float mu = h == 0 ? aff.mu[r] : aff.mu[r < 2 ? 4 + r : 4];
+            const float diff = fmaf(sd, a[r], mu) - t[m * 8 + o];
+            d[r] = o < kMlpOut ? gscale * 2.0f * comp_weight(o) * diff * sd : 0.0f;
+        }
+        dy[0] = half_swap(pk_bf16(d[0], d[1]), pk_bf16(d[2], d[3]), 0u, 0u);
+        dy[1] = __builtin_bit_cast(bf16x8, make_uint4(0u, 0u, 0u, 0u));
+        unsigned p[8];
+        const int oc = m < kMlpOut ? m : 0;
+        const float sd = aff.sd[oc], mu = aff.mu[oc], cw = comp_weight(oc);
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            float e[2];
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int r = 2 * i + k, row = 8 * (r >> 2) + 4 * h + (r & 3);
+                const float diff = fmaf(sd, b[r], mu) - t[row * 8 + oc];
+                e[k] = m < kMlpOut ? gscale * 2.0f * cw * diff * sd : 0.0f;
+            }
+            p[i] = pk_bf16(e[0], e[1]);
+        }
+        tile_operands(p, q);
+        put(kOpY, q);
+        bf16x8 d3[4], d2[4], d1[4], z[2][2];
+        step_back<kMlpOutPad, true>(WT + 2 * kMlpHid * kMlpHid, dy, m, h, s3[0], u3, d3, z);
+        put(kOpZ3, z[0]);
+        put(kOpZ3 + 2, z[1]);
+        step_back<kMlpHid, true>(WT + kMlpHid * kMlpHid, d3, m, h, s2[0], u2, d2, z);
+        put(kOpZ2, z[0]);
+        put(kOpZ2 + 2, z[1]);
+        step_back<kMlpHid, false>(WT, d2, m, h, s1[0], u1, d1, z);
+        put(kOpZ1, z[0]);
+        put(kOpZ1 + 2, z[1]);
+    }
+    __syncthreads();
+    // gradient tile (za, hb): both operands' four sample steps, in order
+    auto grad = [&](float* dst, int ld, int za, int hb) {
+        f32x16 g = {};
+#pragma unroll
+        for (int s = 0; s < 4; s++) g = mma(ops[s >> 1][za + (s & 1)][l], ops[s >> 1][hb + (s & 1)][l], g);
+        store_tile(dst, ld, g, m, h);
+    };
+    if (u == 0) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            grad(P + kMlpW4 + 32 * k, kMlpHid, kOpY, kOpH3 + 2 * k);
+#pragma unroll
+            for (int n = 0; n < 2; n++)
+                grad(P + kMlpW3 + 32 * n * kMlpHid + 32 * k, kMlpHid, kOpZ3 + 2 * n, kOpH2 + 2 * k);
+        }
+    } else {
+        // inputs with the input slot in the lane: eight samples of one slot per operand
+        f32x16 g1[2] = {};
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const u16* px = X + (size_t)(r0 + 16 * s + 8 * h) * kMlpIn + m;
+            unsigned p[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) p[i] = (unsigned)px[2 * i * kMlpIn] | ((unsigned)px[(2 * i + 1) * kMlpIn] << 16);
+            const bf16x8 q = __builtin_bit_cast(bf16x8, make_uint4(p[0], p[1], p[2], p[3]));
+#pragma unroll
+            for (int n = 0; n < 2; n++) g1[n] = mma(ops[s >> 1][kOpZ1 + 2 * n + (s & 1)][l], q, g1[n]);
+        }
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+            store_tile(P + kMlpW1 + 32 * n * kMlpIn, kMlpIn, g1[n], m, h);
+#pragma unroll
+            for (int k = 0; k < 2; k++)
+                grad(P + kMlpW2 + 32 * n * kMlpHid + 32 * k, kMlpHid, kOpZ2 + 2 * n, kOpH1 + 2 * k);
+        }
+    }
+}
+
 struct AdamArgs {
     float lr_t, b1, b2, eps_t;
 };
 
-// Adam on one layer [rows x cols] (FP32 master p), refreshing its BF16 copy
-// wb and (if given) the BF16 transpose wtb. `tie`: layer 1, whose residual
-// input columns kMlpFeat..2*kMlpFeat-1 share the weight of the high-part
-// column: the shared weight's gradient is the sum of both columns.
-__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ p, const float* __restrict__ g,
-                                                  float* __restrict__ m, float* __restrict__ v,
-                                                  const unsigned char* __restrict__ mask, int rows, int cols,
-                                                  u16* __restrict__ wb, u16* __restrict__ wtb, AdamArgs a, int tie) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= rows * cols) return;
-    const int row = idx / cols, col = idx % cols;
-    if (tie && col >= kMlpFeat && col < 2 * kMlpFeat) return;
-    float gg = g[idx];
-    if (tie && col < kMlpFeat) gg += g[idx + kMlpFeat];
+// One parameter's Adam update from its gradient gg, and its BF16 copies.
+__device__ __forceinline__ void adam_update(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
+                                            const unsigned char* __restrict__ mask, int idx, int row, int col,
+                                            int rows, float gg, u16* __restrict__ wb, u16* __restrict__ wtb,
+                                            AdamArgs a, int tie) {
     float w = p[idx];
     if (mask[idx]) {
         const float mm = a.b1 * m[idx] + (1.0f - a.b1) * gg;
@@ -557,6 +874,56 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ p, const f
         wb[idx + kMlpFeat] = wbits;
         if (wtb) wtb[(size_t)(col + kMlpFeat) * rows + row] = wbits;
     }
+}
+
+// Adam on one layer [rows x cols] (FP32 master p), refreshing its BF16 copy
+// wb and (if given) the BF16 transpose wtb. `tie`: layer 1, whose residual
+// input columns kMlpFeat..2*kMlpFeat-1 share the weight of the high-part
+// column: the shared weight's gradient is the sum of both columns.
+__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ p, const float* __restrict__ g,
+                                                  float* __restrict__ m, float* __restrict__ v,
+                                                  const unsigned char* __restrict__ mask, int rows, int cols,
+                                                  u16* __restrict__ wb, u16* __restrict__ wtb, AdamArgs a, int tie) {
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx >= rows * cols) return;
+    const int row = idx / cols, col = idx % cols;
+    if (tie && col >= kMlpFeat && col < 2 * kMlpFeat) return;
+    float gg = g[idx];
+    if (tie && col < kMlpFeat) gg += g[idx + kMlpFeat];
+    adam_update(p, m, v, mask, idx, row, col, rows, gg, wb, wtb, a, tie);
+}
+
+// Sums the waves' partial gradients of k_mlp_step in the order of k_gemm_tn
+// (four waves of a chunk) and k_tn_reduce (chunks), and applies Adam: one
+// thread per parameter of all four layers.
+struct LayerTable {
+    int off[4], rows[4], cols[4], wt[4];
+};
+__global__ __launch_bounds__(256) void k_mlp_reduce_adam(const float* __restrict__ part, int nsplit,
+                                                         float* __restrict__ p, float* __restrict__ g,
+                                                         float* __restrict__ m, float* __restrict__ v,
+                                                         const unsigned char* __restrict__ mask, LayerTable lt,
+                                                         u16* __restrict__ wb, u16* __restrict__ wtb, AdamArgs a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= kMlpNParam) return;
+    auto sum = [&](int e) {
+        float t = 0.0f;
+#pragma unroll 16  // the loads of 16 splits in flight together: each round trip passes the writer's XCD
+        for (int s = 0; s < nsplit; s++) {
+            const float* q = part + (size_t)4 * s * kMlpNParam + e;
+            t += ((q[0] + q[kMlpNParam]) + q[2 * kMlpNParam]) + q[3 * kMlpNParam];
+        }
+        return t;
+    };
+    const int li = i >= lt.off[3] ? 3 : i >= lt.off[2] ? 2 : i >= lt.off[1] ? 1 : 0;
+    const int off = lt.off[li], rows = lt.rows[li], cols = lt.cols[li], idx = i - off;
+    const int row = idx / cols, col = idx % cols, tie = li == 0 ? 1 : 0;
+    float gg = sum(i);
+    g[i] = gg;
+    if (tie && col >= kMlpFeat && col < 2 * kMlpFeat) return;
+    if (tie && col < kMlpFeat) gg += sum(i + kMlpFeat);
+    adam_update(p + off, m + off, v + off, mask + off, idx, row, col, rows, gg, wb + off,
+                lt.wt[li] >= 0 ? wtb + lt.wt[li] : nullptr, a, tie);
 }
 
 // Y[:, 0..5] = mu + sd * Y (the network's plate-frame components).
@@ -594,23 +961,34 @@ static const Layer kLayers[4] = {
 constexpr int kMlpNWt = 2 * kMlpHid * kMlpHid + kMlpHid * kMlpOutPad;
 
 // Activations of one batch, plus the partial-sum buffers of the
-// deterministic reductions: `part` holds kTnMaxSplit split tiles of every
-// layer's weight gradient, `lpart` one (error, target) pair per loss block.
+// deterministic reductions: `part` holds, for kTnMaxSplit splits of the batch,
+// a split's four waves' weight gradients, `lpart` one (error, target) pair per loss block.
 struct Acts {
-    size_t cap = 0;
+    size_t cap = 0, ycap = 0;  // rows of a training batch, rows of outputs
     u16 *h1 = nullptr, *h2 = nullptr, *h3 = nullptr, *dy = nullptr, *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
     float* y = nullptr;
     float* sums = nullptr;
     float* part = nullptr;
     float* lpart = nullptr;
-    ~Acts() { release(); hipFree(sums); hipFree(part); }
+    ~Acts() { release(); hipFree(y); hipFree(lpart); hipFree(sums); hipFree(part); }
     void release() {
         hipFree(h1); hipFree(h2); hipFree(h3); hipFree(dy); hipFree(dz1); hipFree(dz2); hipFree(dz3);
-        hipFree(y); hipFree(lpart);
         h1 = h2 = h3 = dy = dz1 = dz2 = dz3 = nullptr;
+    }
+    // Outputs and loss partials of `rows` samples (k_mlp_infer keeps no activations).
+    int reserve_outputs(size_t rows) {
+        if (rows <= ycap) return TIRA_OK;
+        hipFree(y); hipFree(lpart);
         y = lpart = nullptr;
+        ycap = 0;
+        TH_HIP(hipMalloc(&y, rows * kMlpOutPad * 4));
+        TH_HIP(hipMalloc(&lpart, ((rows + 255) / 256) * 8));
+        if (!sums) TH_HIP(hipMalloc(&sums, 64));
+        ycap = rows;
+        return TIRA_OK;
     }
     int reserve(size_t rows) {
+        TH_TRY(reserve_outputs(rows));
         if (rows <= cap) return TIRA_OK;
         release();
         cap = 0;
@@ -618,10 +996,7 @@ struct Acts {
         TH_HIP(hipMalloc(&h1, hs)); TH_HIP(hipMalloc(&h2, hs)); TH_HIP(hipMalloc(&h3, hs));
         TH_HIP(hipMalloc(&dz1, hb)); TH_HIP(hipMalloc(&dz2, hb)); TH_HIP(hipMalloc(&dz3, hb));
         TH_HIP(hipMalloc(&dy, rows * kMlpOutPad * 2));
-        TH_HIP(hipMalloc(&y, rows * kMlpOutPad * 4));
-        TH_HIP(hipMalloc(&lpart, ((rows + 255) / 256) * 8));
-        if (!sums) TH_HIP(hipMalloc(&sums, 64));
-        if (!part) TH_HIP(hipMalloc(&part, (size_t)kTnMaxSplit * kMlpNParam * 4));
+        if (!part) TH_HIP(hipMalloc(&part, (size_t)4 * kTnMaxSplit * kMlpNParam * 4));
         cap = rows;
         return TIRA_OK;
     }
@@ -677,6 +1052,11 @@ static void mlp_forward(PlateMlp* m, const u16* X, int rows, Acts& a, hipStream_
               nullptr, 0, st);
 }
 
+// The same outputs, without the activations.
+static void mlp_infer(PlateMlp* m, const u16* X, int rows, float* Y, hipStream_t st) {
+    k_mlp_infer<<<ceil_div((size_t)rows, 64), 64, 0, st>>>(X, rows, m->wb, Y);
+}
+
 // Forward + backward of one batch (rows a multiple of 256): gradients into
 // m->grads, loss sums into a.sums. Weight gradients take the activations'
 // high parts; every reduction runs in a fixed order, so the same weights and
@@ -698,12 +1078,17 @@ static void mlp_fwd_bwd(PlateMlp* m, const u16* X, const float* T, int rows, Act
     launch_tn(a.dz1, kMlpHid, kMlpHid, X, kMlpIn, kMlpIn, rows, G + kMlpW1, kMlpIn, a.part, st);
 }
 
-static void mlp_adam(PlateMlp* m, float lr, hipStream_t st) {
+// The next step's Adam constants (advances the step count).
+static AdamArgs adam_args(PlateMlp* m, float lr) {
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     m->adam_t++;
     const double c1 = 1.0 - std::pow((double)b1, (double)m->adam_t);
     const double c2 = 1.0 - std::pow((double)b2, (double)m->adam_t);
-    AdamArgs a{(float)(lr * std::sqrt(c2) / c1), b1, b2, (float)(eps * std::sqrt(c2))};
+    return AdamArgs{(float)(lr * std::sqrt(c2) / c1), b1, b2, (float)(eps * std::sqrt(c2))};
+}
+
+static void mlp_adam(PlateMlp* m, float lr, hipStream_t st) {
+    const AdamArgs a = adam_args(m, lr);
     for (int li = 0; li < 4; li++) {
         const Layer& L = kLayers[li];
         const int n = L.rows * L.cols;
@@ -712,6 +1097,23 @@ static void mlp_adam(PlateMlp* m, float lr, hipStream_t st) {
                                                      m->wb + L.off, L.wt_off >= 0 ? m->wtb + L.wt_off : nullptr, a,
                                                      li == 0 ? 1 : 0);
     }
+}
+
+// Forward, backward and Adam of one batch (rows a multiple of 256, up to
+// kTnMaxSplit * kTnChunk): the same update as mlp_fwd_bwd and mlp_adam, bit for bit, without the loss sums.
+static void mlp_step(PlateMlp* m, const u16* X, const float* T, int rows, Acts& a, float lr, hipStream_t st) {
+    const int nsplit = rows / kTnChunk;
+    k_mlp_step<<<rows / (kTnChunk / 4), 128, 0, st>>>(X, T, m->wb, m->wtb, 1.0f / (float)rows, m->aff, a.part);
+    LayerTable lt;
+    for (int li = 0; li < 4; li++) {
+        lt.off[li] = kLayers[li].off;
+        lt.rows[li] = kLayers[li].rows;
+        lt.cols[li] = kLayers[li].cols;
+        lt.wt[li] = kLayers[li].wt_off;
+    }
+    k_mlp_reduce_adam<<<ceil_div((size_t)kMlpNParam, 256), 256, 0, st>>>(a.part, nsplit, m->params, m->grads, m->adam_m,
+                                                                         m->adam_v, m->mask, lt, m->wb, m->wtb,
+                                                                         adam_args(m, lr));
 }
 
 // Refreshes the BF16 copies from the FP32 master (host round trip).
@@ -806,10 +1208,10 @@ static int mlp_build_vote_table(PlateMlp* m, hipStream_t st) {
             set_error("MLP vote table: out of device memory");
             break;
         }
-        if ((rc = a.reserve(rows)) != TIRA_OK) break;
+        if ((rc = a.reserve_outputs(rows)) != TIRA_OK) break;
         if (hipMemcpy(drho, rho.data(), nrows * 4, hipMemcpyHostToDevice) != hipSuccess) { rc = TIRA_ERR_HIP; break; }
         k_mlp_tab_inputs<<<grid_for(rows), 256, 0, st>>>(rows, nvalid, drho, X);
-        mlp_forward(m, X, (int)rows, a, st);
+        mlp_infer(m, X, (int)rows, a.y, st);
         k_mlp_tab_convert<<<ceil_div((size_t)nrows * kMlpTabM, 256), 256, 0, st>>>(a.y, nrows, m->aff, m->vtab);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
             rc = TIRA_ERR_HIP;
@@ -912,7 +1314,7 @@ static int mlp_bin_table(PlateMlp* m, hipStream_t st) {
             }
     const int noff = (int)offs.size();
     if (noff == 0) return TIRA_OK;
-    const int bins_per = std::max(1, std::min(kMlpBins, (int)((size_t)1 << 20) / noff));
+    const int bins_per = std::max(1, std::min(kMlpBins, (int)((size_t)1 << 18) / noff));
     const size_t cap = ((size_t)bins_per * noff + 255) / 256 * 256;
     float4* doffs = nullptr;
     u16* X = nullptr;
@@ -927,7 +1329,7 @@ static int mlp_bin_table(PlateMlp* m, hipStream_t st) {
             set_error("MLP error table: out of device memory");
             break;
         }
-        if ((rc = a.reserve(cap)) != TIRA_OK) break;
+        if ((rc = a.reserve_outputs(cap)) != TIRA_OK) break;
         if (hipMemcpy(doffs, offs.data(), offs.size() * 16, hipMemcpyHostToDevice) != hipSuccess) { rc = TIRA_ERR_HIP; break; }
         float* rs_tab = rs + 2 * cap;
         for (int b0 = 0; b0 < kMlpBins; b0 += bins_per) {
@@ -935,7 +1337,7 @@ static int mlp_bin_table(PlateMlp* m, hipStream_t st) {
             const size_t valid = (size_t)nb * noff, rows = (valid + 255) / 256 * 256;
             k_mlp_bin_inputs<<<grid_for(rows), 256, 0, st>>>(rows, valid, b0, noff, doffs, m->sigma1, m->sigma2,
                                                              m->power, m->nsamp, X, T, W);
-            mlp_forward(m, X, (int)rows, a, st);
+            mlp_infer(m, X, (int)rows, a.y, st);
             k_mlp_bin_rows<<<grid_for(valid), 256, 0, st>>>(valid, b0, noff, doffs, a.y, T, W, m->aff, m->vtab, rs,
                                                             rs_tab);
             k_sum_partials<<<nb, 256, 0, st>>>(rs, noff, pb + 2 * (size_t)b0);
@@ -968,7 +1370,7 @@ static int mlp_train(PlateMlp* m, size_t nsamples, unsigned epochs, unsigned bat
             set_error("MLP training: out of device memory for %zu samples", steps * B);
             break;
         }
-        if ((rc = a.reserve(std::max(B, vchunk))) != TIRA_OK) break;
+        if ((rc = a.reserve(B)) != TIRA_OK || (rc = a.reserve_outputs(vchunk)) != TIRA_OK) break;
         const double radius = kMlpRhoMax * (double)m->sigma1;
         k_mlp_samples<<<grid_for(steps * B), 256, 0, st>>>(steps * B, seed, m->sigma1, m->sigma2, m->power,
                                                           m->nsamp, radius, X, T, nullptr);
@@ -998,9 +1400,13 @@ static int mlp_train(PlateMlp* m, size_t nsamples, unsigned epochs, unsigned bat
             const double fl = lr_final > 0.0f ? (double)lr_final / (double)lr : 0.01;
             double f = it < warm ? (double)(it + 1) / (double)warm
                                  : fl + (1.0 - fl) * 0.5 * (1.0 + std::cos(M_PI * (double)(it - warm) / (double)(total - warm)));
-            mlp_fwd_bwd(m, X + s * B * kMlpIn, T + s * B * 8, (int)B, a, st);
-            mlp_adam(m, (float)(lr * f), st);
-            if (it + steps >= total && s + 1 == steps) {
+            if (it + 1 < total && B <= (size_t)kTnMaxSplit * kTnChunk) {
+                mlp_step(m, X + s * B * kMlpIn, T + s * B * 8, (int)B, a, (float)(lr * f), st);
+            } else {
+                mlp_fwd_bwd(m, X + s * B * kMlpIn, T + s * B * 8, (int)B, a, st);
+                mlp_adam(m, (float)(lr * f), st);
+            }
+            if (it + 1 == total) {
                 // loss of the last epoch's final batch
                 if (hipMemcpyAsync(hs.data(), a.sums, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
                     hipStreamSynchronize(st) != hipSuccess) { rc = TIRA_ERR_HIP; break; }
@@ -1012,7 +1418,7 @@ static int mlp_train(PlateMlp* m, size_t nsamples, unsigned epochs, unsigned bat
         if (hipGetLastError() != hipSuccess) { rc = TIRA_ERR_HIP; set_error("MLP training launch failed"); break; }
         // validation: block partials of every chunk, then one ordered sum
         for (size_t v0 = 0; v0 < nval; v0 += vchunk) {
-            mlp_forward(m, XV + v0 * kMlpIn, (int)vchunk, a, st);
+            mlp_infer(m, XV + v0 * kMlpIn, (int)vchunk, a.y, st);
             k_mlp_loss<<<vchunk / 256, 256, 0, st>>>(a.y, TV + v0 * 8, (int)vchunk, nullptr, 0.0f, vpart,
                                                      (int)(v0 / 256), nullptr, nullptr, m->aff);
         }
@@ -1128,11 +1534,11 @@ int tira_plate_mlp_forward(void* handle, const void* X, size_t n, float* Y) {
     TH_ARG(n % 32 == 0, "row count must be a multiple of 32 (got %zu)", n);
     if (!n) return TIRA_OK;
     Acts a;
-    TH_TRY(a.reserve(std::min<size_t>(n, 1 << 20)));
+    TH_TRY(a.reserve_outputs(std::min<size_t>(n, 1 << 20)));
     hipStream_t st = stream();
-    for (size_t r0 = 0; r0 < n; r0 += a.cap) {
-        const size_t rows = std::min(a.cap, n - r0);
-        mlp_forward(m, (const u16*)X + r0 * kMlpIn, (int)rows, a, st);
+    for (size_t r0 = 0; r0 < n; r0 += a.ycap) {
+        const size_t rows = std::min(a.ycap, n - r0);
+        mlp_infer(m, (const u16*)X + r0 * kMlpIn, (int)rows, a.y, st);
         k_mlp_affine<<<grid_for(rows * kMlpOut), 256, 0, st>>>(a.y, rows, m->aff);
         TH_HIP(hipMemcpyAsync(Y + r0 * kMlpOutPad, a.y, rows * kMlpOutPad * 4, hipMemcpyDeviceToDevice, st));
     }
