@@ -112,40 +112,50 @@ __device__ __forceinline__ unsigned thin_code(const unsigned char* __restrict__ 
     return code;
 }
 
-// Wave-aggregated append of `take` lanes to list[*count...].
-__device__ __forceinline__ void wave_append(bool take, unsigned value, unsigned* __restrict__ list,
-                                            unsigned* __restrict__ count) {
-    const unsigned long long m = __ballot(take);
-    if (!m) return;
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((long long)m) - 1;
-    unsigned base = 0;
-    if (lane == leader) base = atomicAdd(count, (unsigned)__popcll(m));
-    base = __shfl(base, leader);
-    if (take) list[base + __popcll(m & ((1ull << lane) - 1ull))] = value;
+// The same code of a voxel one or more in from every face: nine 4-byte loads
+// (three voxels of a row each; the fourth byte stays inside the volume's n
+// bytes) instead of 27 byte loads with their bounds. The bytes are 0 or 1.
+__device__ __forceinline__ unsigned thin_code_inner(const unsigned char* __restrict__ v, int s1, int s2, size_t i) {
+    unsigned code = 0;
+#pragma unroll
+    for (int dz = -1; dz <= 1; dz++)
+#pragma unroll
+        for (int dy = -1; dy <= 1; dy++) {
+            unsigned w;
+            __builtin_memcpy(&w, v + (i + (long long)(dz * s1 + dy) * s2 - 1), 4);
+            const unsigned b = (w & 1u) | ((w >> 7) & 2u) | ((w >> 14) & 4u);
+            code |= b << (9 * (dz + 1) + 3 * (dy + 1));
+        }
+    return code;
 }
 
-// As wave_append, with a second value per entry appended to `list2` at the
-// same slot.
-__device__ __forceinline__ void wave_append2(bool take, unsigned value, unsigned value2, unsigned* __restrict__ list,
+// Appends the `take` threads' values (and second values, list2 not NULL) of a
+// block of 256 to list[*count ..]: one atomic per block. Every thread of the
+// block calls it, the same number of times.
+__device__ __forceinline__ void block_append(bool take, unsigned value, unsigned value2, unsigned* __restrict__ list,
                                              unsigned* __restrict__ list2, unsigned* __restrict__ count) {
+    __shared__ unsigned s_cnt[4], s_base;
     const unsigned long long m = __ballot(take);
-    if (!m) return;
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((long long)m) - 1;
-    unsigned base = 0;
-    if (lane == leader) base = atomicAdd(count, (unsigned)__popcll(m));
-    base = __shfl(base, leader);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) s_cnt[wave] = (unsigned)__popcll(m);
+    __syncthreads();
+    const unsigned c0 = s_cnt[0], c1 = s_cnt[1], c2 = s_cnt[2], total = c0 + c1 + c2 + s_cnt[3];
+    if (threadIdx.x == 0 && total) s_base = atomicAdd(count, total);
+    __syncthreads();
     if (take) {
-        const unsigned slot = base + __popcll(m & ((1ull << lane) - 1ull));
+        const unsigned slot = s_base + (wave > 0 ? c0 : 0u) + (wave > 1 ? c1 : 0u) + (wave > 2 ? c2 : 0u) +
+                              (unsigned)__popcll(m & ((1ull << lane) - 1ull));
         list[slot] = value;
-        list2[slot] = value2;
+        if (list2) list2[slot] = value2;
     }
+    __syncthreads();  // the next call writes s_cnt and s_base
 }
 
-__device__ __forceinline__ void wave_count(bool hit, unsigned* __restrict__ count) {
+// Raises *flag if any lane hit. A flag and no count: hits of thousands of
+// waves on one counter queue up, equal stores do not.
+__device__ __forceinline__ void wave_flag(bool hit, unsigned* __restrict__ flag) {
     const unsigned long long m = __ballot(hit);
-    if (m && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)m) - 1)) atomicAdd(count, (unsigned)__popcll(m));
+    if (m && (threadIdx.x & 63) == (unsigned)(__ffsll((long long)m) - 1)) *flag = 1u;
 }
 
 // ---------------------------------------------------------------- thinning kernels
@@ -163,24 +173,84 @@ __global__ __launch_bounds__(256) void k_thin_export(const unsigned char* __rest
         out[i] = (T)v[i];
 }
 
-// Object voxels (value 1) of the volume, or of a previous list, appended to
-// `list`; every lane of a wave runs the same number of iterations.
-__global__ __launch_bounds__(256) void k_thin_objects(const unsigned char* __restrict__ v, size_t n,
-                                                      const unsigned* __restrict__ from, unsigned nfrom,
-                                                      unsigned* __restrict__ list, unsigned* __restrict__ count) {
-    const size_t total = from ? (size_t)nfrom : n;
+// Object voxels (value 1) among the nfrom listed ones (from NULL: of the whole
+// volume, nfrom = n) appended to `list` (NULL: counted); every thread runs the
+// same number of iterations. stall (optional): see k_thin_apply.
+__global__ __launch_bounds__(256) void k_thin_objects(const unsigned char* __restrict__ v,
+                                                      const unsigned* __restrict__ from, size_t nfrom,
+                                                      unsigned* __restrict__ list, unsigned* __restrict__ count,
+                                                      const unsigned* __restrict__ stall) {
+    if (stall && *stall) return;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    const size_t iters = (total + stride - 1) / stride;
+    const size_t iters = (nfrom + stride - 1) / stride;
     for (size_t it = 0; it < iters; it++) {
         const size_t k = it * stride + (size_t)blockIdx.x * blockDim.x + threadIdx.x;
         unsigned i = 0;
         bool take = false;
-        if (k < total) {
+        if (k < nfrom) {
             i = from ? from[k] : (unsigned)k;
             take = v[i] == 1;
         }
-        if (list) wave_append(take, i, list, count);
-        else wave_count(take, count);
+        if (list) {
+            block_append(take, i, 0u, list, nullptr, count);
+        } else {
+            const unsigned long long m = __ballot(take);
+            if (m && (threadIdx.x & 63) == 0) atomicAdd(count, (unsigned)__popcll(m));
+        }
+    }
+}
+
+// The object voxels of a volume of 0 / 1 bytes (16-byte aligned): block b takes
+// the `per` bytes from b * per (a multiple of 4096), counts them, reserves its
+// part of the list with one atomic, reads them again and writes their indices.
+// list NULL: the count only. One atomic per wave and a byte per lane took 170 us
+// a pass over 12.6 M voxels, this 15 us.
+__global__ __launch_bounds__(256) void k_thin_objects_vol(const unsigned char* __restrict__ v, size_t n, size_t per,
+                                                          unsigned* __restrict__ list,
+                                                          unsigned* __restrict__ count) {
+    __shared__ unsigned s_wave[4], s_base;
+    const size_t lo = (size_t)blockIdx.x * per, hi = min(n, lo + per);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // the set bytes of 16 voxels from i on, as four words of 0 / 1 bytes
+    auto words = [&](size_t i) {
+        uint4 w = make_uint4(0, 0, 0, 0);
+        if (i + 16 <= hi) w = *reinterpret_cast<const uint4*>(v + i);
+        else
+            for (int b = 0; b < 16 && i + b < hi; b++)
+                (&w.x)[b >> 2] |= (unsigned)v[i + b] << (8 * (b & 3));
+        return make_uint4(w.x & 0x01010101u, w.y & 0x01010101u, w.z & 0x01010101u, w.w & 0x01010101u);
+    };
+    auto ones = [](const uint4& w) { return __popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w); };
+    unsigned c = 0;
+    for (size_t i = lo + threadIdx.x * 16; i < hi; i += 4096) c += (unsigned)ones(words(i));
+    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor((int)c, d);
+    if (lane == 0) s_wave[wave] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const unsigned t = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        s_base = t ? atomicAdd(count, t) : 0u;
+    }
+    if (!list) return;
+    __syncthreads();
+    unsigned base = s_base;
+    for (size_t i0 = lo; i0 < hi; i0 += 4096) {  // the same trips for every thread of the block
+        const size_t i = i0 + threadIdx.x * 16;
+        const uint4 w = words(i);
+        const unsigned mine = (unsigned)ones(w);
+        unsigned inc = mine;
+        for (int d = 1; d < 64; d <<= 1) {
+            const unsigned o = (unsigned)__shfl_up((int)inc, d);
+            if (lane >= d) inc += o;
+        }
+        __syncthreads();  // the previous trip's sums are read
+        if (lane == 63) s_wave[wave] = inc;
+        __syncthreads();
+        unsigned at = base + inc - mine;
+        for (int k = 0; k < wave; k++) at += s_wave[k];
+        base += s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+        for (int k = 0; k < 4; k++)
+            for (unsigned m = (&w.x)[k]; m; m &= m - 1)
+                list[at++] = (unsigned)(i + 4 * k + (__builtin_ctz(m) >> 3));
     }
 }
 
@@ -196,7 +266,10 @@ __global__ __launch_bounds__(256) void k_thin_candidates_list(const unsigned cha
                                                               unsigned nobj, unsigned char* __restrict__ mark,
                                                               unsigned* __restrict__ list,
                                                               unsigned* __restrict__ codes,
-                                                              unsigned* __restrict__ count) {
+                                                              unsigned* __restrict__ count,
+                                                              const unsigned* __restrict__ stall) {
+    if (*stall) return;
+    const size_t n = (size_t)s0 * s1 * s2;
     const int ddx = dir == 2 ? 1 : dir == 3 ? -1 : 0;
     const int ddy = dir == 0 ? -1 : dir == 1 ? 1 : 0;
     const int ddz = dir == 4 ? 1 : dir == 5 ? -1 : 0;
@@ -215,35 +288,40 @@ __global__ __launch_bounds__(256) void k_thin_candidates_list(const unsigned cha
                 const bool border = (unsigned)X >= (unsigned)s2 || (unsigned)Y >= (unsigned)s1 ||
                                     (unsigned)Z >= (unsigned)s0 || v[((size_t)Z * s1 + Y) * s2 + X] == 0;
                 if (border) {
-                    code = thin_code(v, s0, s1, s2, x, y, z);
+                    // the last of the inner form's reads is 2 past the farthest neighbour row's middle
+                    const bool inner = x > 0 && x + 1 < s2 && y > 0 && y + 1 < s1 && z > 0 && z + 1 < s0 &&
+                                       (size_t)i + ((size_t)s1 + 1) * s2 + 2 < n;
+                    code = inner ? thin_code_inner(v, s1, s2, i) : thin_code(v, s0, s1, s2, x, y, z);
                     take = !thin_endpoint(code) && thin_euler_invariant(code) && thin_simple(code);
                 }
             }
         }
         if (take) mark[i] = 1;
-        wave_append2(take, i, code, list, codes, count);
+        block_append(take, i, code, list, codes, count);
     }
 }
 
-// One Jacobi sweep of the sequential re-check (lee_thinning.h:651-661):
+// The sequential re-check (lee_thinning.h:651-661) as a relaxation in place:
 // candidate p is deleted (mark 1) when it is simple in the volume where the
 // candidates before it in raster order (neighbour bits 0..12) that are
-// currently marked for deletion are removed; otherwise kept (mark 2).
+// currently marked for deletion are removed; otherwise kept (mark 2). A
+// decision depends on earlier candidates only, so whatever the order of the
+// updates the marks settle, level by level, on the one solution; a launch that
+// changes no mark has verified it. `rounds` re-evaluations per launch: the
+// marks other waves wrote meanwhile are seen where the caches show them, and a
+// candidate without earlier candidates around it is done after the first.
 // The candidate count is read from device memory (the candidate pass wrote
 // it), so the host launches over an upper bound without reading it back.
 // codes[k]: candidate k's neighbourhood code (k_thin_candidates_list); a set
 // bit is an object neighbour, inside the volume, so its index is the
 // candidate's plus the bit's offset.
-// prev (optional): the previous sweep's change count; zero means the marks
-// are already a fixed point (mark_in equals mark_out on every candidate), and
-// the sweep returns at once.
+// changes: raised if a mark changed. prev (optional): that of the previous launch; zero means the marks
+// are settled, and the launch returns at once.
 __global__ __launch_bounds__(256) void k_thin_resolve(int s1, int s2, const unsigned* __restrict__ list,
                                                       const unsigned* __restrict__ codes,
                                                       const unsigned* __restrict__ count,
-                                                      const unsigned char* __restrict__ mark_in,
-                                                      unsigned char* __restrict__ mark_out,
-                                                      unsigned* __restrict__ changes,
-                                                      const unsigned* __restrict__ prev) {
+                                                      unsigned char* mark, unsigned* __restrict__ changes,
+                                                      const unsigned* __restrict__ prev, int rounds) {
     if (prev && *prev == 0u) return;
     const unsigned cnt = *count;
     const unsigned stride = gridDim.x * blockDim.x;
@@ -254,29 +332,48 @@ __global__ __launch_bounds__(256) void k_thin_resolve(int s1, int s2, const unsi
         bool changed = false;
         if (k < cnt) {
             const size_t i = list[k];
-            unsigned code = codes[k];
-            unsigned earlier = code & 0x1FFFu;
-            while (earlier) {
-                const int b = __builtin_ctz(earlier);
-                earlier &= earlier - 1;
-                const int dx = b % 3 - 1, dy = (b / 3) % 3 - 1, dz = b / 9 - 1;
-                const size_t q = (size_t)((long long)i + dz * plane + (long long)dy * s2 + dx);
-                if (mark_in[q] == 1) code &= ~(1u << b);
+            const unsigned code = codes[k];
+            unsigned near = code & 0x1FFFu;  // earlier neighbours; from the second round on, candidates only
+            unsigned char own = __hip_atomic_load(mark + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int round = 0; round < rounds; round++) {
+                unsigned c = code, todo = near;
+                while (todo) {
+                    const int b = __builtin_ctz(todo);
+                    todo &= todo - 1;
+                    const int dx = b % 3 - 1, dy = (b / 3) % 3 - 1, dz = b / 9 - 1;
+                    const size_t q = (size_t)((long long)i + dz * plane + (long long)dy * s2 + dx);
+                    const unsigned char m = __hip_atomic_load(mark + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (m == 0) near &= ~(1u << b);
+                    if (m == 1) c &= ~(1u << b);
+                }
+                const unsigned char m = thin_simple(c) ? 1 : 2;
+                if (m != own) {
+                    __hip_atomic_store(mark + i, m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    own = m;
+                    changed = true;
+                }
+                if (!near) break;
             }
-            const unsigned char m = thin_simple(code) ? 1 : 2;
-            mark_out[i] = m;
-            changed = m != mark_in[i];
         }
-        wave_count(changed, changes);
+        wave_flag(changed, changes);
     }
 }
 
-// Apply the decisions: delete marked candidates, clear both mark buffers.
+// Apply the decisions: delete marked candidates (deleted: raised if there is
+// one), clear the marks. unsettled (optional): whether the last re-check changed
+// a mark; if so nothing is
+// applied and *stall becomes `tag`, on which the pass's later launches do
+// nothing, and the host takes this direction up again.
 __global__ __launch_bounds__(256) void k_thin_apply(unsigned char* __restrict__ v, const unsigned* __restrict__ list,
                                                     const unsigned* __restrict__ count,
-                                                    unsigned char* __restrict__ mark_a,
-                                                    unsigned char* __restrict__ mark_b, const int final_is_a,
-                                                    unsigned* __restrict__ deleted) {
+                                                    unsigned char* __restrict__ mark,
+                                                    unsigned* __restrict__ deleted,
+                                                    const unsigned* __restrict__ unsettled,
+                                                    unsigned* __restrict__ stall, unsigned tag) {
+    if (unsettled && *unsettled) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *stall = tag;
+        return;
+    }
     const unsigned cnt = *count;
     const unsigned stride = gridDim.x * blockDim.x;
     const unsigned iters = (cnt + stride - 1) / stride;
@@ -285,12 +382,11 @@ __global__ __launch_bounds__(256) void k_thin_apply(unsigned char* __restrict__ 
         bool del = false;
         if (k < cnt) {
             const size_t i = list[k];
-            del = (final_is_a ? mark_a[i] : mark_b[i]) == 1;
+            del = mark[i] == 1;
             if (del) v[i] = 0;
-            mark_a[i] = 0;
-            mark_b[i] = 0;
+            mark[i] = 0;
         }
-        wave_count(del, deleted);
+        wave_flag(del, deleted);
     }
 }
 
@@ -347,12 +443,22 @@ __device__ __forceinline__ float fkey_inv(unsigned k) {
 
 __global__ __launch_bounds__(256) void k_otsu_max(const float* __restrict__ v, size_t n, int stride,
                                                   unsigned* __restrict__ key) {
+    __shared__ unsigned s_max[4];
     unsigned m = 0;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        m = max(m, fkey(v[i * stride]));
+    const size_t step = (size_t)gridDim.x * blockDim.x;
+    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; i + 3 * step < n; i += 4 * step) {  // four reads in flight
+        const float a = v[i * stride], b = v[(i + step) * stride], c = v[(i + 2 * step) * stride],
+                    d = v[(i + 3 * step) * stride];
+        m = max(max(m, fkey(a)), max(fkey(b), max(fkey(c), fkey(d))));
+    }
+    for (; i < n; i += step) m = max(m, fkey(v[i * stride]));
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
-    if ((threadIdx.x & 63) == 0) atomicMax(key, m);
+    if ((threadIdx.x & 63) == 0) s_max[threadIdx.x >> 6] = m;
+    __syncthreads();
+    // one atomic per block: one per wave of 4096 blocks took 198 us over 12.6 M values
+    if (threadIdx.x == 0) atomicMax(key, max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3])));
 }
 
 // numpy.histogram(values, 256, range=(0, vmax)) for float32 values: float32
@@ -361,59 +467,122 @@ __global__ __launch_bounds__(256) void k_otsu_max(const float* __restrict__ v, s
 __global__ __launch_bounds__(256) void k_otsu_hist(const float* __restrict__ v, size_t n, int stride,
                                                    const unsigned* __restrict__ key,
                                                    unsigned long long* __restrict__ hist) {
-    __shared__ unsigned h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
+    // a histogram per wave: most values of a saliency fall into the first bins
+    __shared__ unsigned hw[4][256];
+    __shared__ float edge[257];
     const float vmax = fkey_inv(*key);
-    if (vmax > 0.0f) {
-        const double dv = (double)vmax, step = dv / 256.0;
-        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-            const float a = v[i * stride];
-            if (!(a >= 0.0f && a <= vmax)) continue;
-            int idx = (int)(((double)a / dv) * 256.0);
+    const double dv = (double)vmax, step = dv / 256.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) hw[k][threadIdx.x] = 0;
+    edge[threadIdx.x] = (float)((double)threadIdx.x * step);
+    if (threadIdx.x == 0) edge[256] = vmax;
+    __syncthreads();
+    unsigned* h = hw[threadIdx.x >> 6];
+    // The quotient's bin and its corrections by one amount to the bin whose
+    // edges enclose the value: found from an FP32 quotient and the edges where
+    // those are distinct floats, else by the FP64 steps themselves. VALU-bound:
+    // 58 us over 12.6 M values (61 us with FP64 quotients and an LDS atomic per
+    // value), where reading them takes 25.
+    const bool distinct = vmax > 1e-30f;
+    const float inv = distinct ? 256.0f / vmax : 0.0f;
+    auto bin = [&](float a) {  // -1: outside the range
+        if (!(a >= 0.0f && a <= vmax)) return -1;
+        int idx;
+        if (distinct) {
+            idx = min((int)(a * inv), 255);
+            while (a < edge[idx]) idx--;  // edge[0] = 0 <= a
+            while (idx != 255 && a >= edge[idx + 1]) idx++;
+        } else {
+            idx = (int)(((double)a / dv) * 256.0);
             if (idx == 256) idx = 255;
-            if (a < (float)((double)idx * step)) idx--;
-            if (idx != 255 && a >= (idx + 1 == 256 ? vmax : (float)((double)(idx + 1) * step))) idx++;
-            atomicAdd(&h[idx], 1u);
+            if (a < edge[idx]) idx--;
+            if (idx != 255 && a >= edge[idx + 1]) idx++;
         }
+        return idx;
+    };
+    // lanes that share a bin add once: equal LDS addresses would queue up
+    auto add = [&](int idx) {
+        for (int round = 0; round < 4; round++) {
+            if (idx < 0) return;
+            const int lead = __builtin_amdgcn_readfirstlane(idx);
+            const unsigned long long same = __ballot(idx == lead);
+            if (idx == lead) {
+                if ((threadIdx.x & 63) == (unsigned)__builtin_ctzll(same)) atomicAdd(&h[lead], (unsigned)__popcll(same));
+                return;
+            }
+        }
+        atomicAdd(&h[idx], 1u);
+    };
+    if (vmax > 0.0f) {
+        const size_t hop = (size_t)gridDim.x * blockDim.x;
+        size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+        for (; i + 3 * hop < n; i += 4 * hop) {  // four reads in flight
+            const float a0 = v[i * stride], a1 = v[(i + hop) * stride], a2 = v[(i + 2 * hop) * stride],
+                        a3 = v[(i + 3 * hop) * stride];
+            add(bin(a0));
+            add(bin(a1));
+            add(bin(a2));
+            add(bin(a3));
+        }
+        for (; i < n; i += hop) add(bin(v[i * stride]));
     }
     __syncthreads();
-    if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+    const unsigned long long c = (unsigned long long)hw[0][threadIdx.x] + hw[1][threadIdx.x] + hw[2][threadIdx.x] +
+                                 hw[3][threadIdx.x];
+    if (c) atomicAdd(&hist[threadIdx.x], c);
 }
 
 // Otsu's between-class variance over the 256 bins, FP64, first maximum
-// (reconstruct.py:46-63); threshold = that bin's float32 centre.
-__global__ void k_otsu_select(const unsigned* __restrict__ key, const unsigned long long* __restrict__ hist,
-                              float* __restrict__ thr) {
-    if (threadIdx.x != 0) return;
+// (reconstruct.py:46-63); threshold = that bin's float32 centre. The sums run
+// in bin order (one thread, from LDS), the variances one per thread. One
+// thread for all of it, each bin read from memory in turn, took 58 us.
+__global__ __launch_bounds__(256) void k_otsu_select(const unsigned* __restrict__ key,
+                                                     const unsigned long long* __restrict__ hist,
+                                                     float* __restrict__ thr) {
+    __shared__ double s_w[256], s_c[256], s_b[256];
+    __shared__ float s_ctr[256];
+    const int i = (int)threadIdx.x;
     const float vmax = fkey_inv(*key);
-    if (!(vmax > 0.0f)) { *thr = 0.0f; return; }
-    const double step = (double)vmax / 256.0;
-    double total = 0.0;
-    for (int i = 0; i < 256; i++) total += (double)hist[i];
-    if (total == 0.0) { *thr = 0.0f; return; }
-    double cum = 0.0, w0 = 0.0, best = 0.0;
-    // mu_total is the last cumulative sum: a first pass in the same order
-    for (int i = 0; i < 256; i++) {
-        const float e0 = (float)((double)i * step), e1 = i == 255 ? vmax : (float)((double)(i + 1) * step);
-        cum += (double)hist[i] * (double)((e0 + e1) / 2.0f);
+    if (!(vmax > 0.0f)) {
+        if (i == 0) *thr = 0.0f;
+        return;
     }
-    const double mu_total = cum;
-    cum = 0.0;
-    float bc = 0.0f;
-    for (int i = 0; i < 256; i++) {
-        const float e0 = (float)((double)i * step), e1 = i == 255 ? vmax : (float)((double)(i + 1) * step);
-        const float c = (e0 + e1) / 2.0f;
-        cum += (double)hist[i] * (double)c;
-        w0 += (double)hist[i];
-        const double w1 = total - w0;
+    const double step = (double)vmax / 256.0;
+    const float e0 = (float)((double)i * step), e1 = i == 255 ? vmax : (float)((double)(i + 1) * step);
+    s_ctr[i] = (e0 + e1) / 2.0f;
+    s_w[i] = (double)hist[i];
+    s_c[i] = s_w[i] * (double)s_ctr[i];
+    __syncthreads();
+    if (i == 0) {  // running sums in place: s_w[255] the total, s_c[255] mu_total
+        double w = 0.0, c = 0.0;
+        for (int k = 0; k < 256; k++) {
+            w += s_w[k];
+            c += s_c[k];
+            s_w[k] = w;
+            s_c[k] = c;
+        }
+    }
+    __syncthreads();
+    const double total = s_w[255], mu_total = s_c[255];
+    if (total == 0.0) {
+        if (i == 0) *thr = 0.0f;
+        return;
+    }
+    {
+        const double w0 = s_w[i], cum = s_c[i], w1 = total - w0;
         const double mu0 = w0 > 0 ? cum / w0 : 0.0;
         const double mu1 = w1 > 0 ? (mu_total - cum) / w1 : 0.0;
         const double d = mu0 - mu1;
-        const double b = w0 * w1 * (d * d);
-        if (i == 0 || b > best) { best = b; bc = c; }
+        s_b[i] = w0 * w1 * (d * d);
     }
-    *thr = bc;
+    __syncthreads();
+    if (i == 0) {
+        double best = s_b[0];
+        int at = 0;
+        for (int k = 1; k < 256; k++)
+            if (s_b[k] > best) { best = s_b[k]; at = k; }
+        *thr = s_ctr[at];
+    }
 }
 
 __global__ __launch_bounds__(256) void k_threshold(const float* __restrict__ v, size_t n, int stride,
@@ -435,39 +604,57 @@ int otsu_run(const float* v, size_t n, int stride, float* thr, hipStream_t st) {
     k_fill_u64<<<1, 256, 0, st>>>(hist, 256);
     k_thin_zero<<<1, 64, 0, st>>>(key, 1);
     ProfScope prof("otsu", st);
-    k_otsu_max<<<grid_for(n, 256, 4096), 256, 0, st>>>(v, n, stride, key);
-    k_otsu_hist<<<grid_for(n, 256 * 16, 2048), 256, 0, st>>>(v, n, stride, key, hist);
-    k_otsu_select<<<1, 64, 0, st>>>(key, hist, thr);
+    k_otsu_max<<<grid_for(n, 256 * 16, 1024), 256, 0, st>>>(v, n, stride, key);
+    k_otsu_hist<<<grid_for(n, 256 * 16, 512), 256, 0, st>>>(v, n, stride, key, hist);
+    k_otsu_select<<<1, 256, 0, st>>>(key, hist, thr);
     TH_HIP(hipGetLastError());
     return TIRA_OK;
 }
 
-constexpr int kThinSlots = 34;  // counters per direction in an outer pass (1 + 33 sweeps)
-constexpr unsigned kThinFirst = 4;  // re-check sweeps of a direction before its first read-back
+constexpr int kThinSlots = 4;   // per direction: its candidates, whether each re-check launch changed a mark
+constexpr int kThinRounds = 4;  // re-evaluations per re-check launch but the verifying one
 
 // Lee thinning of the 0/1 byte volume `v` (device) in place; blocking. The
 // object voxels are compacted into a list once and the list is refiltered
 // after every outer pass, so each border direction examines the remaining
 // object voxels only instead of the whole volume.
+//
+// An outer pass is queued whole: per direction the candidates, two re-checks of
+// kThinRounds rounds, one that verifies them, and the deletions, then the next
+// object list, and the host reads the pass's counters once. A direction whose
+// re-check had not settled applies nothing and makes the rest of the pass do
+// nothing; the host then repeats its re-check until it settles and queues the
+// directions after it. A read-back after every direction and Jacobi sweeps of
+// one evaluation a launch took 2.2 ms where this takes 1.0 (192 x 256 x 256
+// vessels, 5 outer passes); with one re-check and its verification a direction
+// in eight was taken up again.
 int lee_run(unsigned char* v, unsigned s0, unsigned s1, unsigned s2, unsigned* iterations, hipStream_t st) {
     const size_t n = (size_t)s0 * s1 * s2;
-    unsigned char *ma = nullptr, *mb = nullptr;
+    unsigned char* mark = nullptr;
     unsigned *list = nullptr, *cnt = nullptr, *objA = nullptr, *objB = nullptr;
-    TH_TRY(ws_get(WS_SCRATCH0, n, (void**)&ma));
-    TH_TRY(ws_get(WS_SCRATCH1, n, (void**)&mb));
-    TH_TRY(ws_get(WS_COUNTER, (16 + 6 * kThinSlots) * 4, (void**)&cnt));
-    k_fill_u8<<<grid_for(n), 256, 0, st>>>(ma, n);
-    k_fill_u8<<<grid_for(n), 256, 0, st>>>(mb, n);
+    // [0 .. 5] whether a direction deleted a voxel, [6] object voxels, [7] stall, then per
+    // direction kThinSlots
+    constexpr int kObj = 6, kStall = 7, kDir = 8, kAll = kDir + 6 * kThinSlots;
+    TH_TRY(ws_get(WS_SCRATCH0, n, (void**)&mark));
+    TH_TRY(ws_get(WS_COUNTER, kAll * 4, (void**)&cnt));
+    k_fill_u8<<<grid_for(n), 256, 0, st>>>(mark, n);
     TH_HIP(hipGetLastError());
-    unsigned host[4];
     ProfScope prof("lee_thin", st);
     // object list: count, size the buffers, gather
-    k_thin_zero<<<1, 64, 0, st>>>(cnt, 4);
-    k_thin_objects<<<grid_for(n), 256, 0, st>>>(v, n, nullptr, 0, nullptr, cnt + 3);
-    TH_HIP(hipGetLastError());
-    TH_HIP(hipMemcpyAsync(host + 3, cnt + 3, 4, hipMemcpyDeviceToHost, st));
+    const bool aligned = ((uintptr_t)v & 15) == 0;
+    const size_t per = std::max<size_t>((n / 1024 + 4095) & ~size_t(4095), 4096);
+    auto objects = [&](unsigned* to) -> int {
+        k_thin_zero<<<1, 64, 0, st>>>(cnt + kObj, 2);
+        if (aligned) k_thin_objects_vol<<<(unsigned)((n + per - 1) / per), 256, 0, st>>>(v, n, per, to, cnt + kObj);
+        else k_thin_objects<<<grid_for(n), 256, 0, st>>>(v, nullptr, n, to, cnt + kObj, nullptr);
+        TH_HIP(hipGetLastError());
+        return TIRA_OK;
+    };
+    unsigned host[8];
+    TH_TRY(objects(nullptr));
+    TH_HIP(hipMemcpyAsync(host + kObj, cnt + kObj, 4, hipMemcpyDeviceToHost, st));
     TH_HIP(hipStreamSynchronize(st));
-    unsigned nobj = host[3];
+    unsigned nobj = host[kObj];
     if (nobj == 0) {
         if (iterations) *iterations = 1;  // one outer pass finds nothing to delete
         return TIRA_OK;
@@ -475,69 +662,65 @@ int lee_run(unsigned char* v, unsigned s0, unsigned s1, unsigned s2, unsigned* i
     TH_TRY(ws_get(WS_SCRATCH2, (size_t)nobj * 4, (void**)&list));
     TH_TRY(ws_get(WS_THIN0, (size_t)nobj * 4, (void**)&objA));
     TH_TRY(ws_get(WS_THIN1, (size_t)nobj * 4, (void**)&objB));
-    k_thin_zero<<<1, 64, 0, st>>>(cnt + 3, 1);
-    k_thin_objects<<<grid_for(n), 256, 0, st>>>(v, n, nullptr, 0, objA, cnt + 3);
-    TH_HIP(hipGetLastError());
-    // Counters: [1] [2] changes of the two sweeps of a batch beyond the
-    // per-direction slots, [3] object voxels, [8 + dir] deletions of this
-    // outer pass, then per direction kThinSlots slots: [0] its candidates,
-    // [1 + s] the changes of its re-check sweep s. One launch clears a pass's
-    // counters; the re-check and apply passes read the candidate count on the
-    // device (launched over the object count, an upper bound), so a direction
-    // needs one read-back for its first kThinFirst sweeps and one per two
-    // after, and an outer pass one more. The
-    // candidates' neighbourhood codes go to objB, which is free until the
-    // pass's object list is rebuilt.
+    TH_TRY(objects(objA));
+    // The candidates' neighbourhood codes go to objB, which is free until the
+    // pass's object list is rebuilt. The re-check and apply passes read the
+    // candidate count on the device (launched over the object count, an upper
+    // bound).
+    auto resolve = [&](unsigned* dc, unsigned* ch, const unsigned* prev, int rounds) {
+        k_thin_resolve<<<grid_for(nobj), 256, 0, st>>>((int)s1, (int)s2, list, objB, dc, mark, ch, prev, rounds);
+    };
     int iters = 0;
-    unsigned host_pass[6];
     for (;;) {
         iters++;
-        k_thin_zero_n<<<1, 256, 0, st>>>(cnt + 8, 8 + 6 * kThinSlots);
-        for (int dir = 0; dir < 6; dir++) {
-            unsigned* dc = cnt + 16 + dir * kThinSlots;
-            k_thin_candidates_list<<<grid_for(nobj), 256, 0, st>>>(v, (int)s0, (int)s1, (int)s2, dir, objA, nobj, ma,
-                                                                   list, objB, dc);
-            TH_HIP(hipGetLastError());
-            unsigned char *in = ma, *out = mb;
-            // the first batch runs kThinFirst sweeps (most directions settle
-            // within them; a sweep after a fixed point returns at once), later
-            // batches two, each batch ending with one read-back
-            for (unsigned sweep = 0;;) {
-                // bounded: each sweep settles at least one more level of the raster-order DAG, and
-                // there are at most nobj candidates; a sweep that changes nothing is a fixed point,
-                // so the later sweeps of a batch may repeat a settled state harmlessly
-                TH_ARG(sweep <= nobj + kThinFirst, "thinning re-check did not settle (internal error)");
-                const unsigned nb = sweep == 0 ? kThinFirst : 2;
-                unsigned* ch = dc + 1 + sweep;
-                if (sweep + nb > (unsigned)kThinSlots - 1) {  // beyond the cleared slots
-                    ch = cnt + 1;
-                    k_thin_zero<<<1, 64, 0, st>>>(ch, 2);
-                }
-                for (unsigned b = 0; b < nb; b++) {
-                    k_thin_resolve<<<grid_for(nobj), 256, 0, st>>>((int)s1, (int)s2, list, objB, dc, in, out, ch + b,
-                                                                   b ? ch + b - 1 : nullptr);
-                    std::swap(in, out);
-                }
+        k_thin_zero_n<<<1, 256, 0, st>>>(cnt, kAll);
+        for (int first = 0; first < 6;) {
+            for (int dir = first; dir < 6; dir++) {
+                unsigned* dc = cnt + kDir + dir * kThinSlots;
+                k_thin_candidates_list<<<grid_for(nobj), 256, 0, st>>>(v, (int)s0, (int)s1, (int)s2, dir, objA, nobj,
+                                                                       mark, list, objB, dc, cnt + kStall);
+                resolve(dc, dc + 1, nullptr, kThinRounds);
+                resolve(dc, dc + 2, dc + 1, kThinRounds);
+                resolve(dc, dc + 3, dc + 2, 1);
+                k_thin_apply<<<grid_for(nobj), 256, 0, st>>>(v, list, dc, mark, cnt + dir, dc + 3, cnt + kStall,
+                                                             (unsigned)dir + 1);
                 TH_HIP(hipGetLastError());
-                TH_HIP(hipMemcpyAsync(host + 2, ch + nb - 1, 4, hipMemcpyDeviceToHost, st));
-                TH_HIP(hipStreamSynchronize(st));
-                if (host[2] == 0) break;
-                sweep += nb;
             }
-            k_thin_apply<<<grid_for(nobj), 256, 0, st>>>(v, list, dc, ma, mb, in == ma ? 1 : 0, cnt + 8 + dir);
+            // drop deleted voxels from the object list; read it with this pass's deletions
+            k_thin_objects<<<grid_for(nobj), 256, 0, st>>>(v, objA, nobj, objB, cnt + kObj, cnt + kStall);
             TH_HIP(hipGetLastError());
+            TH_HIP(hipMemcpyAsync(host, cnt, 8 * 4, hipMemcpyDeviceToHost, st));
+            TH_HIP(hipStreamSynchronize(st));
+            if (!host[kStall]) break;
+            const int dir = (int)host[kStall] - 1;
+            unsigned* dc = cnt + kDir + dir * kThinSlots;
+            // bounded: each launch settles at least one more level of the raster-order DAG, and
+            // there are at most nobj candidates
+            for (unsigned k = 0;; k++) {
+                TH_ARG(k <= nobj, "thinning re-check did not settle (internal error)");
+                k_thin_zero<<<1, 64, 0, st>>>(dc + 1, 2);
+                resolve(dc, dc + 1, nullptr, kThinRounds);
+                resolve(dc, dc + 2, dc + 1, 1);
+                TH_HIP(hipGetLastError());
+                TH_HIP(hipMemcpyAsync(host, dc + 2, 4, hipMemcpyDeviceToHost, st));
+                TH_HIP(hipStreamSynchronize(st));
+                if (host[0] == 0) break;
+            }
+            k_thin_apply<<<grid_for(nobj), 256, 0, st>>>(v, list, dc, mark, cnt + dir, nullptr, nullptr, 0u);
+            k_thin_zero<<<1, 64, 0, st>>>(cnt + kObj, 2);
+            TH_HIP(hipGetLastError());
+            first = dir + 1;
+            if (first == 6) {  // only the object list is left
+                k_thin_objects<<<grid_for(nobj), 256, 0, st>>>(v, objA, nobj, objB, cnt + kObj, nullptr);
+                TH_HIP(hipGetLastError());
+                TH_HIP(hipMemcpyAsync(host, cnt, 8 * 4, hipMemcpyDeviceToHost, st));
+                TH_HIP(hipStreamSynchronize(st));
+            }
         }
-        // drop deleted voxels from the object list; read it with this pass's deletions
-        k_thin_zero<<<1, 64, 0, st>>>(cnt + 3, 1);
-        k_thin_objects<<<grid_for(nobj), 256, 0, st>>>(v, n, objA, nobj, objB, cnt + 3);
-        TH_HIP(hipGetLastError());
-        TH_HIP(hipMemcpyAsync(host + 3, cnt + 3, 4, hipMemcpyDeviceToHost, st));
-        TH_HIP(hipMemcpyAsync(host_pass, cnt + 8, 6 * 4, hipMemcpyDeviceToHost, st));
-        TH_HIP(hipStreamSynchronize(st));
         bool deleted_any = false;
-        for (int d = 0; d < 6; d++) deleted_any = deleted_any || host_pass[d] != 0;
+        for (int d = 0; d < 6; d++) deleted_any = deleted_any || host[d] != 0;
         if (!deleted_any) break;  // a whole pass of six directions deleted nothing
-        nobj = host[3];
+        nobj = host[kObj];
         std::swap(objA, objB);
         if (nobj == 0) {  // the next outer pass would find no candidate in any direction
             iters++;
