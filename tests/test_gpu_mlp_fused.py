@@ -47,3 +47,19 @@ def test_forward_rows_do_not_depend_on_the_batch(hip, rows):
     full = net.forward(X).to_host()
     x = _rows(X, 0, rows, 32, np.uint16)
     np.testing.assert_array_equal(net.forward(x).to_host(), full[:rows])
+
+
+@pytest.mark.parametrize("nsamples", [256, 16640, 65536, 131072])
+def test_output_standardisation(hip, nsamples):
+    """Means and deviations of the first 65536 training targets against FP64 sums in
+    sample order: sums of n terms in another order differ by at most n ulp of FP64,
+    7e-12 relative to the sum of magnitudes, so the FP32 results by one rounding."""
+    net = api.PlateMLP(1.5, 0.5, 1, 16, seed=8)
+    net.train(nsamples=nsamples, epochs=1, batch=256, seed=21)
+    _, T, _ = net.samples(nsamples, seed=21)
+    t = T.to_host().reshape(nsamples, 8)[:65536, :6].astype(np.float64)
+    mu = t.mean(0)
+    sd = np.maximum(np.sqrt(np.maximum((t * t).mean(0) - mu * mu, 0)), 1e-3 * (np.abs(mu) + 1e-3))
+    got = net.affine()
+    np.testing.assert_allclose(got[0], mu, rtol=2.0 ** -23, atol=1e-11 * np.abs(t).max())
+    np.testing.assert_allclose(got[1], sd, rtol=2.0 ** -22)

@@ -120,7 +120,8 @@ struct PlateMlp {
     unsigned power = 1;
     unsigned nsamp = 64;         // integrator samples behind every training target
     bool trained = false;
-    // device state
+    // device state: all but vtab cut from one allocation
+    void* store = nullptr;
     float* params = nullptr;     // kMlpNParam FP32
     float* grads = nullptr;
     float* adam_m = nullptr;
