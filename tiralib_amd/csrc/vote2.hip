@@ -394,7 +394,10 @@ __device__ __forceinline__ void listed2_pair(float qx, float qy, float z, float 
             pow_pair(1.0f - q2, q2, power, e1, e2);
             D = fmaf(e.a.z, e1, e.a.w * e2);
         }
-        const float t2 = -2.0f * qTd, Rqx = fmaf(t2, e.a.x, qx), Rqy = fmaf(t2, e.a.y, qy);
+        // R = I - 2 d d^T entry by entry: q - 2 (q . d) d would carry the rounding of
+        // q . d twice (3% further from FP64 over a search population)
+        const float mx = -2.0f * e.a.x, my = -2.0f * e.a.y, Rb = mx * e.a.y;
+        const float Rqx = fmaf(fmaf(mx, e.a.x, 1.0f), qx, Rb * qy), Rqy = fmaf(fmaf(my, e.a.y, 1.0f), qy, Rb * qx);
         const float f = D * z;
         const float fx = f * Rqx;
         s.x = fmaf(fx, Rqx, s.x); s.y = fmaf(fx, Rqy, s.y); s.z = fmaf(f * Rqy, Rqy, s.z);
@@ -436,6 +439,7 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
             // two entries in turn: the next voter's is in flight while this one is evaluated
             Grid2Entry ea, eb;
             int ja = __builtin_ctzll(m), jb = 0;
+            float3 t = make_float3(0.0f, 0.0f, 0.0f);  // up to 64 voters' sum: shorter chains than one running sum
             grid2_fetch<PLATE>(grid, n, __builtin_amdgcn_readlane(base, ja), lane_off, ea);
             for (;;) {
                 m &= m - 1;
@@ -444,7 +448,7 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
                     grid2_fetch<PLATE>(grid, n, __builtin_amdgcn_readlane(base, jb), lane_off, eb);
                 }
                 listed2_pair<STICK, PLATE, P1>(lane_f(v.x, ja), lane_f(v.y, ja), lane_f(v.z, ja), lane_f(v.w, ja), ea,
-                                               power, s);
+                                               power, t);
                 if (!m) break;
                 m &= m - 1;
                 if (m) {
@@ -452,9 +456,12 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
                     grid2_fetch<PLATE>(grid, n, __builtin_amdgcn_readlane(base, ja), lane_off, ea);
                 }
                 listed2_pair<STICK, PLATE, P1>(lane_f(v.x, jb), lane_f(v.y, jb), lane_f(v.z, jb), lane_f(v.w, jb), eb,
-                                               power, s);
+                                               power, t);
                 if (!m) break;
             }
+            s.x += t.x;
+            s.y += t.y;
+            s.z += t.z;
         }
     }
     return s;
