@@ -207,7 +207,7 @@ __global__ __launch_bounds__(256) void k_vote2_prep_tk(const float2* __restrict_
 }
 
 // (t1^p, t2^p) for a wave-uniform p >= 1 by squaring: about 2 log2 p products
-// each instead of p - 1 (and as many roundings fewer).
+// each instead of p - 1.
 __device__ __forceinline__ void pow_pair(float t1, float t2, int p, float& e1, float& e2) {
     e1 = e2 = 1.0f;
     for (;;) {
