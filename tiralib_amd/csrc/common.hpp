@@ -57,8 +57,12 @@ enum Slot {
 int ws_get(int slot, size_t bytes, void** p);
 // Bytes held by `slot` for this thread on the current device (0 if none).
 size_t ws_capacity(int slot);
-// Changes whenever any workspace buffer of this thread is allocated or released.
-unsigned long long ws_generation();
+// Number of the allocation behind `slot` (thread and current device): another
+// one after the buffer has grown or was released, also where the new buffer
+// lies at the old address. What a slot holds is kept between calls by this
+// number; allocations of other slots leave it alone, so a call that found its
+// tables once finds them again (under stream capture they cannot be uploaded).
+unsigned long long ws_generation(int slot);
 
 // Device view of a caller buffer: `src` itself when it is device memory,
 // else a workspace copy (H2D on the library stream).

@@ -256,6 +256,7 @@ struct SparseTabCache {
     float s1 = 0.0f;
     int device = -1;
     void* ptr = nullptr;
+    unsigned long long gen = 0;  // workspace generation: a released buffer may come back at its address
 };
 static thread_local SparseTabCache g_stab;
 
@@ -271,10 +272,12 @@ static int sparse_tables(int w, float s1, int vtab_rows, hipStream_t st, float4*
     *ent = (float4*)buf;
     *entrow = (int*)(buf + n * 16);
     *rows = (int*)(buf + n * 20);
-    if (g_stab.w == w && g_stab.s1 == s1 && g_stab.device == dev && g_stab.ptr == buf) {
+    if (g_stab.w == w && g_stab.s1 == s1 && g_stab.device == dev && g_stab.ptr == buf &&
+        g_stab.gen == ws_generation(WS_TABLE5)) {
         *nrows = g_stab.nrows;
         return TIRA_OK;
     }
+    g_stab.device = -1;
     std::vector<int> shells, used, slot;
     mlp_shells(s1, shells);
     slot.assign(shells.size() + 2, -1);
@@ -303,6 +306,7 @@ static int sparse_tables(int w, float s1, int vtab_rows, hipStream_t st, float4*
     TH_HIP(hipStreamSynchronize(st));
     TH_HIP(hipMemcpy(buf, h.data(), bytes, hipMemcpyHostToDevice));
     g_stab.w = w; g_stab.s1 = s1; g_stab.nrows = *nrows; g_stab.device = dev; g_stab.ptr = buf;
+    g_stab.gen = ws_generation(WS_TABLE5);
     return TIRA_OK;
 }
 

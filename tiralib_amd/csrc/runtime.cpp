@@ -74,16 +74,13 @@ int use_device(int device) {
 struct Workspace {
     void* ptr[WS_NSLOTS] = {};
     size_t cap[WS_NSLOTS] = {};
+    unsigned long long gen[WS_NSLOTS] = {};  // the allocation's number, unique in the thread
 };
 static constexpr int kMaxDevices = 16;
 // Deliberately not freed at thread exit: the HIP runtime may already be torn
 // down then. tira_hip_release_workspace() frees explicitly.
 static thread_local Workspace* g_ws[kMaxDevices] = {};
-// Bumped whenever a workspace buffer is allocated or released, so that
-// callers caching the contents of a slot can tell it is still the same buffer.
-static thread_local unsigned long long g_ws_gen = 1;
-
-unsigned long long ws_generation() { return g_ws_gen; }
+static thread_local unsigned long long g_ws_gen = 0;
 
 int ws_get(int slot, size_t bytes, void** p) {
     int dev = 0;
@@ -103,9 +100,9 @@ int ws_get(int slot, size_t bytes, void** p) {
             w.cap[slot] = 0;
         }
         size_t b = (bytes + 4095) & ~size_t(4095);
-        g_ws_gen++;
         TH_HIP(hipMalloc(&w.ptr[slot], b));
         w.cap[slot] = b;
+        w.gen[slot] = ++g_ws_gen;
     }
     *p = w.ptr[slot];
     return TIRA_OK;
@@ -117,6 +114,14 @@ size_t ws_capacity(int slot) {
         !g_ws[dev])
         return 0;
     return g_ws[dev]->cap[slot];
+}
+
+unsigned long long ws_generation(int slot) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices || slot < 0 || slot >= WS_NSLOTS ||
+        !g_ws[dev])
+        return 0;
+    return g_ws[dev]->gen[slot];
 }
 
 int stage_in(const void* src, size_t bytes, int slot, const void** dev) {
@@ -325,7 +330,6 @@ int tira_hip_release_workspace(void) {
     int dev = 0;
     TH_HIP(hipGetDevice(&dev));
     if (dev >= 0 && dev < kMaxDevices && g_ws[dev]) {
-        g_ws_gen++;
         TH_HIP(hipStreamSynchronize(g_stream));
         for (int s = 0; s < WS_NSLOTS; s++)
             if (g_ws[dev]->ptr[s]) TH_HIP(hipFree(g_ws[dev]->ptr[s]));

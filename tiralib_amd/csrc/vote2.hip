@@ -144,7 +144,7 @@ __global__ __launch_bounds__(256) void k_build_nb2(int w, float s1, float s2, un
 }
 
 // Device copy of a host table in workspace `slot`, kept while its bytes and
-// the buffer (same device, address and workspace generation) are unchanged:
+// the buffer (same device, address and allocation) are unchanged:
 // repeated calls with the same parameters skip the stream wait and the copy.
 struct TableCache {
     int dev = -1;
@@ -157,7 +157,7 @@ static int table_to_device(int slot, const void* host, size_t nbytes, TableCache
     TH_TRY(ws_get(slot, nbytes ? nbytes : 1, &d));
     int dev = 0;
     TH_HIP(hipGetDevice(&dev));
-    const bool same = nbytes > 0 && c.dev == dev && c.buf == d && c.gen == ws_generation() &&
+    const bool same = nbytes > 0 && c.dev == dev && c.buf == d && c.gen == ws_generation(slot) &&
                       c.bytes.size() == nbytes && std::memcmp(c.bytes.data(), host, nbytes) == 0;
     if (nbytes > 0 && !same) {
         // pageable source; the buffer may still be read by earlier work on the stream
@@ -166,7 +166,7 @@ static int table_to_device(int slot, const void* host, size_t nbytes, TableCache
         TH_HIP(hipMemcpy(d, host, nbytes, hipMemcpyHostToDevice));
         c.bytes.assign((const unsigned char*)host, (const unsigned char*)host + nbytes);
         c.buf = d;
-        c.gen = ws_generation();
+        c.gen = ws_generation(slot);
         c.dev = dev;
     }
     *out = d;

@@ -1239,6 +1239,7 @@ struct TableCache {
     TableKey key{-1, 0, 0, 0, 0, 0};
     int device = -1;
     void* ptr = nullptr;
+    unsigned long long gen = 0;  // workspace generation: a released buffer may come back at its address
 };
 static thread_local TableCache g_tab;
 
@@ -1263,7 +1264,9 @@ static int table_for(const TableKey& key, int P, hipStream_t st, char** dtab, fl
     TH_TRY(ws_get(WS_TABLE, cs_off + cs_bytes + 256, &buf));
     *dtab = (char*)buf;
     *dcs = key.sum == 1 ? (float2*)((char*)buf + cs_off) : nullptr;
-    if (g_tab.key == key && g_tab.device == dev && g_tab.ptr == buf) return TIRA_OK;
+    if (g_tab.key == key && g_tab.device == dev && g_tab.ptr == buf && g_tab.gen == ws_generation(WS_TABLE))
+        return TIRA_OK;
+    g_tab.device = -1;
     if (key.sum == 2) {
         build_atv3_table(key.w, key.s1, tab);
     } else if (key.sum == 1) {
@@ -1285,6 +1288,7 @@ static int table_for(const TableKey& key, int P, hipStream_t st, char** dtab, fl
     g_tab.key = key;
     g_tab.device = dev;
     g_tab.ptr = buf;
+    g_tab.gen = ws_generation(WS_TABLE);
     return TIRA_OK;
 }
 
@@ -1471,6 +1475,7 @@ struct MlpTabCache {
     float s1 = 0, s2 = 0;
     int device = -1;
     void* ptr = nullptr;
+    unsigned long long gen = 0;
 };
 static thread_local MlpTabCache g_mtab;
 
@@ -1481,13 +1486,16 @@ static int mlp_table_for(int w, float s1, float s2, hipStream_t st, float4** dta
     void* buf = nullptr;
     TH_TRY(ws_get(WS_TABLE3, bytes, &buf));
     *dtab = (float4*)buf;
-    if (g_mtab.w == w && g_mtab.s1 == s1 && g_mtab.s2 == s2 && g_mtab.device == dev && g_mtab.ptr == buf)
+    if (g_mtab.w == w && g_mtab.s1 == s1 && g_mtab.s2 == s2 && g_mtab.device == dev && g_mtab.ptr == buf &&
+        g_mtab.gen == ws_generation(WS_TABLE3))
         return TIRA_OK;
+    g_mtab.device = -1;
     std::vector<float4> t;
     build_mlp_table(w, s1, s2, t);
     TH_HIP(hipStreamSynchronize(st));
     TH_HIP(hipMemcpy(buf, t.data(), bytes, hipMemcpyHostToDevice));
     g_mtab.w = w; g_mtab.s1 = s1; g_mtab.s2 = s2; g_mtab.device = dev; g_mtab.ptr = buf;
+    g_mtab.gen = ws_generation(WS_TABLE3);
     return TIRA_OK;
 }
 
@@ -1497,6 +1505,7 @@ struct MlpCompactCache {
     unsigned power = 0;
     int device = -1;
     void* ptr = nullptr;
+    unsigned long long gen = 0;
 };
 static thread_local MlpCompactCache g_ctab;
 
@@ -1510,14 +1519,16 @@ static int mlptab_table_for(int P, int w, float s1, float s2, unsigned power, hi
     TH_TRY(ws_get(WS_TABLE4, bytes, &buf));
     *dtab = (float*)buf;
     if (g_ctab.P == P && g_ctab.w == w && g_ctab.s1 == s1 && g_ctab.s2 == s2 && g_ctab.power == power &&
-        g_ctab.device == dev && g_ctab.ptr == buf)
+        g_ctab.device == dev && g_ctab.ptr == buf && g_ctab.gen == ws_generation(WS_TABLE4))
         return TIRA_OK;
+    g_ctab.device = -1;
     std::vector<float> t;
     build_mlptab_table(P, w, s1, s2, power, t);
     TH_HIP(hipStreamSynchronize(st));
     TH_HIP(hipMemcpy(buf, t.data(), bytes, hipMemcpyHostToDevice));
     g_ctab.P = P; g_ctab.w = w; g_ctab.s1 = s1; g_ctab.s2 = s2; g_ctab.power = power; g_ctab.device = dev;
     g_ctab.ptr = buf;
+    g_ctab.gen = ws_generation(WS_TABLE4);
     return TIRA_OK;
 }
 
