@@ -73,3 +73,33 @@ def test_listed_session_bad_voter(hip, bad):
     np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
     ok = np.isfinite(ref)
     _close(got[ok], ref[ok], 13 * 13)
+
+
+@pytest.mark.parametrize("share", [0.05, 0.7])
+def test_session_of_a_device_field_still_being_written(hip, share):
+    """A session bound to device memory that work queued on the library's stream
+    still has to write (a long kernel ahead of the copy) holds what was written."""
+    import ctypes as C
+    from tiralib_amd import _lib
+    shape = (300, 260)
+    f, stale = _field(shape, share, 5), _field(shape, 0.02, 6)
+    src, field, busy = _lib.DeviceArray.from_host(f), _lib.DeviceArray.from_host(stale), _lib.DeviceArray((1024,))
+    h, st, got = C.c_void_p(), C.c_void_p(), np.empty(shape + (4,), np.float32)
+    _lib.call("tira_hip_stream_create", C.byref(st))
+    try:
+        _lib.call("tira_hip_set_stream", st)
+        _lib.call("tira_hip_fma_loop_async", busy.ptr, 1024, 1 << 18)  # tens of milliseconds
+        _lib.call("tira_hip_copy_async", field.ptr, src.ptr, f.nbytes)
+        _lib.call("tira_vote2_session_create", C.byref(h), field.ptr, *shape)
+        for p in (1, 3):
+            _lib.call("tira_vote2_session_vote", h, got.ctypes.data, None, 0, 3.0, 1.0, p, 19, 1, 1, 20)
+            with tvk.Session(f) as ref:
+                np.testing.assert_array_equal(got, ref.tensorvote_tk(3.0, 1.0, p, w=19))
+    finally:
+        _lib.call("tira_hip_synchronize")
+        _lib.call("tira_hip_set_stream", None)
+        if h:
+            _lib.call("tira_vote2_session_destroy", h)
+        _lib.call("tira_hip_stream_destroy", st)
+        for d in (src, field, busy):
+            d.free()

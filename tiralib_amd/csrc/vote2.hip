@@ -1156,7 +1156,13 @@ int tira_vote2_session_create(void** session, const float* t_in, unsigned s0, un
             st = TIRA_ERR_OUT_OF_MEMORY;
             break;
         }
-        if (hipMemcpy(s->field, t_in, bytes, hipMemcpyDefault) != hipSuccess) {
+        // The field may be device memory that the library stream or the null stream
+        // is still writing, and a copy between device buffers need not have ended
+        // when hipMemcpy returns: both are waited for, so that the list below and
+        // votes on any stream read the whole field.
+        if (hipStreamSynchronize(stream()) != hipSuccess ||
+            hipMemcpy(s->field, t_in, bytes, hipMemcpyDefault) != hipSuccess ||
+            hipStreamSynchronize(nullptr) != hipSuccess) {
             set_error("copying the field into the vote session failed");
             st = TIRA_ERR_HIP;
             break;
