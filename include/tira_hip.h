@@ -172,9 +172,11 @@ int tira_build_neighbors2d_async(int w, float sigma1, float sigma2, unsigned pow
  * (tira_build_neighbors2d_async). Each session keeps the device copies of its
  * last 64 tables (keyed by parameters or by the table's bytes) and runs each
  * vote as one replay of an instantiated graph. Results are identical to
- * tira_tensorvote2_prebuilt with the same table; with a device-built table
- * they are within a few FP32 ulps of tira_tensorvote2 (whose host table can
- * differ in c1, c2 by one ulp). t_out host or device; blocking.
+ * tira_tensorvote2_prebuilt with the same table. With nb == NULL a field of few
+ * voters is summed voter by voter, in another order than tira_tensorvote2 and
+ * with FP64 partial sums: the two differ by FP32 rounding (2e-7 of the field's
+ * 2-norm, up to 1e-6 of its largest component), and neither is further from
+ * 64 bits than the other. t_out host or device; blocking.
  * A session belongs to the device current at create; calls on one session
  * must not overlap. */
 int tira_vote2_session_create(void** session, const float* t_in, unsigned s0, unsigned s1);

@@ -103,3 +103,19 @@ def test_session_of_a_device_field_still_being_written(hip, share):
         _lib.call("tira_hip_stream_destroy", st)
         for d in (src, field, busy):
             d.free()
+
+
+@pytest.mark.parametrize("share", [0.1, 0.7])
+@pytest.mark.parametrize("s1,s2,p", [(14.0, 0.0, 29), (12.0, 2.0, 23), (8.0, 8.0, 30)])
+def test_vote_scale_at_high_powers(hip, oracle, share, s1, s2, p):
+    """The common scale of a vote at high powers against FP64: the least-squares
+    factor between the two fields. What scales all sticks alike is the norm (one
+    rounding, 6e-8) and the sums' bias (below one rounding); the float product of p
+    ratios that the norm was taken from is 4e-7 off at p = 29."""
+    f = _field((48, 56), share, 11)
+    w = 2 * int(3 * max(s1, s2)) + 1
+    ref = oracle.tensorvote2_f64(f, s1, s2, p, w, True, False, 20, nthreads=8)
+    with tvk.Session(f) as s:
+        for got in (s.tensorvote_tk(s1, s2, p, w=w, plate=False), tvk.tensorvote_tk(f, s1, s2, p, w=w, plate=False)):
+            scale = ((got.astype(np.float64) - ref) * ref).sum() / (ref * ref).sum()
+            assert abs(scale) <= (1.3e-7 if s2 == 0.0 else 2.5e-7), scale

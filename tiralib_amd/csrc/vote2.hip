@@ -59,6 +59,15 @@ __host__ __device__ float stick_norm_2d(float s1, float s2, unsigned power) {
     return ratio / ((float)M_PI * (s1 * s1 + s2 * s2));
 }
 
+// The same in FP64, rounded once: the scale of a whole vote's sticks. The float
+// product above is within p roundings of it (4.7e-7 at p = 29, more than all
+// the rounding of the sums); the neighbour table keeps the reference's.
+static float stick_scale_2d(float s1, float s2, unsigned power) {
+    double ratio = 1.0;
+    for (unsigned k = 1; k <= power; ++k) ratio *= (2.0 * k) / (2.0 * k - 1.0);
+    return (float)(ratio / (M_PI * ((double)s1 * s1 + (double)s2 * s2)));
+}
+
 __host__ __device__ inline void stickvote_2d(float rx, float ry, float s1, float s2, unsigned power, float theta,
                                              float& Va, float& Vb, float& Vc) {
 #pragma clang fp contract(off)
@@ -207,7 +216,8 @@ __global__ __launch_bounds__(256) void k_vote2_prep_tk(const float2* __restrict_
 }
 
 // (t1^p, t2^p) for a wave-uniform p >= 1 by squaring: about 2 log2 p products
-// each instead of p - 1.
+// each instead of p - 1. (In FP64 the powers brought the error of a search
+// population from 2.9e-7 to 2.8e-7 and cost the generation 5%.)
 __device__ __forceinline__ void pow_pair(float t1, float t2, int p, float& e1, float& e2) {
     e1 = e2 = 1.0f;
     for (;;) {
@@ -292,12 +302,13 @@ __global__ __launch_bounds__(256) void k_vote2_reduce(const float4* __restrict__
                                                       float* __restrict__ out) {
     const size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
-    float4 v = part[p];
+    const float4 v = part[p];
+    double a = v.x, b = v.y, c = v.z;
     for (int z = 1; z < chunks; z++) {
         const float4 q = part[(size_t)z * n + p];
-        v.x += q.x; v.y += q.y; v.z += q.z;
+        a += q.x; b += q.y; c += q.z;
     }
-    reinterpret_cast<float4*>(out)[p] = make_float4(v.x, v.y, v.y, v.z);
+    reinterpret_cast<float4*>(out)[p] = make_float4((float)a, (float)b, (float)b, (float)c);
 }
 
 // ---------------------------------------------------------------- listed gather
@@ -317,8 +328,8 @@ constexpr int kTile2 = 8;
 
 // The w x w table as a grid of two float4 planes, (dx, dy, c1, c2) and
 // (Va, Vb, Vc, 0), padded by a tile's edge on every side; padding has c1 = -1.
-// The reflection R of the 48-byte entry is I - 2 d d^T and is applied as
-// q - 2 (q.d) d: a third of the bytes and two products less per pair.
+// The reflection R = I - 2 d d^T of the 48-byte entry is formed from d per
+// pair: a third of the bytes.
 __host__ __device__ inline int grid2_edge(int w) { return w / 2 * 2 + 2 * kTile2 - 1; }
 __global__ __launch_bounds__(256) void k_build_grid2(int w, float s1, float s2, unsigned power, unsigned samples,
                                                      int stick, int plate, float4* __restrict__ out) {
@@ -416,7 +427,7 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
     const unsigned n = (unsigned)(D * D);
     const unsigned lane_off = (unsigned)((kTile2 - 1 - (lane >> 3)) * D + (kTile2 - 1 - (lane & 7))) * 16u;
     const int xlo = max(x0 - r, 0), xhi = min(x0 + kTile2 - 1 + r, s1 - 1);
-    float3 s = make_float3(0.0f, 0.0f, 0.0f);
+    double sx = 0.0, sy = 0.0, sz = 0.0;
     for (int xb = xlo / 64; xb <= xhi / 64; xb++) {
         const unsigned row = (unsigned)(xb * s0);
         const unsigned k0 = seg_start(cnt, tot, row + ylo), k1 = seg_start(cnt, tot, row + yhi);
@@ -439,7 +450,9 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
             // two entries in turn: the next voter's is in flight while this one is evaluated
             Grid2Entry ea, eb;
             int ja = __builtin_ctzll(m), jb = 0;
-            float3 t = make_float3(0.0f, 0.0f, 0.0f);  // up to 64 voters' sum: shorter chains than one running sum
+            // the sums of up to 32 voters each, added up in FP64: one running sum had the
+            // longer chains of the two gathers, and was the further from FP64
+            float3 ta = make_float3(0.0f, 0.0f, 0.0f), tb = ta;
             grid2_fetch<PLATE>(grid, n, __builtin_amdgcn_readlane(base, ja), lane_off, ea);
             for (;;) {
                 m &= m - 1;
@@ -448,7 +461,7 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
                     grid2_fetch<PLATE>(grid, n, __builtin_amdgcn_readlane(base, jb), lane_off, eb);
                 }
                 listed2_pair<STICK, PLATE, P1>(lane_f(v.x, ja), lane_f(v.y, ja), lane_f(v.z, ja), lane_f(v.w, ja), ea,
-                                               power, t);
+                                               power, ta);
                 if (!m) break;
                 m &= m - 1;
                 if (m) {
@@ -456,15 +469,15 @@ __device__ __forceinline__ float3 listed2_sum(const float4* __restrict__ lv, con
                     grid2_fetch<PLATE>(grid, n, __builtin_amdgcn_readlane(base, ja), lane_off, ea);
                 }
                 listed2_pair<STICK, PLATE, P1>(lane_f(v.x, jb), lane_f(v.y, jb), lane_f(v.z, jb), lane_f(v.w, jb), eb,
-                                               power, t);
+                                               power, tb);
                 if (!m) break;
             }
-            s.x += t.x;
-            s.y += t.y;
-            s.z += t.z;
+            sx += (double)ta.x + tb.x;
+            sy += (double)ta.y + tb.y;
+            sz += (double)ta.z + tb.z;
         }
     }
-    return s;
+    return make_float3((float)sx, (float)sy, (float)sz);
 }
 
 __global__ __launch_bounds__(256) void k_vote2_listed(const float4* __restrict__ lv, const unsigned* __restrict__ lp,
@@ -683,7 +696,7 @@ static int vote2_launch(const float* tin, const float* lam, const float* th, flo
                         unsigned samples, float4* part, hipStream_t st) {
     const size_t n = (size_t)s0 * s1n;
     const unsigned p = power < 1 ? 1 : (unsigned)power;
-    const float eta_s = stick_norm_2d(s1, s2, p);
+    const float eta_s = stick_scale_2d(s1, s2, p);
     {
         ProfScope prof("vote2_prep", st);
         if (tin) k_vote2_prep<<<ceil_div(n, 256), 256, 0, st>>>((const float4*)tin, n, eta_s, pay);
@@ -1212,7 +1225,7 @@ int tira_vote2_session_vote(void* session, float* t_out, const void* nb, int nb_
         s.part_cap = part_bytes;
     }
     SessionArgs a;
-    a.field = s.field; a.n = s.n; a.eta_s = stick_norm_2d(sigma1, sigma2, p); a.pay = s.pay;
+    a.field = s.field; a.n = s.n; a.eta_s = stick_scale_2d(sigma1, sigma2, p); a.pay = s.pay;
     a.nb = dnb; a.nbc = nbc; a.per = vote2_per(nbc, chunks); a.s0 = (int)s.s0; a.s1 = (int)s.s1;
     a.power = (int)p; a.stick = stick ? 1 : 0; a.plate = use_plate ? 1 : 0;
     a.out = host_out ? (float*)s.out : t_out;

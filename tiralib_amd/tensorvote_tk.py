@@ -14,8 +14,10 @@ optimize.py:256-288), bind the field once:
         out = s.tensorvote_tk_prebuilt(nb_buf, nb_count, w, sigma1, sigma2, power)
 
 The session keeps the field and its recent neighbour tables on the device and
-runs each vote as one graph replay; results are identical to the module
-functions.
+runs each vote as one graph replay. With a caller's table the results are those
+of the module function, bit for bit; a vote from parameters may be summed in
+another order (a field of few voters voter by voter), so it agrees with the
+module function to FP32 rounding.
 """
 from __future__ import annotations
 
