@@ -126,3 +126,45 @@ def test_stick_of_other_length_is_voted_by_window(hip):
                     V += sn * s * eta * np.outer(r, r)
         g = out[name].reshape(shape + (3, 3))[at]
         assert np.abs(g - V).max() <= 1e-5 * np.abs(V).max(), name
+
+
+@pytest.mark.parametrize("power", [2, 3, 4])
+@pytest.mark.parametrize("normal", [(0, 0, 1), (0, 1, 0), (1, 0, 0), (0, .6, .8), (.6, .8, 0), (.8, 0, .6), (.48, .6, .64)])
+@pytest.mark.parametrize("scale", [1e38, 3e36])
+def test_wild_plate_is_voted_by_window(hip, power, normal, scale):
+    """A finite plate whose features overflow (all of them to NaN where the normal has
+    a zero component) leaves the rest of the volume as the window gather has it."""
+    shape, w, at = (32, 34, 36), 11, (15, 16, 17)
+    f = _field(shape, seed=5)
+    n = np.array(normal, np.float64)
+    f[at] = (scale * (np.eye(3) - np.outer(n, n))).astype(np.float32).ravel()
+    got, _ = _run(f, shape, _lib.PLATE_AUTO, 2.0, 0.0, w, power)
+    ref, _ = _run(f, shape, _lib.PLATE_CLOSED, 2.0, 0.0, w, power)
+    inside = np.zeros(shape, bool)
+    inside[tuple(slice(c - w // 2, c + w // 2 + 1) for c in at)] = True
+    assert np.isfinite(ref[~inside]).all()
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(ref))
+    assert np.abs(got[~inside].astype(np.float64) - ref[~inside]).max() <= 1e-5 * np.abs(ref[~inside]).max()
+
+
+@pytest.mark.parametrize("power", [2, 3, 4])
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 3e38])
+def test_wild_eigenvalue_is_voted_by_window(hip, power, bad):
+    """The same through eigenpair input, plates only and sticks only."""
+    shape, w, at = (32, 34, 36), 11, (15, 16, 17)
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(power)
+    e = np.linalg.qr(rng.normal(size=(n, 3, 3)))[0]
+    e[np.ravel_multi_index(at, shape)] = np.eye(3)  # zero components
+    e2, e0 = (np.ascontiguousarray(e[:, :, k], np.float32) for k in (0, 1))
+    lam = np.sort(rng.random((n, 3)), axis=1).astype(np.float32)
+    lam[np.ravel_multi_index(at, shape)] = 0
+    inside = np.zeros(shape, bool)
+    inside[tuple(slice(c - w // 2, c + w // 2 + 1) for c in at)] = True
+    for stick, plate in ((False, True), (True, False)):
+        clean = api.tensorvote3_tk(lam, e2, e0, shape, 1.5, 0.0, power, w, stick, plate, 20).reshape(shape + (9,))
+        l = lam.copy()
+        l[np.ravel_multi_index(at, shape), 1 if plate else 2] = bad
+        got = api.tensorvote3_tk(l, e2, e0, shape, 1.5, 0.0, power, w, stick, plate, 20).reshape(shape + (9,))
+        assert np.isfinite(got[~inside]).all()
+        assert np.abs(got[~inside].astype(np.float64) - clean[~inside]).max() <= 1e-5 * np.abs(clean[~inside]).max()

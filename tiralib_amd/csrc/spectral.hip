@@ -914,15 +914,15 @@ __global__ __launch_bounds__(kFT, P == 1 ? 4 : 2) void k_spec_xfwd(
                     voter_features<(P > 1 ? P : 2)>(S, make_float4(N.x, N.y, N.z, N.w * g.alpha), g.stick != 0,
                                                     g.plate != 0, A);
                     if (NF & 1) A[NF] = 0.0f;
-                    float big = 0.0f;
-#pragma unroll
-                    for (int m = 0; m < NF; m++) big = fmaxf(big, fabsf(A[m]));
-                    // fmaxf drops NaN: a NaN feature shows in the sum of squares of the voter
+                    // The scales themselves: features formed from one that is not finite
+                    // can all be NaN, which no maximum over them shows.
+                    const bool big = (g.stick && !(fabsf(S.w) < kSpecWild)) ||
+                                     (g.plate && !(fabsf(N.w * g.alpha) < kSpecWild));
                     const float nan = fmaf(S.w, S.x + S.y + S.z, N.w * (N.x + N.y + N.z));
                     // the features take a stick of unit length (a caller's eigenvectors need not be)
                     const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
                     const bool odd = g.stick && S.w != 0.0f && !(fabsf(q2 - 1.0f) < 2e-6f);
-                    if (wild && (!(big < kSpecWild) || nan != nan || odd)) atomicAdd(wild, 1ull);
+                    if (wild && (big || nan != nan || odd)) atomicAdd(wild, 1ull);
                 } else {
                     mono15(g.stick ? S : make_float4(0.0f, 0.0f, 0.0f, 0.0f), A);
                     A[NF] = 0.0f;
