@@ -168,3 +168,34 @@ def test_wild_eigenvalue_is_voted_by_window(hip, power, bad):
         got = api.tensorvote3_tk(l, e2, e0, shape, 1.5, 0.0, power, w, stick, plate, 20).reshape(shape + (9,))
         assert np.isfinite(got[~inside]).all()
         assert np.abs(got[~inside].astype(np.float64) - clean[~inside]).max() <= 1e-5 * np.abs(clean[~inside]).max()
+
+
+@pytest.mark.parametrize("wild", [False, True])
+@pytest.mark.parametrize("power", [2, 4])
+def test_input_may_lie_in_the_output(hip, power, wild):
+    """Eigenpairs in the memory of the output, and a field voted in place: as with an
+    output of its own, also where a voter has the field voted by window."""
+    shape, w = (32, 33, 35), 11
+    n = int(np.prod(shape))
+    rng = np.random.default_rng(7)
+    e = np.linalg.qr(rng.normal(size=(n, 3, 3)))[0].astype(np.float32)
+    lam = np.sort(rng.random((n, 3)), axis=1).astype(np.float32)
+    f = _field(shape, seed=9).reshape(n, 9)
+    if wild:
+        lam[n // 2] = np.inf
+        f[n // 2] = np.inf
+    parts = np.concatenate([lam.ravel(), e[:, :, 0].ravel(), e[:, :, 1].ravel()])
+    one, own, two = _lib.DeviceArray.from_host(parts), _lib.DeviceArray((n, 9)), _lib.DeviceArray.from_host(f)
+    try:
+        src = [one.ptr + 12 * n * k for k in range(3)]
+        for out in (own.ptr, one.ptr):
+            _lib.call("tira_tensorvote3_tk", out, *src, *shape, 1.5, 0.0, power, w, 1, 1, 20)
+        np.testing.assert_array_equal(one.to_host().reshape(n, 9), own.to_host())
+        assert np.isfinite(own.to_host()).any()
+        for out in (own, two):
+            api.tensorvote3_async(two, out, shape, 1.5, 0.0, w, power)
+        _lib.call("tira_hip_synchronize")
+        np.testing.assert_array_equal(two.to_host(), own.to_host())
+    finally:
+        for d in (one, own, two):
+            d.free()

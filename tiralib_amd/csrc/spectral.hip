@@ -70,7 +70,6 @@ constexpr int kMaxL = 1024;    // longest transform
 constexpr int kMaxStages = 16;
 constexpr int kMono = 15;      // quartic monomials
 constexpr unsigned kSpecMaxPower = 4;
-constexpr float kSpecWild = 1e30f;  // features from here on could overflow the transforms
 // Monomials of the degree 2 p + 2 of a power-p vote.
 __host__ __device__ constexpr int mono_count(int power) { return (2 * power + 3) * (power + 2); }
 constexpr int kMaxMono = mono_count((int)kSpecMaxPower);
@@ -855,14 +854,11 @@ __device__ __forceinline__ void voter_features(const float4 S, const float4 N, b
 // voxel).
 // Four waves per SIMD (at most 128 VGPRs): unbounded, the eigen-solve and the
 // features take 136 and three waves; bounded, they fit in 120 without a spill.
-// wild (power above 1): set when a feature is not finite or so large that the
-// transforms' sums could overflow, for the caller to vote by window instead.
-template <bool FROM_TENSORS, int P>
-__global__ __launch_bounds__(kFT, P == 1 ? 4 : 2) void k_spec_xfwd(
-    const float4* __restrict__ ps, const float4* __restrict__ pp, const float* __restrict__ tensors, int layout,
-    SpecGeom g, int B, int C, int FG, FftPlan pl, const float2* __restrict__ twg, float2* __restrict__ Z,
-    unsigned long long* __restrict__ wild) {
-    constexpr int NF = mono_count(P);
+template <bool FROM_TENSORS>
+__global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__ ps, const float4* __restrict__ pp,
+                                                   const float* __restrict__ tensors, int layout, SpecGeom g, int B,
+                                                   int C, int FG, FftPlan pl, const float2* __restrict__ twg,
+                                                   float2* __restrict__ Z) {
     extern __shared__ float2 xs_dyn[];  // C B L staged values, then L twiddles
     const int L = pl.L;
     float2* s = xs_dyn;
@@ -891,7 +887,8 @@ __global__ __launch_bounds__(kFT, P == 1 ? 4 : 2) void k_spec_xfwd(
             // part); the stick features are written first, zero when the vote
             // has no stick part (zeroing A ahead of the eigen-solve kept 15
             // registers live through it and spilled 80 bytes per lane)
-            float A[(NF + 2) & ~1];
+            float A[kMono + 1];
+            A[kMono] = 0.0f;
             {
                 const size_t vox = (size_t)(row0 + b) * g.n2 + e;
                 float4 S = make_float4(0.0f, 0.0f, 0.0f, 0.0f), N = S;
@@ -910,25 +907,9 @@ __global__ __launch_bounds__(kFT, P == 1 ? 4 : 2) void k_spec_xfwd(
                     if (g.stick) S = ps[vox];
                     if (g.plate) N = pp[vox];
                 }
-                if (P > 1) {
-                    voter_features<(P > 1 ? P : 2)>(S, make_float4(N.x, N.y, N.z, N.w * g.alpha), g.stick != 0,
-                                                    g.plate != 0, A);
-                    if (NF & 1) A[NF] = 0.0f;
-                    // The scales themselves: features formed from one that is not finite
-                    // can all be NaN, which no maximum over them shows.
-                    const bool big = (g.stick && !(fabsf(S.w) < kSpecWild)) ||
-                                     (g.plate && !(fabsf(N.w * g.alpha) < kSpecWild));
-                    const float nan = fmaf(S.w, S.x + S.y + S.z, N.w * (N.x + N.y + N.z));
-                    // the features take a stick of unit length (a caller's eigenvectors need not be)
-                    const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
-                    const bool odd = g.stick && S.w != 0.0f && !(fabsf(q2 - 1.0f) < 2e-6f);
-                    if (wild && (big || nan != nan || odd)) atomicAdd(wild, 1ull);
-                } else {
-                    mono15(g.stick ? S : make_float4(0.0f, 0.0f, 0.0f, 0.0f), A);
-                    A[NF] = 0.0f;
-                    if (g.plate) add_circle_average(make_float4(N.x, N.y, N.z, N.w * g.alpha), A);
-                }
-                if (P == 1 && g.atv) {  // three times the sphere averages: 1/5 for x^4, 1/15 for x^2 y^2
+                mono15(g.stick ? S : make_float4(0.0f, 0.0f, 0.0f, 0.0f), A);
+                if (g.plate) add_circle_average(make_float4(N.x, N.y, N.z, N.w * g.alpha), A);
+                if (g.atv) {  // three times the sphere averages: 1/5 for x^4, 1/15 for x^2 y^2
                     A[0] = fmaf(0.6f, s3, A[0]);
                     A[3] = fmaf(0.2f, s3, A[3]);
                     A[5] = fmaf(0.2f, s3, A[5]);
@@ -938,13 +919,66 @@ __global__ __launch_bounds__(kFT, P == 1 ? 4 : 2) void k_spec_xfwd(
                 }
             }
 #pragma unroll
-            for (int j = 0; j < (NF + 1) / 2; j++)
+            for (int j = 0; j < (kMono + 1) / 2; j++)
                 if (j >= j0 && j < j0 + Cv) s[((j - j0) * Bv + b) * L + e] = make_float2(A[2 * j], A[2 * j + 1]);
         }
         __syncthreads();
         // the staged lines in groups of FG (each group fits the stages' register rounds)
         for (int l0 = 0; l0 < Cv * Bv; l0 += FG) fft_lines<false>(s + l0 * L, pl, min(FG, Cv * Bv - l0), tw);
         // each wave stores whole lines (their bases are wave-uniform)
+        for (int line = (int)threadIdx.x >> 6; line < Cv * Bv; line += kFT / 64) {
+            const int ln = __builtin_amdgcn_readfirstlane(line);
+            const int c = fdiv(ln, Bv, rB), b = ln - c * Bv;
+            const int row = row0 + b;
+            const int z = fdiv(row, g.n1, rn1), y = row - z * g.n1;
+            float2* dst = Z + (size_t)(j0 + c) * g.cs + ((size_t)z * g.L1 + y) * g.P2;
+            for (int e = (int)threadIdx.x & 63; e < L; e += 64) dst[e] = s[ln * L + e];
+        }
+    }
+}
+
+// The same for powers above 1, from the padded voter payloads of the window
+// gather (vg): they are formed before this vote, with the FP64 re-solve of close
+// pairs, and serve the gather too where it has to vote instead.
+template <int P>
+__global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restrict__ ps, const float4* __restrict__ pp,
+                                                          VoteGeom vg, SpecGeom g, int B, int C, int FG, FftPlan pl,
+                                                          const float2* __restrict__ twg, float2* __restrict__ Z) {
+    constexpr int NF = mono_count(P);
+    extern __shared__ float2 xs_dyn[];  // C B L staged values, then L twiddles
+    const int L = pl.L;
+    float2* s = xs_dyn;
+    float2* tw = xs_dyn + C * B * L;
+    const int row0 = (int)blockIdx.x * B;
+    const int nrows = g.n0 * g.n1;
+    if (row0 >= nrows) return;
+    const int Bv = min(B, nrows - row0);
+    load_twiddles(tw, twg, L);
+    const int npad = L - g.n2;
+    const float rB = 1.0f / (float)Bv, rn1 = 1.0f / (float)g.n1, rn2 = 1.0f / (float)g.n2,
+                rpad = 1.0f / (float)max(npad, 1);
+    for (int j0 = 0; j0 < g.nz; j0 += C) {
+        const int Cv = min(C, g.nz - j0);
+        if (j0) __syncthreads();  // the previous group's stores have read s
+        for (int idx = (int)threadIdx.x; idx < Cv * Bv * npad; idx += kFT) {
+            const int line = fdiv(idx, npad, rpad);
+            s[line * L + g.n2 + (idx - line * npad)] = make_float2(0.0f, 0.0f);
+        }
+        for (int idx = (int)threadIdx.x; idx < Bv * g.n2; idx += kFT) {
+            const int b = fdiv(idx, g.n2, rn2), e = idx - b * g.n2;
+            const int row = row0 + b, z = fdiv(row, g.n1, rn1), y = row - z * g.n1;
+            const size_t v = ((size_t)(z + vg.r) * vg.P1 + y + vg.r) * vg.P2 + e + vg.r;
+            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const float4 S = g.stick ? ps[v] : zero, N = g.plate ? pp[v] : zero;
+            float A[(NF + 2) & ~1];
+            voter_features<P>(S, make_float4(N.x, N.y, N.z, N.w * g.alpha), g.stick != 0, g.plate != 0, A);
+            if (NF & 1) A[NF] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < (NF + 1) / 2; j++)
+                if (j >= j0 && j < j0 + Cv) s[((j - j0) * Bv + b) * L + e] = make_float2(A[2 * j], A[2 * j + 1]);
+        }
+        __syncthreads();
+        for (int l0 = 0; l0 < Cv * Bv; l0 += FG) fft_lines<false>(s + l0 * L, pl, min(FG, Cv * Bv - l0), tw);
         for (int line = (int)threadIdx.x >> 6; line < Cv * Bv; line += kFT / 64) {
             const int ln = __builtin_amdgcn_readfirstlane(line);
             const int c = fdiv(ln, Bv, rB), b = ln - c * Bv;
@@ -1669,8 +1703,9 @@ bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsig
     const size_t nf = (size_t)mono_count((int)p), nz = (nf + 1) / 2;  // the combined features
     const size_t W = 2 * (w / 2) + 1;
     const size_t h0 = L0 / 2 + 1, h1 = L1 / 2 + 1, h2 = L2 / 2 + 1;
-    const size_t need = nz * (size_t)L0 * L1 * L2 * 8 + 6 * nf * h0 * h1 * h2 * 4 + 6 * nf * W * h1 * h2 * 8 +
-                        (size_t)s0 * s1 * s2 * 32;
+    // payloads: of the field, above power 1 padded for the window gather
+    const size_t pay = p == 1 ? (size_t)s0 * s1 * s2 : vote3_payload_voxels(s0, s1, s2, (unsigned)W);
+    const size_t need = nz * (size_t)L0 * L1 * L2 * 8 + 6 * nf * h0 * h1 * h2 * 4 + 6 * nf * W * h1 * h2 * 8 + pay * 32;
     size_t free_b = 0, total_b = 0;
     int dev = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
@@ -1683,28 +1718,25 @@ bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsig
     return need <= total_b / 10 * 8 && need <= (free_b + held) / 10 * 9;
 }
 
-template <bool FROM_TENSORS>
-static void launch_xfwd(int power, unsigned grid, size_t lds, hipStream_t st, const float4* ps, const float4* pp,
-                        const float* tensors, int layout, const SpecGeom& g, int B, int C, int FG, const FftPlan& pl,
-                        const float2* tw, float2* Z, unsigned long long* wild) {
+static void launch_xfwd_pay(int power, unsigned grid, size_t lds, hipStream_t st, const SpecPayload& v,
+                            const SpecGeom& g, int B, int C, int FG, const FftPlan& pl, const float2* tw, float2* Z) {
     switch (power) {
-        case 1: k_spec_xfwd<FROM_TENSORS, 1><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
-        case 2: k_spec_xfwd<FROM_TENSORS, 2><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
-        case 3: k_spec_xfwd<FROM_TENSORS, 3><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
-        default: k_spec_xfwd<FROM_TENSORS, 4><<<grid, kFT, lds, st>>>(ps, pp, tensors, layout, g, B, C, FG, pl, tw, Z, wild); break;
+        case 2: k_spec_xfwd_pay<2><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z); break;
+        case 3: k_spec_xfwd_pay<3><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z); break;
+        default: k_spec_xfwd_pay<4><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z); break;
     }
 }
 
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        float* out, int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1,
                        float sigma2, unsigned w, unsigned power, bool stick, bool plate, unsigned samples,
-                       bool atv, hipStream_t st, EigOut* eig, unsigned long long* wild) {
+                       bool atv, hipStream_t st, EigOut* eig, const SpecPayload* pay) {
     const unsigned p = power < 1 || atv ? 1 : power;
     if (atv) {  // sigma2, power, stick, plate and samples do not apply to ATV
         stick = plate = true;
         sigma2 = 0.0f;
         if (!tensors) return kSpectralNotApplicable;
-    } else if (!spectral_serves(p, plate, samples)) {
+    } else if (!spectral_serves(p, plate, samples) || (p > 1) != (pay != nullptr)) {
         return kSpectralNotApplicable;
     }
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);
@@ -1773,7 +1805,7 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     const size_t xlds = ((size_t)C * B * g.L2 + g.L2) * 8;
     // tensor input: the x pass decomposes the voxels itself, in every channel
     // group (no payload round trip); eigenpair input goes through the payload
-    const bool fused = tensors != nullptr;
+    const bool fused = pay || tensors != nullptr;
     float4 *ps = nullptr, *pp = nullptr;
     float2* Z = nullptr;
     // Out of device memory for the spectral buffers: clear the error and let
@@ -1806,10 +1838,12 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
         const size_t nrows = (size_t)s0 * s1;
         const size_t nblk = ceil_div(nrows, (size_t)B);
         TH_ARG(nblk < (1ull << 31), "spectral vote: volume too large");
-        if (fused)
-            launch_xfwd<true>(g.power, (unsigned)nblk, xlds, st, ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z, wild);
+        if (pay)
+            launch_xfwd_pay(g.power, (unsigned)nblk, xlds, st, *pay, g, B, C, FG, p2, tw2, Z);
+        else if (fused)
+            k_spec_xfwd<true><<<(unsigned)nblk, kFT, xlds, st>>>(ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z);
         else
-            launch_xfwd<false>(g.power, (unsigned)nblk, xlds, st, ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z, wild);
+            k_spec_xfwd<false><<<(unsigned)nblk, kFT, xlds, st>>>(ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z);
         TH_HIP(hipGetLastError());
     }
     {

@@ -595,12 +595,32 @@ __device__ __forceinline__ void plate_basis(const float n[3], float u[3], float 
     v[2] = n[0] * u[1] - n[1] * u[0];
 }
 
+// Voters that a spectral vote would spread beyond their window: not finite, of
+// a scale whose sums in the transforms could overflow (the scale itself is
+// tested: of features formed from it, all can be NaN), or a caller's stick that
+// is not of unit length, which the features take.
+constexpr float kWildScale = 1e30f;
+__device__ __forceinline__ bool wild_stick(const float4 S) {
+    const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
+    if (S.w == 0.0f) return !(q2 < kWildScale);
+    return !(fabsf(S.w) < kWildScale) || !(fabsf(q2 - 1.0f) < 2e-6f);
+}
+// alpha: the factor of the plate's features (sticknorm3).
+__device__ __forceinline__ bool wild_plate(const float4 N, float alpha) {
+    return !(fabsf(N.w * alpha) < kWildScale) || !(fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z)) < 2.0f);
+}
+// Raises *flag if any lane's voters were wild (equal stores do not queue up).
+__device__ __forceinline__ void raise_wild(bool wild, unsigned long long* flag) {
+    if (flag && __any(wild) && (threadIdx.x & 63) == 0) *flag = 1ull;
+}
+
 // Writes the voter payload for one voxel given its eigen-decomposition.
 __device__ __forceinline__ void write_payload(const VoteGeom& g, size_t pidx, float l0, float l1, float l2,
                                               const float* e0, const float* e2, float4* pay_s, float4* pay_p,
-                                              float4* pay_v, float sum_inv_n) {
+                                              float4* pay_v, float sum_inv_n, float alpha, bool& wild) {
     float4 S, N;
     stick_plate_payload(l0, l1, l2, e0, e2, S, N);
+    wild = wild || (pay_s && wild_stick(S)) || (pay_p && wild_plate(N, alpha));
     if (pay_s) pay_s[pidx] = S;
     if (pay_p) {
         if (!pay_v) {
@@ -616,12 +636,13 @@ __device__ __forceinline__ void write_payload(const VoteGeom& g, size_t pidx, fl
 }
 
 // Grid-stride over the padded payload volume: voxels outside the field get a
-// zero payload. gate (optional): the launch does nothing while *gate == 0.
+// zero payload. wild (optional): raised if a voter is such that a spectral vote
+// cannot serve (wild_stick, wild_plate).
 __global__ __launch_bounds__(256) void k_vote3_prep(const float* __restrict__ in, int layout, VoteGeom g,
                                                     float4* __restrict__ pay_s, float4* __restrict__ pay_p,
                                                     float4* __restrict__ pay_v, float sum_inv_n,
-                                                    const unsigned long long* __restrict__ gate) {
-    if (gate && *gate == 0ull) return;
+                                                    float alpha, unsigned long long* __restrict__ wild) {
+    bool odd = false;
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
@@ -636,8 +657,9 @@ __global__ __launch_bounds__(256) void k_vote3_prep(const float* __restrict__ in
         const size_t v = ((size_t)z * g.s1 + y) * g.s2 + x;
         float l0, l1, l2, e0[3], e2[3];
         voxel_eig(in, layout, v, l0, l1, l2, e0, e2);
-        write_payload(g, p, l0, l1, l2, e0, e2, pay_s, pay_p, pay_v, sum_inv_n);
+        write_payload(g, p, l0, l1, l2, e0, e2, pay_s, pay_p, pay_v, sum_inv_n, alpha, odd);
     }
+    raise_wild(odd, wild);
 }
 
 // Payload from caller eigenpairs (_tensorvote3_tk inputs).
@@ -645,8 +667,8 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
                                                        const float* __restrict__ ev0, VoteGeom g,
                                                        float4* __restrict__ pay_s, float4* __restrict__ pay_p,
                                                        float4* __restrict__ pay_v, float sum_inv_n,
-                                                       const unsigned long long* __restrict__ gate) {
-    if (gate && *gate == 0ull) return;
+                                                       float alpha, unsigned long long* __restrict__ wild) {
+    bool odd = false;
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
@@ -662,8 +684,9 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
         const float z3[3] = {0, 0, 0};
         const float* e2 = ev2 ? ev2 + v * 3 : z3;
         const float* e0 = ev0 ? ev0 + v * 3 : z3;
-        write_payload(g, p, lam[v * 3], lam[v * 3 + 1], lam[v * 3 + 2], e0, e2, pay_s, pay_p, pay_v, sum_inv_n);
+        write_payload(g, p, lam[v * 3], lam[v * 3 + 1], lam[v * 3 + 2], e0, e2, pay_s, pay_p, pay_v, sum_inv_n, alpha, odd);
     }
+    raise_wild(odd, wild);
 }
 
 // ---------------------------------------------------------------- learned plate (MLP)
@@ -673,19 +696,18 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
 // surrogate's error check -- their plate votes come from the integrator (the
 // closed form of the N-sample sum). Without pay_u (the tabulated network)
 // a flagged voter gets plate scale 0 in pay_n and its (n, scale) in pay_f,
-// which is zero for every other voter. n_wild (optional) counts the voters
-// whose stick an FFT would spread beyond its window: not finite, or of a scale
-// whose sums could overflow.
-constexpr float kWildScale = 1e30f;
+// which is zero for every other voter. wild (optional): raised if there is a
+// stick that a spectral vote cannot serve (wild_stick).
 __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict__ in, int layout, VoteGeom g,
                                                         float4* __restrict__ pay_s, float4* __restrict__ pay_n,
                                                         float4* __restrict__ pay_u, float4* __restrict__ pay_f,
                                                         const float* __restrict__ bin_err, float tol,
                                                         unsigned long long* __restrict__ n_fallback,
-                                                        unsigned long long* __restrict__ n_wild) {
+                                                        unsigned long long* __restrict__ wild) {
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
-    unsigned nf = 0, wild = 0;
+    unsigned nf = 0;
+    bool odd = false;
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
         const int px = (int)(p % g.P2), py = (int)((p / g.P2) % g.P1), pz = (int)(p / ((size_t)g.P1 * g.P2));
         const int x = px - g.r, y = py - g.r, z = pz - g.r;
@@ -700,8 +722,9 @@ __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict_
         float l0, l1, l2, e0[3], e2[3];
         voxel_eig(in, layout, v, l0, l1, l2, e0, e2);
         const float ss = copysignf(fabsf(l2) - fabsf(l1), l2);
-        if (pay_s) pay_s[p] = make_float4(e2[0], e2[1], e2[2], ss);
-        wild += !(fabsf(ss) < kWildScale) || !isfinite(e2[0] + e2[1] + e2[2]) ? 1u : 0u;
+        const float4 S = make_float4(e2[0], e2[1], e2[2], ss);
+        if (pay_s) pay_s[p] = S;
+        odd = odd || wild_stick(S);
         float n[3] = {e0[0], e0[1], e0[2]};
         const float nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
         float sp = copysignf(fabsf(l1) - fabsf(l0), l1);
@@ -722,7 +745,7 @@ __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict_
         }
     }
     if (n_fallback && nf) atomicAdd(n_fallback, (unsigned long long)nf);
-    if (n_wild && wild) atomicAdd(n_wild, (unsigned long long)wild);
+    raise_wild(odd, wild);
 }
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -1199,6 +1222,14 @@ VoteGeom make_geom(unsigned s0, unsigned s1, unsigned s2, unsigned w, int bz) {
     return g;
 }
 
+constexpr int kBZ = 4;     // receivers per lane along z: closed, literal-sum and ATV gathers
+constexpr int kBZMlp = 8;  // the tabulated-network gather (its LDS rows are staged per offset column)
+
+size_t vote3_payload_voxels(unsigned s0, unsigned s1, unsigned s2, unsigned w) {
+    const VoteGeom g = make_geom(s0, s1, s2, w, kBZ);
+    return (size_t)g.P0 * g.P1 * g.P2;
+}
+
 // Unpadded voter payloads (stick (e2, scale), plate (e0, scale)) of every
 // voxel, for the spectral vote; either pointer may be NULL.
 int vote3_payload_flat(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
@@ -1209,8 +1240,8 @@ int vote3_payload_flat(const float* tensors, int in_layout, const float* lam, co
     g.P0 = (int)s0; g.P1 = (int)s1; g.P2 = (int)s2;
     const size_t n = (size_t)s0 * s1 * s2;
     const unsigned grid = (unsigned)std::min<size_t>(ceil_div(n, 256), 65536);
-    if (tensors) k_vote3_prep<<<grid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, nullptr, 1.0f, nullptr);
-    else k_vote3_prep_tk<<<grid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, nullptr, 1.0f, nullptr);
+    if (tensors) k_vote3_prep<<<grid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, nullptr, 1.0f, 1.0f, nullptr);
+    else k_vote3_prep_tk<<<grid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, nullptr, 1.0f, 1.0f, nullptr);
     TH_HIP(hipGetLastError());
     return TIRA_OK;
 }
@@ -1292,8 +1323,6 @@ static int table_for(const TableKey& key, int P, hipStream_t st, char** dtab, fl
     return TIRA_OK;
 }
 
-constexpr int kBZ = 4;     // receivers per lane along z: closed, literal-sum and ATV gathers
-constexpr int kBZMlp = 8;  // the tabulated-network gather (its LDS rows are staged per offset column)
 
 template <int P>
 static void launch_closed(bool stick, bool plate, unsigned grid, hipStream_t st, const float4* ps, const float4* pp,
@@ -1328,33 +1357,24 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
         TH_HIP(hipGetLastError());
         return TIRA_OK;
     }
+    const unsigned p = power < 1 ? 1 : power;
     // (a request for the spectral vote above power 1 is served where AUTO takes it)
-    if (plate_mode == TIRA_PLATE_AUTO || (plate_mode == TIRA_VOTE_SPECTRAL && power > 1))
+    if (plate_mode == TIRA_PLATE_AUTO || (plate_mode == TIRA_VOTE_SPECTRAL && p > 1))
         plate_mode = spectral_preferred(s0, s1, s2, w, power, stick, plate, samples) ? TIRA_VOTE_SPECTRAL
                                                                                      : TIRA_PLATE_AUTO;
-    const unsigned p = power < 1 ? 1 : power;
-    // Above power 1 a spectral vote met by a voter that an FFT would spread
-    // beyond its window (not finite, a scale whose sums could overflow, a
-    // caller's stick that is not of unit length) is voted again by window: the
-    // launches below do nothing while *gate is 0.
-    unsigned long long* gate = nullptr;
+    // Above power 1 the spectral vote takes the gather's payloads, so that a voter
+    // that an FFT would spread beyond its window can have the field voted by
+    // window instead: the payload pass raises *gate, and the gather does nothing
+    // while it is 0. All buffers and tables are there before the vote begins, and
+    // the input is not read after it, so that it may share memory with the output.
+    const bool spectral = plate_mode == TIRA_VOTE_SPECTRAL && p > 1;
     if (plate_mode == TIRA_VOTE_SPECTRAL) {
-        const size_t ob = nvox * (out_layout == TIRA_LAYOUT_MAT9 ? 36 : 24),
-                     ib = nvox * (in_layout == TIRA_LAYOUT_MAT9 ? 36 : 24);
-        const bool aliased = tensors && (const char*)out < (const char*)tensors + ib &&
-                             (const char*)tensors < (const char*)out + ob;
-        if (p > 1 && !aliased) {
-            TH_TRY(ws_get(WS_WILD, 8, (void**)&gate));
-            k_fill_zero<<<1, 64, 0, st>>>((float*)gate, 2);
+        if (!spectral) {
+            const int rc = vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0, s1, s2, sigma1,
+                                              sigma2, w, power, stick, plate, samples, false, st, eig);
+            if (rc != kSpectralNotApplicable) return rc;
         }
-        // (in place, the windows could not be voted again)
-        const int rc = p > 1 && aliased ? kSpectralNotApplicable
-                                        : vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0,
-                                                             s1, s2, sigma1, sigma2, w, power, stick, plate, samples,
-                                                             false, st, p > 1 ? nullptr : eig, gate);
-        if (rc != kSpectralNotApplicable && (rc != TIRA_OK || p == 1)) return rc;
-        if (rc == kSpectralNotApplicable) gate = nullptr;
-        plate_mode = TIRA_PLATE_AUTO;  // power, samples or size outside the spectral method: direct gather
+        plate_mode = TIRA_PLATE_AUTO;  // samples or size outside the spectral method: direct gather
     }
     const int mode = plate ? resolve_plate_mode(plate_mode, power, samples) : TIRA_PLATE_CLOSED;
     if (mode == TIRA_PLATE_MLP) {
@@ -1371,11 +1391,18 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     const unsigned nsamp = samples == 0 ? p + 2 : samples;  // samples == 0 (analytic) equals the exact integral
     if (sum) TH_TRY(ws_get(WS_SCRATCH0, ptotal * 16, (void**)&pv));
     const float inv_n = sum ? 1.0f / (float)nsamp : 1.0f;
-    const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), gate ? 4096 : 65536);
+    unsigned long long* gate = nullptr;
+    float alpha = 1.0f;
+    if (spectral) {
+        TH_TRY(ws_get(WS_WILD, 8, (void**)&gate));
+        k_fill_zero<<<1, 64, 0, st>>>((float*)gate, 2);
+        alpha = sticknorm3_host(sigma1, sigma2, p);
+    }
+    const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), 65536);
     {
-        ProfScope prof(gate ? "vote3_prep_gated" : "vote3_prep", st);
-        if (tensors) k_vote3_prep<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, pv, inv_n, gate);
-        else k_vote3_prep_tk<<<pgrid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, pv, inv_n, gate);
+        ProfScope prof("vote3_prep", st);
+        if (tensors) k_vote3_prep<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, pv, inv_n, alpha, gate);
+        else k_vote3_prep_tk<<<pgrid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, pv, inv_n, alpha, gate);
     }
     TH_HIP(hipGetLastError());
 
@@ -1387,6 +1414,13 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     char* dtab = nullptr;
     float2* dcs = nullptr;
     TH_TRY(table_for(key, P, st, &dtab, &dcs));
+    if (spectral) {
+        const SpecPayload pay{ps, pp, g};
+        const int rc = vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0, s1, s2, sigma1, sigma2,
+                                          w, power, stick, plate, samples, false, st, nullptr, &pay);
+        if (rc == kSpectralNotApplicable) gate = nullptr;  // no memory for it: the gather, as it stands
+        else TH_TRY(rc);
+    }
     const unsigned grid = g.nbx * g.nby * g.nbz;
     const float* t = (const float*)dtab;
     ProfScope prof_vote(gate ? "vote3_closed_gated" : sum ? "vote3_sum" : "vote3_closed", st);
@@ -1630,8 +1664,10 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
         // sticks overwrites the spectral ones if any voter is such.
         bool spectral = false;
         if (stick && spectral_preferred(s0, s1, s2, w, m->power, true, false, 0)) {
+            const SpecPayload pay{ps, nullptr, g};
             const int rc = vote3_spectral_run(tensors, in_layout, nullptr, nullptr, nullptr, out, out_layout, s0, s1, s2,
-                                              m->sigma1, m->sigma2, w, m->power, true, false, 0, false, st);
+                                              m->sigma1, m->sigma2, w, m->power, true, false, 0, false, st, nullptr,
+                                              m->power > 1 ? &pay : nullptr);
             if (rc != TIRA_OK && rc != kSpectralNotApplicable) return rc;
             spectral = rc == TIRA_OK;
         }

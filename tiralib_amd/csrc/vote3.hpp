@@ -36,12 +36,19 @@ struct EigOut {
 };
 // Status of vote3_spectral_run when the request is outside the spectral method.
 constexpr int kSpectralNotApplicable = -1;
-// wild (optional, device): raised when a power above 1 met a feature that is not
-// finite or could overflow; such a voter spoils the whole spectral output.
+// Voters of a spectral vote above power 1: the padded payloads of the window
+// gather, formed (and the voters looked over, see k_vote3_prep) before it.
+struct SpecPayload {
+    const float4 *ps, *pp;
+    VoteGeom g;
+};
+// Padded payload voxels of the window gather.
+size_t vote3_payload_voxels(unsigned s0, unsigned s1, unsigned s2, unsigned w);
+// pay: given above power 1 and only there.
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        float* out, int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1,
                        float sigma2, unsigned w, unsigned power, bool stick, bool plate, unsigned samples,
-                       bool atv, hipStream_t st, EigOut* eig = nullptr, unsigned long long* wild = nullptr);
+                       bool atv, hipStream_t st, EigOut* eig = nullptr, const SpecPayload* pay = nullptr);
 int resolve_plate_mode(int plate_mode, unsigned power, unsigned samples);
 int vote3_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0, float* out,
               int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1, float sigma2, unsigned w,
