@@ -199,3 +199,44 @@ def test_input_may_lie_in_the_output(hip, power, wild):
     finally:
         for d in (one, own, two):
             d.free()
+
+
+@pytest.mark.parametrize("power,w", [(2, 9), (3, 9), (4, 11)])
+@pytest.mark.parametrize("bright", [1.0, 1e3, 1e6])
+def test_faint_votes_beside_a_bright_voter(hip, oracle, power, w, bright):
+    """The vote of faint voters keeps its digits where a bright voter stands elsewhere
+    in the field: receivers outside its window, against the window gather (whose
+    rounding knows nothing of it) and, one by one, against FP64. Transforms in FP32
+    lose 1e-10 of the bright voter: 1e-4 of these votes at 1e6."""
+    shape, at = (36, 40, 44), (4, 5, 6)
+    f = _field(shape, seed=8)
+    f[tuple(slice(0, c + w) for c in at)] = 0
+    f[at] = bright * np.diag([1.0, 0.25, 0.0]).astype(np.float32).ravel()
+    got, n = _run(f, shape, _lib.PLATE_AUTO, 1.5, 0.0, w, power)
+    ref, _ = _run(f, shape, _lib.PLATE_CLOSED, 1.5, 0.0, w, power)
+    assert n == 1
+    far = np.ones(shape, bool)
+    far[tuple(slice(0, c + w // 2 + 1) for c in at)] = False
+    assert _rel(got[far], ref[far]) <= 2e-6
+    # receiver by receiver, down to a thousandth of the largest of these votes
+    size = np.linalg.norm(ref, axis=-1)
+    strong = np.flatnonzero(far & (size > 1e-3 * size[far].max()))
+    recv = np.sort(np.random.default_rng(3).choice(strong, 300, replace=False))
+    exact = oracle.tensorvote3_f64(f, 1.5, 0.0, power, w, samples=20, recv=recv, nthreads=8)
+    err = np.linalg.norm(got.reshape(-1, 9)[recv].astype(np.float64) - exact, axis=1) / np.linalg.norm(exact, axis=1)
+    # a voter's FP32 direction enters a vote 2 p + 2 times, 6e-8 each, and votes of opposite
+    # sign cancel to a sixth of their magnitudes at most where they are this large
+    assert err.max() <= (2 * power + 2) * 6e-8 * 6
+
+
+@pytest.mark.parametrize("power", [2, 3, 4])
+def test_spectral_power_is_closer_to_64_bits_than_the_gather(hip, oracle, power):
+    shape, w = (32, 35, 33), 11
+    f = _field(shape, seed=13)
+    rng = np.random.default_rng(2)
+    recv = np.sort(rng.choice(int(np.prod(shape)), 300, replace=False))
+    ref = oracle.tensorvote3_f64(f, 2.0, 1.0, power, w, samples=20, recv=recv, nthreads=8)[:, SLOTS]
+    err = [_rel(_run(f, shape, mode, 2.0, 1.0, w, power)[0].reshape(-1, 9)[recv][:, SLOTS], ref)
+           for mode in (_lib.PLATE_AUTO, _lib.PLATE_CLOSED)]
+    # voters and result in FP32, all between in FP64: a few roundings of 6e-8, averaged over the voters
+    assert err[0] <= min(err[1], 1.2e-7)

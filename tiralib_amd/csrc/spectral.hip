@@ -11,8 +11,8 @@
 // On the unit sphere the even polynomials of degree <= 4 span exactly the 15
 // quartic monomials q_x^a q_y^b q_z^c (a + b + c = 4), so
 //     V_c(x) = sum_f sum_d K_{c,f}(d) F_f(x + d),      c = xx, xy, xz, yy, yz, zz,
-// with offset kernels K_{c,f}(d) of the stick vote fitted once on the host in
-// FP64. The plate vote integrates the stick vote over the great circle
+// with offset kernels K_{c,f}(d) of the stick vote fitted in FP64 (on the device,
+// once per parameter set). The plate vote integrates the stick vote over the great circle
 // perpendicular to n, and averaging a quartic over that circle is a fixed
 // linear map on the 15 monomials (add_circle_average), so the plate kernels
 // are the stick kernels times that map and both votes share them: the voter
@@ -23,7 +23,9 @@
 // Powers 2 to 4 are the same with degree g = 2 p + 2 (eta has degree 2 p):
 // (g + 1)(g + 2) / 2 = 28, 45 or 66 monomials. Their circle averages are
 // evaluated as the mean over p + 2 equispaced directions of the half circle,
-// which is exact for a trigonometric polynomial of degree g.
+// which is exact for a trigonometric polynomial of degree g. The window gather
+// serves every other request of these powers, so theirs runs in FP64 from the
+// gather's payloads (spectral_run64): no vote is further from 64 bits than it was.
 //
 // Pipeline of one call (device buffers, zero padding to L >= n + w/2 per axis
 // so the circular convolution equals the reference's bounded window):
@@ -43,8 +45,7 @@
 //     the inverse x pass fused with the output write (either layout).
 // FFTs are Stockham autosort, mixed radix 2/3/4/5/7/8/9, one block per batch of
 // lines staged in LDS; the twiddle table is FP64-built and rounded once.
-// The kernel spectra depend on (L0, L1, L2, w, sigma1, sigma2, stick, plate)
-// only: built on the device (separable FP64 cosine/sine transforms of the
+// The kernel spectra depend on (L0, L1, L2, w, sigma1, sigma2, power) only: built on the device (separable FP64 cosine/sine transforms of the
 // offset kernels) and cached per host thread and device.
 #include "common.hpp"
 #include "vote3.hpp"
@@ -53,6 +54,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 namespace th {
@@ -66,13 +68,14 @@ constexpr int kFftBL = TH_FFT_BL;  // complex values staged per block (32 KB of 
 // took 54 KB, two blocks per CU, and ran its pass 1.4x slower than B = 8)
 constexpr size_t kColsLds = 40960;
 
+constexpr int kFftBL64 = kFftBL / 2;  // FP64 values of the middle stages of a column batch
+
 constexpr int kMaxL = 1024;    // longest transform
 constexpr int kMaxStages = 16;
 constexpr int kMono = 15;      // quartic monomials
 constexpr unsigned kSpecMaxPower = 4;
 // Monomials of the degree 2 p + 2 of a power-p vote.
 __host__ __device__ constexpr int mono_count(int power) { return (2 * power + 3) * (power + 2); }
-constexpr int kMaxMono = mono_count((int)kSpecMaxPower);
 
 // Exponents (a, b, c) of monomial m of degree g: a = g..0, b = g-a..0, c = g-a-b.
 __host__ __device__ constexpr int mono_k(int m) {  // g - a: the k with k (k + 1) / 2 <= m < (k + 1)(k + 2) / 2
@@ -176,56 +179,69 @@ static unsigned spectral_length(unsigned n, unsigned w) {
 }
 
 // ---------------------------------------------------------------- device FFT
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-    return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
+// A complex value V is a float2 or a double2.
+template <class V> using real_of = std::conditional_t<std::is_same_v<V, double2>, double, float>;
+template <class V>
+__device__ __forceinline__ V mkc(real_of<V> x, real_of<V> y) {
+    V v;
+    v.x = x;
+    v.y = y;
+    return v;
 }
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ float fmad(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fmad(double a, double b, double c) { return fma(a, b, c); }
+template <class V>
+__device__ __forceinline__ V cmul(V a, V b) {
+    return mkc<V>(fmad(a.x, b.x, -a.y * b.y), fmad(a.x, b.y, a.y * b.x));
+}
+template <class V>
+__device__ __forceinline__ V cadd(V a, V b) {
+    return mkc<V>(a.x + b.x, a.y + b.y);
+}
+template <class V>
+__device__ __forceinline__ V csub(V a, V b) {
+    return mkc<V>(a.x - b.x, a.y - b.y);
+}
 
-// cos / sin of 2 pi n / R for the generic small DFTs.
-template <int R> __device__ __forceinline__ float dcos(int n);
-template <int R> __device__ __forceinline__ float dsin(int n);
-template <> __device__ __forceinline__ float dcos<5>(int n) {
-    constexpr float t[5] = {1.0f, 0.309016994374947424f, -0.809016994374947424f, -0.809016994374947424f,
-                            0.309016994374947424f};
-    return t[n];
+// cos / sin of 2 pi n / R for the generic small DFTs (R = 5, 7).
+template <int R, class T>
+__device__ __forceinline__ T dcos(int n) {
+    constexpr T t5[5] = {T(1), T(0.309016994374947424), T(-0.809016994374947424), T(-0.809016994374947424),
+                         T(0.309016994374947424)};
+    constexpr T t7[7] = {T(1), T(0.623489801858733531), T(-0.222520933956314404), T(-0.900968867902419126),
+                         T(-0.900968867902419126), T(-0.222520933956314404), T(0.623489801858733531)};
+    return R == 5 ? t5[n % 5] : t7[n];
 }
-template <> __device__ __forceinline__ float dsin<5>(int n) {
-    constexpr float t[5] = {0.0f, 0.951056516295153572f, 0.587785252292473129f, -0.587785252292473129f,
-                            -0.951056516295153572f};
-    return t[n];
-}
-template <> __device__ __forceinline__ float dcos<7>(int n) {
-    constexpr float t[7] = {1.0f, 0.623489801858733531f, -0.222520933956314404f, -0.900968867902419126f,
-                            -0.900968867902419126f, -0.222520933956314404f, 0.623489801858733531f};
-    return t[n];
-}
-template <> __device__ __forceinline__ float dsin<7>(int n) {
-    constexpr float t[7] = {0.0f, 0.781831482468029809f, 0.974927912181823607f, 0.433883739117558120f,
-                            -0.433883739117558120f, -0.974927912181823607f, -0.781831482468029809f};
-    return t[n];
+template <int R, class T>
+__device__ __forceinline__ T dsin(int n) {
+    constexpr T t5[5] = {T(0), T(0.951056516295153572), T(0.587785252292473129), T(-0.587785252292473129),
+                         T(-0.951056516295153572)};
+    constexpr T t7[7] = {T(0), T(0.781831482468029809), T(0.974927912181823607), T(0.433883739117558120),
+                         T(-0.433883739117558120), T(-0.974927912181823607), T(-0.781831482468029809)};
+    return R == 5 ? t5[n % 5] : t7[n];
 }
 // In-register DFT of length R: y_k = sum_j u_j W^(jk), W = e^(-+2 pi i / R).
-template <int R, bool INV>
-__device__ __forceinline__ void dft_small(float2 (&u)[R]) {
+template <int R, bool INV, class V>
+__device__ __forceinline__ void dft_small(V (&u)[R]) {
+    using T = real_of<V>;
     if constexpr (R == 2) {
-        const float2 a = u[0], b = u[1];
+        const V a = u[0], b = u[1];
         u[0] = cadd(a, b);
         u[1] = csub(a, b);
     } else if constexpr (R == 3) {
-        constexpr float kS = 0.866025403784438647f;  // sin(2 pi / 3)
-        const float2 s = cadd(u[1], u[2]), d = csub(u[1], u[2]);
-        const float2 t = make_float2(fmaf(-0.5f, s.x, u[0].x), fmaf(-0.5f, s.y, u[0].y));
-        const float sg = INV ? kS : -kS;  // i * sg * d
+        constexpr T kS = T(0.866025403784438647);  // sin(2 pi / 3)
+        const V s = cadd(u[1], u[2]), d = csub(u[1], u[2]);
+        const V t = mkc<V>(fmad(T(-0.5), s.x, u[0].x), fmad(T(-0.5), s.y, u[0].y));
+        const T sg = INV ? kS : -kS;  // i * sg * d
         u[0] = cadd(u[0], s);
-        u[1] = make_float2(t.x - sg * d.y, t.y + sg * d.x);
-        u[2] = make_float2(t.x + sg * d.y, t.y - sg * d.x);
+        u[1] = mkc<V>(t.x - sg * d.y, t.y + sg * d.x);
+        u[2] = mkc<V>(t.x + sg * d.y, t.y - sg * d.x);
     } else if constexpr (R == 4) {
-        const float2 a = cadd(u[0], u[2]), b = csub(u[0], u[2]);
-        const float2 c = cadd(u[1], u[3]), d = csub(u[1], u[3]);
+        const V a = cadd(u[0], u[2]), b = csub(u[0], u[2]);
+        const V c = cadd(u[1], u[3]), d = csub(u[1], u[3]);
         // forward: y1 = b - i d, y3 = b + i d
-        const float2 mid = INV ? make_float2(b.x - d.y, b.y + d.x) : make_float2(b.x + d.y, b.y - d.x);
-        const float2 oth = INV ? make_float2(b.x + d.y, b.y - d.x) : make_float2(b.x - d.y, b.y + d.x);
+        const V mid = INV ? mkc<V>(b.x - d.y, b.y + d.x) : mkc<V>(b.x + d.y, b.y - d.x);
+        const V oth = INV ? mkc<V>(b.x + d.y, b.y - d.x) : mkc<V>(b.x - d.y, b.y + d.x);
         u[0] = cadd(a, c);
         u[2] = csub(a, c);
         u[1] = mid;
@@ -233,26 +249,26 @@ __device__ __forceinline__ void dft_small(float2 (&u)[R]) {
     } else if constexpr (R == 9) {
         // 3 x 3 Cooley-Tukey: j = 3a + b, k = c + 3d, W9^(jk) = W3^(ac) W9^(bc) W3^(bd):
         // length-3 DFTs over a, twiddles W9^(bc), length-3 DFTs over b
-        constexpr float c1 = 0.766044443118978035f, s1 = 0.642787609686539326f;   // 2 pi / 9
-        constexpr float c2 = 0.173648177666930349f, s2 = 0.984807753012208059f;   // 4 pi / 9
-        constexpr float c4 = -0.939692620785908384f, s4 = 0.342020143325668733f;  // 8 pi / 9
-        const float sg = INV ? 1.0f : -1.0f;
-        float2 v[3][3];
+        constexpr T c1 = T(0.766044443118978035), s1 = T(0.642787609686539326);   // 2 pi / 9
+        constexpr T c2 = T(0.173648177666930349), s2 = T(0.984807753012208059);   // 4 pi / 9
+        constexpr T c4 = T(-0.939692620785908384), s4 = T(0.342020143325668733);  // 8 pi / 9
+        const T sg = INV ? T(1.0) : T(-1.0);
+        V v[3][3];
 #pragma unroll
         for (int b = 0; b < 3; b++) {
-            float2 t[3] = {u[b], u[3 + b], u[6 + b]};
+            V t[3] = {u[b], u[3 + b], u[6 + b]};
             dft_small<3, INV>(t);
             v[b][0] = t[0];
             v[b][1] = t[1];
             v[b][2] = t[2];
         }
-        v[1][1] = cmul(v[1][1], make_float2(c1, sg * s1));
-        v[1][2] = cmul(v[1][2], make_float2(c2, sg * s2));
-        v[2][1] = cmul(v[2][1], make_float2(c2, sg * s2));
-        v[2][2] = cmul(v[2][2], make_float2(c4, sg * s4));
+        v[1][1] = cmul(v[1][1], mkc<V>(c1, sg * s1));
+        v[1][2] = cmul(v[1][2], mkc<V>(c2, sg * s2));
+        v[2][1] = cmul(v[2][1], mkc<V>(c2, sg * s2));
+        v[2][2] = cmul(v[2][2], mkc<V>(c4, sg * s4));
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            float2 t[3] = {v[0][c], v[1][c], v[2][c]};
+            V t[3] = {v[0][c], v[1][c], v[2][c]};
             dft_small<3, INV>(t);
             u[c] = t[0];
             u[c + 3] = t[1];
@@ -261,36 +277,36 @@ __device__ __forceinline__ void dft_small(float2 (&u)[R]) {
     } else if constexpr (R == 27) {
         // 3 x 9 Cooley-Tukey: j = 9a + b, k = c + 3d, W27^(jk) = W3^(ac) W27^(bc) W9^(bd):
         // length-3 DFTs over a, twiddles W27^(bc), length-9 DFTs over b
-        constexpr float tc[17] = {1.0f, 0.973044870579823806f, 0.893632640323412275f, 0.766044443118978013f,
-                                  0.597158591702786179f, 0.396079766039156900f, 0.173648177666930414f,
-                                  -0.058144828910475774f, -0.286803232711090206f, -0.5f,
-                                  -0.686241637868733489f, -0.835487811412936265f, -0.939692620785908317f,
-                                  -0.993238357741943023f, -0.993238357741943023f, -0.939692620785908539f,
-                                  -0.835487811412936487f};
-        constexpr float ts[17] = {0.0f, 0.230615870742440165f, 0.448799180200462167f, 0.642787609686539252f,
-                                  0.802123192755043735f, 0.918216106880273997f, 0.984807753012208020f,
-                                  0.998308158271268176f, 0.957989512315488900f, 0.866025403784438708f,
-                                  0.727373641573048846f, 0.549508978070806231f, 0.342020143325668879f,
-                                  0.116092914125229929f, -0.116092914125230123f, -0.342020143325668213f,
-                                  -0.549508978070806009f};
-        const float sg = INV ? 1.0f : -1.0f;
+        constexpr T tc[17] = {T(1.0), T(0.973044870579823806), T(0.893632640323412275), T(0.766044443118978013),
+                                  T(0.597158591702786179), T(0.396079766039156900), T(0.173648177666930414),
+                                  T(-0.058144828910475774), T(-0.286803232711090206), T(-0.5),
+                                  T(-0.686241637868733489), T(-0.835487811412936265), T(-0.939692620785908317),
+                                  T(-0.993238357741943023), T(-0.993238357741943023), T(-0.939692620785908539),
+                                  T(-0.835487811412936487)};
+        constexpr T ts[17] = {T(0.0), T(0.230615870742440165), T(0.448799180200462167), T(0.642787609686539252),
+                                  T(0.802123192755043735), T(0.918216106880273997), T(0.984807753012208020),
+                                  T(0.998308158271268176), T(0.957989512315488900), T(0.866025403784438708),
+                                  T(0.727373641573048846), T(0.549508978070806231), T(0.342020143325668879),
+                                  T(0.116092914125229929), T(-0.116092914125230123), T(-0.342020143325668213),
+                                  T(-0.549508978070806009)};
+        const T sg = INV ? T(1.0) : T(-1.0);
 #pragma unroll
         for (int b = 0; b < 9; b++) {
-            float2 t[3] = {u[b], u[9 + b], u[18 + b]};
+            V t[3] = {u[b], u[9 + b], u[18 + b]};
             dft_small<3, INV>(t);
             u[b] = t[0];
             if (b == 0) {
                 u[9] = t[1];
                 u[18] = t[2];
             } else {
-                u[9 + b] = cmul(t[1], make_float2(tc[b], sg * ts[b]));
-                u[18 + b] = cmul(t[2], make_float2(tc[2 * b], sg * ts[2 * b]));
+                u[9 + b] = cmul(t[1], mkc<V>(tc[b], sg * ts[b]));
+                u[18 + b] = cmul(t[2], mkc<V>(tc[2 * b], sg * ts[2 * b]));
             }
         }
-        float2 y[27];
+        V y[27];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            float2 t[9];
+            V t[9];
 #pragma unroll
             for (int b = 0; b < 9; b++) t[b] = u[9 * c + b];
             dft_small<9, INV>(t);
@@ -302,7 +318,7 @@ __device__ __forceinline__ void dft_small(float2 (&u)[R]) {
     } else if constexpr (R == 15) {
         // Good-Thomas (3 and 5 coprime, no twiddles): input n = (5 n1 + 3 n2) mod 15,
         // output k = (10 k1 + 6 k2) mod 15, so W15^(nk) = W3^(n1 k1) W5^(n2 k2)
-        float2 v[3][5];
+        V v[3][5];
 #pragma unroll
         for (int a = 0; a < 3; a++) {
 #pragma unroll
@@ -311,21 +327,21 @@ __device__ __forceinline__ void dft_small(float2 (&u)[R]) {
         }
 #pragma unroll
         for (int b = 0; b < 5; b++) {
-            float2 t[3] = {v[0][b], v[1][b], v[2][b]};
+            V t[3] = {v[0][b], v[1][b], v[2][b]};
             dft_small<3, INV>(t);
 #pragma unroll
             for (int a = 0; a < 3; a++) u[(10 * a + 6 * b) % 15] = t[a];
         }
     } else if constexpr (R == 8) {
         // two length-4 DFTs (even and odd inputs), the odd ones turned by W8^k
-        float2 e[4] = {u[0], u[2], u[4], u[6]}, o[4] = {u[1], u[3], u[5], u[7]};
+        V e[4] = {u[0], u[2], u[4], u[6]}, o[4] = {u[1], u[3], u[5], u[7]};
         dft_small<4, INV>(e);
         dft_small<4, INV>(o);
-        constexpr float r = 0.707106781186547524f;
-        const float sg = INV ? 1.0f : -1.0f;  // W8 = r (1 + sg i)
-        const float2 w1 = make_float2(r * (o[1].x - sg * o[1].y), r * (o[1].y + sg * o[1].x));
-        const float2 w2 = make_float2(-sg * o[2].y, sg * o[2].x);
-        const float2 w3 = make_float2(r * (-o[3].x - sg * o[3].y), r * (-o[3].y + sg * o[3].x));
+        constexpr T r = T(0.707106781186547524);
+        const T sg = INV ? T(1.0) : T(-1.0);  // W8 = r (1 + sg i)
+        const V w1 = mkc<V>(r * (o[1].x - sg * o[1].y), r * (o[1].y + sg * o[1].x));
+        const V w2 = mkc<V>(-sg * o[2].y, sg * o[2].x);
+        const V w3 = mkc<V>(r * (-o[3].x - sg * o[3].y), r * (-o[3].y + sg * o[3].x));
         u[0] = cadd(e[0], o[0]);
         u[4] = csub(e[0], o[0]);
         u[1] = cadd(e[1], w1);
@@ -340,30 +356,30 @@ __device__ __forceinline__ void dft_small(float2 (&u)[R]) {
         // a_k = u_0 + sum_m cos(2 pi m k / R) s_m and b_k = sum_m sin(2 pi m k / R) d_m
         static_assert(R % 2 == 1, "symmetric-pair DFT needs an odd length");
         constexpr int H = (R - 1) / 2;
-        float2 s[H], d[H];
-        float2 y0 = u[0];
+        V s[H], d[H];
+        V y0 = u[0];
 #pragma unroll
         for (int m = 1; m <= H; m++) {
             s[m - 1] = cadd(u[m], u[R - m]);
             d[m - 1] = csub(u[m], u[R - m]);
             y0 = cadd(y0, s[m - 1]);
         }
-        float2 y[R];
+        V y[R];
         y[0] = y0;
 #pragma unroll
         for (int k = 1; k <= H; k++) {
-            float2 a = u[0], b = make_float2(0.0f, 0.0f);
+            V a = u[0], b = mkc<V>(T(0.0), T(0.0));
 #pragma unroll
             for (int m = 1; m <= H; m++) {
                 const int n = (m * k) % R;
-                const float c = dcos<R>(n), sn = dsin<R>(n);
-                a.x = fmaf(c, s[m - 1].x, a.x);
-                a.y = fmaf(c, s[m - 1].y, a.y);
-                b.x = fmaf(sn, d[m - 1].x, b.x);
-                b.y = fmaf(sn, d[m - 1].y, b.y);
+                const T c = dcos<R, T>(n), sn = dsin<R, T>(n);
+                a.x = fmad(c, s[m - 1].x, a.x);
+                a.y = fmad(c, s[m - 1].y, a.y);
+                b.x = fmad(sn, d[m - 1].x, b.x);
+                b.y = fmad(sn, d[m - 1].y, b.y);
             }
-            const float2 amib = make_float2(a.x + b.y, a.y - b.x);  // a - i b
-            const float2 apib = make_float2(a.x - b.y, a.y + b.x);  // a + i b
+            const V amib = mkc<V>(a.x + b.y, a.y - b.x);  // a - i b
+            const V apib = mkc<V>(a.x - b.y, a.y + b.x);  // a + i b
             y[k] = INV ? apib : amib;
             y[R - k] = INV ? amib : apib;
         }
@@ -375,13 +391,22 @@ __device__ __forceinline__ void dft_small(float2 (&u)[R]) {
 // LDS pointers keep their address space across the (non-inlined) stage calls,
 // so the stages use ds_read / ds_write.
 typedef float __attribute__((ext_vector_type(2))) f2v;
+typedef double __attribute__((ext_vector_type(2))) d2v;
 typedef __attribute__((address_space(3))) f2v lds_f2;
+typedef __attribute__((address_space(3))) d2v lds_d2;
+template <class V> using lds_v = std::conditional_t<std::is_same_v<V, double2>, lds_d2, lds_f2>;
 __device__ __forceinline__ lds_f2* to_lds(float2* p) { return (lds_f2*)p; }
+__device__ __forceinline__ lds_d2* to_lds(double2* p) { return (lds_d2*)p; }
 __device__ __forceinline__ float2 ld2(const lds_f2* p) {
     const f2v v = *p;
     return make_float2(v.x, v.y);
 }
+__device__ __forceinline__ double2 ld2(const lds_d2* p) {
+    const d2v v = *p;
+    return make_double2(v.x, v.y);
+}
 __device__ __forceinline__ void st2(lds_f2* p, float2 a) { *p = f2v{a.x, a.y}; }
+__device__ __forceinline__ void st2(lds_d2* p, double2 a) { *p = d2v{a.x, a.y}; }
 
 // n / d for 0 <= n < 2^22 and d >= 1, with rd = 1 / d in FP32: the float
 // quotient is within one of the exact one, which the remainder corrects.
@@ -408,31 +433,31 @@ __device__ __forceinline__ int fdiv(int n, int d, float rd) {
 // TW = false compiles no twiddles at all, for a stage that only ever runs
 // first (p = 1). TAG gives one kernel stage functions of its own, so that its
 // launch bound reaches them (a bound does not constrain a shared callee).
-template <int R, bool INV, int BL = kFftBL, bool FIXED = true, bool TW = true, int TAG = 0>
-__device__ __noinline__ void fft_stage(lds_f2* __restrict__ s, int L, int nlines, int p,
-                                       const lds_f2* __restrict__ tw) {
+template <int R, bool INV, class V, int BL = kFftBL, bool FIXED = true, bool TW = true, int TAG = 0>
+__device__ __noinline__ void fft_stage(lds_v<V>* __restrict__ s, int L, int nlines, int p,
+                                       const lds_v<V>* __restrict__ tw) {
     constexpr int MAXQ = (BL / R + kFT - 1) / kFT;
     const int m = L / R;
     const int nb = nlines * m;
     const int step = L / (p * R);
     const float rm = 1.0f / (float)m, rp = 1.0f / (float)p;
-    float2 u[MAXQ][R];
+    V u[MAXQ][R];
     const int G = kFT / m;
     if (FIXED && G > 0 && (nlines + G - 1) / G <= (nb + kFT - 1) / kFT) {
         const int l0 = fdiv((int)threadIdx.x, m, rm), i = (int)threadIdx.x - l0 * m;
         const bool act = l0 < G;  // threadIdx.x < G m
         const int k = i - fdiv(i, p, rp) * p;
-        float2 w[R];
+        V w[R];
 #pragma unroll
         for (int r = 1; r < R; r++) {
-            w[r] = (TW && act) ? ld2(tw + r * k * step) : make_float2(1.0f, 0.0f);  // r k step < L
+            w[r] = (TW && act) ? ld2(tw + r * k * step) : mkc<V>(1.0f, 0.0f);  // r k step < L
             if (INV) w[r].y = -w[r].y;
         }
 #pragma unroll
         for (int q = 0; q < MAXQ; q++) {  // rounds: ceil(nlines / G) <= MAXQ
             const int line = l0 + q * G;
             if (act && line < nlines) {
-                const lds_f2* src = s + line * L + i;
+                const lds_v<V>* src = s + line * L + i;
 #pragma unroll
                 for (int r = 0; r < R; r++) u[q][r] = ld2(src + r * m);
             }
@@ -447,7 +472,7 @@ __device__ __noinline__ void fft_stage(lds_f2* __restrict__ s, int L, int nlines
                     for (int r = 1; r < R; r++) u[q][r] = cmul(u[q][r], w[r]);
                 }
                 dft_small<R, INV>(u[q]);
-                lds_f2* dst = s + line * L + (i - k) * R + k;
+                lds_v<V>* dst = s + line * L + (i - k) * R + k;
 #pragma unroll
                 for (int r = 0; r < R; r++) st2(dst + r * p, u[q][r]);
             }
@@ -460,7 +485,7 @@ __device__ __noinline__ void fft_stage(lds_f2* __restrict__ s, int L, int nlines
         const int t = (int)threadIdx.x + q * kFT;
         if (t < nb) {
             const int line = fdiv(t, m, rm), i = t - line * m;
-            const lds_f2* src = s + line * L + i;
+            const lds_v<V>* src = s + line * L + i;
 #pragma unroll
             for (int r = 0; r < R; r++) u[q][r] = ld2(src + r * m);
         }
@@ -475,13 +500,13 @@ __device__ __noinline__ void fft_stage(lds_f2* __restrict__ s, int L, int nlines
             if (TW && p > 1) {  // p = 1: every twiddle is W^0
 #pragma unroll
                 for (int r = 1; r < R; r++) {
-                    float2 w = ld2(tw + r * k * step);  // r k step < L
+                    V w = ld2(tw + r * k * step);  // r k step < L
                     if (INV) w.y = -w.y;
                     u[q][r] = cmul(u[q][r], w);
                 }
             }
             dft_small<R, INV>(u[q]);
-            lds_f2* dst = s + line * L + (i - k) * R + k;
+            lds_v<V>* dst = s + line * L + (i - k) * R + k;
 #pragma unroll
             for (int r = 0; r < R; r++) st2(dst + r * p, u[q][r]);
         }
@@ -490,31 +515,32 @@ __device__ __noinline__ void fft_stage(lds_f2* __restrict__ s, int L, int nlines
 }
 
 // Transform `nlines` lines staged in LDS (nlines * L <= kFftBL).
-template <bool INV>
-__device__ __forceinline__ void fft_lines(float2* __restrict__ s_, const FftPlan& pl, int nlines,
-                                          const float2* __restrict__ tw_) {
-    lds_f2* s = to_lds(s_);
-    const lds_f2* tw = to_lds(const_cast<float2*>(tw_));
+template <bool INV, class V>
+__device__ __forceinline__ void fft_lines(V* __restrict__ s_, const FftPlan& pl, int nlines,
+                                          const V* __restrict__ tw_) {
+    lds_v<V>* s = to_lds(s_);
+    const lds_v<V>* tw = to_lds(const_cast<V*>(tw_));
     int p = 1;
     for (int st = 0; st < pl.nst; st++) {
         const int R = pl.rad[st];
         switch (R) {
-            case 2: fft_stage<2, INV>(s, pl.L, nlines, p, tw); break;
-            case 3: fft_stage<3, INV>(s, pl.L, nlines, p, tw); break;
-            case 4: fft_stage<4, INV>(s, pl.L, nlines, p, tw); break;
-            case 5: fft_stage<5, INV>(s, pl.L, nlines, p, tw); break;
-            case 7: fft_stage<7, INV>(s, pl.L, nlines, p, tw); break;
-            case 9: fft_stage<9, INV>(s, pl.L, nlines, p, tw); break;
+            case 2: fft_stage<2, INV, V>(s, pl.L, nlines, p, tw); break;
+            case 3: fft_stage<3, INV, V>(s, pl.L, nlines, p, tw); break;
+            case 4: fft_stage<4, INV, V>(s, pl.L, nlines, p, tw); break;
+            case 5: fft_stage<5, INV, V>(s, pl.L, nlines, p, tw); break;
+            case 7: fft_stage<7, INV, V>(s, pl.L, nlines, p, tw); break;
+            case 9: fft_stage<9, INV, V>(s, pl.L, nlines, p, tw); break;
             // one round per thread at 4096 staged values; make_lines_plan puts it
             // first (p = 1), so it has no twiddles, and none hold registers
-            case 27: fft_stage<27, INV, kFftBL, false, false>(s, pl.L, nlines, p, tw); break;
-            default: fft_stage<8, INV>(s, pl.L, nlines, p, tw); break;
+            case 27: fft_stage<27, INV, V, kFftBL, false, false>(s, pl.L, nlines, p, tw); break;
+            default: fft_stage<8, INV, V>(s, pl.L, nlines, p, tw); break;
         }
         p *= R;
     }
 }
 
-__device__ __forceinline__ void load_twiddles(float2* __restrict__ tw, const float2* __restrict__ g, int L) {
+template <class V>
+__device__ __forceinline__ void load_twiddles(V* __restrict__ tw, const V* __restrict__ g, int L) {
     for (int i = (int)threadIdx.x; i < L; i += kFT) tw[i] = g[i];
 }
 
@@ -576,15 +602,15 @@ __global__ __launch_bounds__(kFT) void k_fft_lines(float2* __restrict__ data, Li
 // (p = 1: no twiddles), the last one writes its outputs straight back
 // (p = L / R: output r of butterfly i is element i + r L/R), so the lines
 // touch LDS only between stages.
-template <int R, bool INV, int BL>
-__device__ __forceinline__ void cols_first(const float2* __restrict__ base, lds_f2* __restrict__ s, int L, int B,
+template <int R, bool INV, int BL, class V>
+__device__ __forceinline__ void cols_first(const V* __restrict__ base, lds_v<V>* __restrict__ s, int L, int B,
                                            int lb, int Bv, size_t estride, int n_in) {
     // every load of a round of MAXQ butterflies per thread is issued before
     // its first butterfly; batches above BL values (B L > BL) take more rounds
     constexpr int MAXQ = (BL / R + kFT - 1) / kFT;
     const int m = L / R;
     const int nb = B * m;
-    float2 u[MAXQ][R];
+    V u[MAXQ][R];
     for (int t0 = 0; t0 < nb; t0 += MAXQ * kFT) {
 #pragma unroll
         for (int q = 0; q < MAXQ; q++) {
@@ -593,7 +619,7 @@ __device__ __forceinline__ void cols_first(const float2* __restrict__ base, lds_
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const int e = i + r * m;
-                u[q][r] = (t < nb && l < Bv && e < n_in) ? base[(size_t)e * estride + l] : make_float2(0.0f, 0.0f);
+                u[q][r] = (t < nb && l < Bv && e < n_in) ? base[(size_t)e * estride + l] : mkc<V>(0.0f, 0.0f);
             }
         }
 #pragma unroll
@@ -602,7 +628,7 @@ __device__ __forceinline__ void cols_first(const float2* __restrict__ base, lds_
             if (t < nb) {
                 const int l = t & (B - 1), i = t >> lb;
                 dft_small<R, INV>(u[q]);
-                lds_f2* d = s + l * L + i * R;
+                lds_v<V>* d = s + l * L + i * R;
 #pragma unroll
                 for (int r = 0; r < R; r++) st2(d + r, u[q][r]);
             }
@@ -610,20 +636,20 @@ __device__ __forceinline__ void cols_first(const float2* __restrict__ base, lds_
     }
 }
 
-template <int R, bool INV>
-__device__ __forceinline__ void cols_last(const lds_f2* __restrict__ s, float2* __restrict__ base,
-                                          const lds_f2* __restrict__ tw, int L, int B, int lb, int Bv,
+template <int R, bool INV, class V>
+__device__ __forceinline__ void cols_last(const lds_v<V>* __restrict__ s, V* __restrict__ base,
+                                          const lds_v<V>* __restrict__ tw, int L, int B, int lb, int Bv,
                                           size_t estride, int n_out) {
     const int m = L / R;
     for (int t = (int)threadIdx.x; t < B * m; t += kFT) {
         const int l = t & (B - 1), i = t >> lb;
-        float2 u[R];
-        const lds_f2* src = s + l * L + i;
+        V u[R];
+        const lds_v<V>* src = s + l * L + i;
 #pragma unroll
         for (int r = 0; r < R; r++) u[r] = ld2(src + r * m);
 #pragma unroll
         for (int r = 1; r < R; r++) {
-            float2 w = ld2(tw + r * i);  // W_L^(r i), r i < L
+            V w = ld2(tw + r * i);  // W_L^(r i), r i < L
             if (INV) w.y = -w.y;
             u[r] = cmul(u[r], w);
         }
@@ -639,14 +665,14 @@ __device__ __forceinline__ void cols_last(const lds_f2* __restrict__ s, float2* 
 }
 
 // Whole transform of a length-R line (R <= 9) in registers.
-template <int R, bool INV>
-__device__ __forceinline__ void cols_single(float2* __restrict__ base, int B, int Bv, size_t estride, int n_in,
+template <int R, bool INV, class V>
+__device__ __forceinline__ void cols_single(V* __restrict__ base, int B, int Bv, size_t estride, int n_in,
                                             int n_out) {
     for (int l = (int)threadIdx.x; l < B; l += kFT) {
-        float2 u[R];
+        V u[R];
 #pragma unroll
         for (int r = 0; r < R; r++)
-            u[r] = (l < Bv && r < n_in) ? base[(size_t)r * estride + l] : make_float2(0.0f, 0.0f);
+            u[r] = (l < Bv && r < n_in) ? base[(size_t)r * estride + l] : mkc<V>(0.0f, 0.0f);
         dft_small<R, INV>(u);
         if (l < Bv) {
 #pragma unroll
@@ -679,16 +705,20 @@ __device__ __forceinline__ void cols_single(float2* __restrict__ base, int B, in
 // waves), 1% faster at L = 135; eight waves spill and run 25% slower. Smaller
 // groups (L > 256) take no bound: there the bounded code ran 8% slower and
 // fetched 1.3x the algorithmic bytes.
-template <bool INV, int BL, int MINW>
-__global__ __launch_bounds__(kFT, MINW) void k_fft_cols(float2* __restrict__ data, LineGeom g, FftPlan pl,
-                                                  const float2* __restrict__ twg) {
+// stop (FP64 only, optional): nothing is done where *stop is set.
+template <bool INV, int BL, int MINW, class V>
+__global__ __launch_bounds__(kFT, MINW) void k_fft_cols(V* __restrict__ data, LineGeom g, FftPlan pl,
+                                                        const V* __restrict__ twg,
+                                                        const unsigned long long* __restrict__ stop) {
+    if constexpr (std::is_same_v<V, double2>)
+        if (stop && *stop) return;
     // B L staged values, then L twiddles: sized at launch (at most kColsLds
     // bytes), 18 KB at L = 135 where a static BL-value array took 40 KB and
     // held the pass to four blocks per CU
-    extern __shared__ float2 cols_dyn[];
+    extern __shared__ __align__(16) unsigned char fft_dyn[];
     const int L = pl.L;
-    float2* s_ = cols_dyn;
-    float2* tw_ = cols_dyn + g.B * L;
+    V* s_ = reinterpret_cast<V*>(fft_dyn);
+    V* tw_ = s_ + g.B * L;
     // XCD-major order: neighbouring column batches (which share 128-byte
     // lines when B < 16) run on one XCD and meet in its L2
     unsigned bid = xcd_remap(blockIdx.x, gridDim.x);
@@ -700,15 +730,15 @@ __global__ __launch_bounds__(kFT, MINW) void k_fft_cols(float2* __restrict__ dat
     const int B = g.B, lb = g.lb;
     const int a0 = ab * B;
     const int Bv = min(B, g.na - a0);
-    float2* base = data + (size_t)c * g.cstride + (size_t)b * g.bstride + (size_t)a0;
+    V* base = data + (size_t)c * g.cstride + (size_t)b * g.bstride + (size_t)a0;
     if (pl.nst == 0) return;  // length 1: the identity
     if (pl.nst == 1) {
         TH_RADIX_SWITCH_LAST(pl.rad[0], (cols_single<RR, INV>(base, B, Bv, g.estride, g.n_in, g.n_out)));
         return;
     }
     load_twiddles(tw_, twg, L);
-    lds_f2* s = to_lds(s_);
-    const lds_f2* tw = to_lds(tw_);
+    lds_v<V>* s = to_lds(s_);
+    const lds_v<V>* tw = to_lds(tw_);
     TH_RADIX_SWITCH(pl.rad[0], (cols_first<RR, INV, BL>(base, s, L, B, lb, Bv, g.estride, g.n_in)));
     __syncthreads();
     // the middle stages take the batch in groups of Bh lines (Bh L <= BL, the
@@ -718,7 +748,7 @@ __global__ __launch_bounds__(kFT, MINW) void k_fft_cols(float2* __restrict__ dat
         int p = pl.rad[0];
         for (int st = 1; st < pl.nst - 1; st++) {
             const int R = pl.rad[st];
-            TH_RADIX_SWITCH(R, (fft_stage<RR, INV, BL, false, true, MINW>(s + h0 * L, L, g.Bh, p, tw)));
+            TH_RADIX_SWITCH(R, (fft_stage<RR, INV, V, BL, false, true, MINW>(s + h0 * L, L, g.Bh, p, tw)));
             p *= R;
         }
     }
@@ -788,11 +818,11 @@ __device__ __forceinline__ void add_circle_average(const float4 N, float* __rest
 
 // The monomials of degree 2 P + 2 of (x, y, z) times w, added to A.
 template <int P>
-__device__ __forceinline__ void add_mono(float x, float y, float z, float w, float* __restrict__ A) {
+__device__ __forceinline__ void add_mono(double x, double y, double z, double w, double* __restrict__ A) {
     constexpr int G = 2 * P + 2;
-    float px[G + 1], py[G + 1], pz[G + 1];
+    double px[G + 1], py[G + 1], pz[G + 1];
     px[0] = w;
-    py[0] = pz[0] = 1.0f;
+    py[0] = pz[0] = 1.0;
 #pragma unroll
     for (int i = 1; i <= G; i++) {
         px[i] = px[i - 1] * x;
@@ -803,41 +833,48 @@ __device__ __forceinline__ void add_mono(float x, float y, float z, float w, flo
 #pragma unroll
     for (int k = 0; k <= G; k++)
 #pragma unroll
-        for (int c = 0; c <= k; c++, m++) A[m] = fmaf(px[G - k], py[k - c] * pz[c], A[m]);
+        for (int c = 0; c <= k; c++, m++) A[m] = fma(px[G - k], py[k - c] * pz[c], A[m]);
 }
 
-// Features of a power-P voter: the stick's monomials, and the plate's as the
-// mean of the stick's over the half circle perpendicular to n (P + 2
-// equispaced directions; N.w carries the plate's scale and sticknorm3).
+// Features of a power-P voter in FP64: the stick's monomials, and the plate's as
+// the mean of the stick's over the half circle perpendicular to n (P + 2
+// equispaced directions), times alpha (sticknorm3). The monomials take unit
+// vectors: the payload's, rounded to FP32 or a caller's, are brought to length 1,
+// and the square of a stick's length stays a factor, as the window gather has it.
 template <int P>
-__device__ __forceinline__ void voter_features(const float4 S, const float4 N, bool stick, bool plate,
-                                               float* __restrict__ A) {
+__device__ __forceinline__ void voter_features(const float4 S, const float4 N, double alpha, bool stick, bool plate,
+                                               double* __restrict__ A) {
 #pragma unroll
-    for (int m = 0; m < mono_count(P); m++) A[m] = 0.0f;
-    if (stick) add_mono<P>(S.x, S.y, S.z, S.w, A);
-    if (plate) {
+    for (int m = 0; m < mono_count(P); m++) A[m] = 0.0;
+    if (stick && S.w != 0.0f) {
+        const double x = S.x, y = S.y, z = S.z, q2 = fma(x, x, fma(y, y, z * z)), il = 1.0 / sqrt(q2);
+        add_mono<P>(x * il, y * il, z * il, q2 * S.w, A);
+    }
+    if (plate && N.w != 0.0f) {
+        double n0 = N.x, n1 = N.y, n2 = N.z;
+        const double in = 1.0 / sqrt(fma(n0, n0, fma(n1, n1, n2 * n2)));
+        n0 *= in; n1 *= in; n2 *= in;
         // u, v span the plane: u = a x n for the axis a of the smaller |n_a|
-        const bool ax = fabsf(N.x) < fabsf(N.z);
-        float u0 = ax ? 0.0f : N.y, u1 = ax ? -N.z : -N.x, u2 = ax ? N.y : 0.0f;
-        const float il = rsqrtf(fmaf(u0, u0, fmaf(u1, u1, u2 * u2)));
-        const bool ok = N.w != 0.0f;  // a voter without a plate may carry no normal
-        u0 = ok ? u0 * il : 0.0f;
-        u1 = ok ? u1 * il : 0.0f;
-        u2 = ok ? u2 * il : 0.0f;
-        const float v0 = N.y * u2 - N.z * u1, v1 = N.z * u0 - N.x * u2, v2 = N.x * u1 - N.y * u0;
-        const float w = N.w * (1.0f / (P + 2));
-        constexpr float cs[3][6] = {{1.0f, 0.707106781186547524f, 0.0f, -0.707106781186547524f, 0.0f, 0.0f},
-                                    {1.0f, 0.809016994374947424f, 0.309016994374947424f, -0.309016994374947424f,
-                                     -0.809016994374947424f, 0.0f},
-                                    {1.0f, 0.866025403784438647f, 0.5f, 0.0f, -0.5f, -0.866025403784438647f}};
-        constexpr float sn[3][6] = {{0.0f, 0.707106781186547524f, 1.0f, 0.707106781186547524f, 0.0f, 0.0f},
-                                    {0.0f, 0.587785252292473129f, 0.951056516295153572f, 0.951056516295153572f,
-                                     0.587785252292473129f, 0.0f},
-                                    {0.0f, 0.5f, 0.866025403784438647f, 1.0f, 0.866025403784438647f, 0.5f}};
+        const bool ax = fabs(n0) < fabs(n2);
+        double u0 = ax ? 0.0 : n1, u1 = ax ? -n2 : -n0, u2 = ax ? n1 : 0.0;
+        const double il = 1.0 / sqrt(fma(u0, u0, fma(u1, u1, u2 * u2)));
+        u0 *= il; u1 *= il; u2 *= il;
+        const double v0 = n1 * u2 - n2 * u1, v1 = n2 * u0 - n0 * u2, v2 = n0 * u1 - n1 * u0;
+        const double w = alpha * N.w * (1.0 / (P + 2));
+        constexpr double cs[4][6] = {{1.0, 0.5, -0.5, 0.0, 0.0, 0.0},
+                                     {1.0, 0.707106781186547524, 0.0, -0.707106781186547524, 0.0, 0.0},
+                                     {1.0, 0.809016994374947424, 0.309016994374947424, -0.309016994374947424,
+                                      -0.809016994374947424, 0.0},
+                                     {1.0, 0.866025403784438647, 0.5, 0.0, -0.5, -0.866025403784438647}};
+        constexpr double sn[4][6] = {{0.0, 0.866025403784438647, 0.866025403784438647, 0.0, 0.0, 0.0},
+                                     {0.0, 0.707106781186547524, 1.0, 0.707106781186547524, 0.0, 0.0},
+                                     {0.0, 0.587785252292473129, 0.951056516295153572, 0.951056516295153572,
+                                      0.587785252292473129, 0.0},
+                                     {0.0, 0.5, 0.866025403784438647, 1.0, 0.866025403784438647, 0.5}};
 #pragma unroll
         for (int i = 0; i < P + 2; i++) {
-            const float c = cs[P - 2][i], t = sn[P - 2][i];
-            add_mono<P>(fmaf(c, u0, t * v0), fmaf(c, u1, t * v1), fmaf(c, u2, t * v2), w, A);
+            const double c = cs[P - 1][i], t = sn[P - 1][i];
+            add_mono<P>(fma(c, u0, t * v0), fma(c, u1, t * v1), fma(c, u2, t * v2), w, A);
         }
     }
 }
@@ -937,18 +974,20 @@ __global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__
     }
 }
 
-// The same for powers above 1, from the padded voter payloads of the window
-// gather (vg): they are formed before this vote, with the FP64 re-solve of close
-// pairs, and serve the gather too where it has to vote instead.
+// The same in FP64 from the padded voter payloads of the window gather (vg):
+// they are formed before this vote, with the FP64 re-solve of close pairs, and
+// serve the gather too where it has to vote instead (*stop is set).
 template <int P>
 __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restrict__ ps, const float4* __restrict__ pp,
                                                           VoteGeom vg, SpecGeom g, int B, int C, int FG, FftPlan pl,
-                                                          const float2* __restrict__ twg, float2* __restrict__ Z) {
+                                                          const double2* __restrict__ twg, double2* __restrict__ Z,
+                                                          const unsigned long long* __restrict__ stop) {
+    if (*stop) return;
     constexpr int NF = mono_count(P);
-    extern __shared__ float2 xs_dyn[];  // C B L staged values, then L twiddles
+    extern __shared__ __align__(16) unsigned char fft_dyn[];  // C B L staged values, then L twiddles
     const int L = pl.L;
-    float2* s = xs_dyn;
-    float2* tw = xs_dyn + C * B * L;
+    double2* s = reinterpret_cast<double2*>(fft_dyn);
+    double2* tw = s + C * B * L;
     const int row0 = (int)blockIdx.x * B;
     const int nrows = g.n0 * g.n1;
     if (row0 >= nrows) return;
@@ -962,7 +1001,7 @@ __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restri
         if (j0) __syncthreads();  // the previous group's stores have read s
         for (int idx = (int)threadIdx.x; idx < Cv * Bv * npad; idx += kFT) {
             const int line = fdiv(idx, npad, rpad);
-            s[line * L + g.n2 + (idx - line * npad)] = make_float2(0.0f, 0.0f);
+            s[line * L + g.n2 + (idx - line * npad)] = make_double2(0.0, 0.0);
         }
         for (int idx = (int)threadIdx.x; idx < Bv * g.n2; idx += kFT) {
             const int b = fdiv(idx, g.n2, rn2), e = idx - b * g.n2;
@@ -970,12 +1009,12 @@ __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restri
             const size_t v = ((size_t)(z + vg.r) * vg.P1 + y + vg.r) * vg.P2 + e + vg.r;
             const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             const float4 S = g.stick ? ps[v] : zero, N = g.plate ? pp[v] : zero;
-            float A[(NF + 2) & ~1];
-            voter_features<P>(S, make_float4(N.x, N.y, N.z, N.w * g.alpha), g.stick != 0, g.plate != 0, A);
-            if (NF & 1) A[NF] = 0.0f;
+            double A[(NF + 2) & ~1];
+            voter_features<P>(S, N, (double)g.alpha, g.stick != 0, g.plate != 0, A);
+            if (NF & 1) A[NF] = 0.0;
 #pragma unroll
             for (int j = 0; j < (NF + 1) / 2; j++)
-                if (j >= j0 && j < j0 + Cv) s[((j - j0) * Bv + b) * L + e] = make_float2(A[2 * j], A[2 * j + 1]);
+                if (j >= j0 && j < j0 + Cv) s[((j - j0) * Bv + b) * L + e] = make_double2(A[2 * j], A[2 * j + 1]);
         }
         __syncthreads();
         for (int l0 = 0; l0 < Cv * Bv; l0 += FG) fft_lines<false>(s + l0 * L, pl, min(FG, Cv * Bv - l0), tw);
@@ -984,7 +1023,7 @@ __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restri
             const int c = fdiv(ln, Bv, rB), b = ln - c * Bv;
             const int row = row0 + b;
             const int z = fdiv(row, g.n1, rn1), y = row - z * g.n1;
-            float2* dst = Z + (size_t)(j0 + c) * g.cs + ((size_t)z * g.L1 + y) * g.P2;
+            double2* dst = Z + (size_t)(j0 + c) * g.cs + ((size_t)z * g.L1 + y) * g.P2;
             for (int e = (int)threadIdx.x & 63; e < L; e += 64) dst[e] = s[ln * L + e];
         }
     }
@@ -999,8 +1038,12 @@ __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restri
 // (the 1/2 and the inverse-FFT 1/(L0 L1 L2) are folded into the octant values);
 // then W_i(k) = Y_{2i}(k) + i Y_{2i+1}(k) and W_i(-k) = conj Y_{2i}(k) + i conj Y_{2i+1}(k)
 // overwrite Z_0..Z_2 (each group's frequencies belong to this thread only).
-__global__ __launch_bounds__(256) void k_spec_mul(float2* __restrict__ Z, const float* __restrict__ Kh,
-                                                  SpecGeom g) {
+// stop (FP64 only): nothing is done where *stop is set.
+template <class T, class V>
+__global__ __launch_bounds__(256) void k_spec_mul(V* __restrict__ Z, const T* __restrict__ Kh, SpecGeom g,
+                                                  const unsigned long long* __restrict__ stop) {
+    if constexpr (std::is_same_v<T, double>)
+        if (*stop) return;
     const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= g.ocs) return;
     const int kx = (int)(gid % (size_t)g.h2);
@@ -1013,22 +1056,22 @@ __global__ __launch_bounds__(256) void k_spec_mul(float2* __restrict__ Z, const 
 #pragma unroll
     for (int sl = 0; sl < 8; sl++)
         off[sl] = ((size_t)fz[(sl >> 2) & 1] * g.L1 + fy[(sl >> 1) & 1]) * g.P2 + fx[sl & 1];
-    float2 Y[4][6];
+    V Y[4][6];
 #pragma unroll
     for (int sl = 0; sl < 4; sl++)
 #pragma unroll
-        for (int c = 0; c < 6; c++) Y[sl][c] = make_float2(0.0f, 0.0f);
+        for (int c = 0; c < 6; c++) Y[sl][c] = mkc<V>(0, 0);
 
     // the next channel's eight values are in flight while this one is multiplied
-    float2 zn[8];
+    V zn[8];
 #pragma unroll
     for (int sl = 0; sl < 8; sl++) zn[sl] = Z[off[sl]];
     for (int j = 0; j < g.nz; j++) {
-        float2 z8[8];
+        V z8[8];
 #pragma unroll
         for (int sl = 0; sl < 8; sl++) z8[sl] = zn[sl];
         if (j + 1 < g.nz) {
-            const float2* zq = Z + (size_t)(j + 1) * g.cs;
+            const V* zq = Z + (size_t)(j + 1) * g.cs;
 #pragma unroll
             for (int sl = 0; sl < 8; sl++) zn[sl] = zq[off[sl]];
         }
@@ -1038,21 +1081,21 @@ __global__ __launch_bounds__(256) void k_spec_mul(float2* __restrict__ Z, const 
             if (f >= g.nf) break;
             const int odx = f < 64 ? (int)(g.odd_x >> f) : (int)(g.odd_x1 >> (f - 64));
             const int ody = f < 64 ? (int)(g.odd_y >> f) : (int)(g.odd_y1 >> (f - 64));
-            float2 F[4];
+            V F[4];
 #pragma unroll
             for (int sl = 0; sl < 4; sl++) {
-                const float2 a = z8[sl], bc = make_float2(z8[sl ^ 7].x, -z8[sl ^ 7].y);
-                F[sl] = h == 0 ? cadd(a, bc) : make_float2(a.y - bc.y, bc.x - a.x);
+                const V a = z8[sl], bc = mkc<V>(z8[sl ^ 7].x, -z8[sl ^ 7].y);
+                F[sl] = h == 0 ? cadd(a, bc) : mkc<V>(a.y - bc.y, bc.x - a.x);
             }
 #pragma unroll
             for (int c = 0; c < 6; c++) {
-                const float k = Kh[(size_t)(c * g.nf + f) * g.ocs + gid];
+                const T k = Kh[(size_t)(c * g.nf + f) * g.ocs + gid];
                 const bool ox = ((comp_nx(c) + odx) & 1) != 0, oy = ((comp_ny(c) + ody) & 1) != 0;
-                const float k1 = ox ? -k : k, k2 = oy ? -k : k, k3 = (ox != oy) ? -k : k;
-                Y[0][c].x = fmaf(k, F[0].x, Y[0][c].x);  Y[0][c].y = fmaf(k, F[0].y, Y[0][c].y);
-                Y[1][c].x = fmaf(k1, F[1].x, Y[1][c].x); Y[1][c].y = fmaf(k1, F[1].y, Y[1][c].y);
-                Y[2][c].x = fmaf(k2, F[2].x, Y[2][c].x); Y[2][c].y = fmaf(k2, F[2].y, Y[2][c].y);
-                Y[3][c].x = fmaf(k3, F[3].x, Y[3][c].x); Y[3][c].y = fmaf(k3, F[3].y, Y[3][c].y);
+                const T k1 = ox ? -k : k, k2 = oy ? -k : k, k3 = (ox != oy) ? -k : k;
+                Y[0][c].x = fmad(k, F[0].x, Y[0][c].x);  Y[0][c].y = fmad(k, F[0].y, Y[0][c].y);
+                Y[1][c].x = fmad(k1, F[1].x, Y[1][c].x); Y[1][c].y = fmad(k1, F[1].y, Y[1][c].y);
+                Y[2][c].x = fmad(k2, F[2].x, Y[2][c].x); Y[2][c].y = fmad(k2, F[2].y, Y[2][c].y);
+                Y[3][c].x = fmad(k3, F[3].x, Y[3][c].x); Y[3][c].y = fmad(k3, F[3].y, Y[3][c].y);
             }
         }
     }
@@ -1060,10 +1103,10 @@ __global__ __launch_bounds__(256) void k_spec_mul(float2* __restrict__ Z, const 
     for (int sl = 0; sl < 4; sl++) {
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            const float2 ya = Y[sl][2 * i], yb = Y[sl][2 * i + 1];
-            float2* zc = Z + (size_t)i * g.cs;
-            zc[off[sl]] = make_float2(ya.x - yb.y, ya.y + yb.x);
-            zc[off[sl ^ 7]] = make_float2(ya.x + yb.y, yb.x - ya.y);
+            const V ya = Y[sl][2 * i], yb = Y[sl][2 * i + 1];
+            V* zc = Z + (size_t)i * g.cs;
+            zc[off[sl]] = mkc<V>(ya.x - yb.y, ya.y + yb.x);
+            zc[off[sl ^ 7]] = mkc<V>(ya.x + yb.y, yb.x - ya.y);
         }
     }
 }
@@ -1113,6 +1156,48 @@ __global__ __launch_bounds__(kFT) void k_spec_xinv(const float2* __restrict__ Z,
     }
 }
 
+// The same in FP64, rounded as it is written.
+__global__ __launch_bounds__(kFT) void k_spec_xinv64(const double2* __restrict__ Z, SpecGeom g, int B, FftPlan pl,
+                                                     const double2* __restrict__ twg, float* __restrict__ out,
+                                                     int layout, const unsigned long long* __restrict__ stop) {
+    if (*stop) return;
+    extern __shared__ __align__(16) unsigned char fft_dyn[];  // 3 B L staged values, then L twiddles
+    const int L = pl.L;
+    double2* s = reinterpret_cast<double2*>(fft_dyn);
+    double2* tw = s + 3 * B * L;
+    const int row0 = (int)blockIdx.x * B;
+    const int nrows = g.n0 * g.n1;
+    if (row0 >= nrows) return;
+    const int Bv = min(B, nrows - row0);
+    load_twiddles(tw, twg, L);
+    const float rL = 1.0f / (float)L, rn1 = 1.0f / (float)g.n1, rn2 = 1.0f / (float)g.n2;
+    for (int idx = (int)threadIdx.x; idx < 3 * Bv * L; idx += kFT) {
+        const int line = fdiv(idx, L, rL), e = idx - line * L;  // line = 3 l + i
+        const int l = fdiv(line, 3, 1.0f / 3.0f), i = line - 3 * l;
+        const int row = row0 + l;
+        const int z = fdiv(row, g.n1, rn1), y = row - z * g.n1;
+        s[line * L + e] = Z[(size_t)i * g.cs + ((size_t)z * g.L1 + y) * g.P2 + e];
+    }
+    __syncthreads();
+    fft_lines<true>(s, pl, 3 * Bv, tw);
+    for (int idx = (int)threadIdx.x; idx < Bv * g.n2; idx += kFT) {
+        const int l = fdiv(idx, g.n2, rn2), x = idx - l * g.n2;
+        const double2 w0 = s[(3 * l + 0) * L + x], w1 = s[(3 * l + 1) * L + x], w2 = s[(3 * l + 2) * L + x];
+        const float xx = (float)w0.x, xy = (float)w0.y, xz = (float)w1.x, yy = (float)w1.y, yz = (float)w2.x,
+                    zz = (float)w2.y;
+        const size_t v = (size_t)(row0 + l) * g.n2 + x;
+        if (layout == TIRA_LAYOUT_MAT9) {
+            float* o = out + v * 9;
+            o[0] = xx; o[1] = xy; o[2] = xz;
+            o[3] = xy; o[4] = yy; o[5] = yz;
+            o[6] = xz; o[7] = yz; o[8] = zz;
+        } else {
+            float* o = out + v * 6;
+            o[0] = xx; o[1] = xy; o[2] = xz; o[3] = yy; o[4] = yz; o[5] = zz;
+        }
+    }
+}
+
 // ---------------------------------------------------------------- kernel spectra
 // Separable FP64 transforms of the offset kernels K[ch][dw][dv][du] (parity
 // of channel ch along x / y / z in bits 0 / 1 / 2 of par[ch]): cosine along
@@ -1151,8 +1236,9 @@ __global__ __launch_bounds__(256) void k_khat_y(const double* __restrict__ T1, c
     }
 }
 
+template <class T>
 __global__ __launch_bounds__(256) void k_khat_z(const double* __restrict__ T2, const double* __restrict__ trig,
-                                                const unsigned char* __restrict__ par, float* __restrict__ Kh,
+                                                const unsigned char* __restrict__ par, T* __restrict__ Kh,
                                                 int w, int h0, int h1, int h2, int nch, double scale) {
     const size_t plane = (size_t)h1 * h2;
     const size_t n = (size_t)nch * h0 * plane;
@@ -1166,7 +1252,7 @@ __global__ __launch_bounds__(256) void k_khat_z(const double* __restrict__ T2, c
         double acc = 0.0;
         for (int d = 0; d < w; d++) acc = fma(src[(size_t)d * plane], tr[d], acc);
         const int odd = (pb & 1) + ((pb >> 1) & 1) + ((pb >> 2) & 1);
-        Kh[i] = (float)((odd == 2 ? -scale : scale) * acc);  // (-i)^2 for two sine axes
+        Kh[i] = (T)((odd == 2 ? -scale : scale) * acc);  // (-i)^2 for two sine axes
     }
 }
 
@@ -1407,10 +1493,10 @@ static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate
 struct SpecKey {
     int L0, L1, L2, w;
     float s1, s2;
-    int power, atv;
+    int power, atv, f64;
     bool operator==(const SpecKey& o) const {
         return L0 == o.L0 && L1 == o.L1 && L2 == o.L2 && w == o.w && s1 == o.s1 && s2 == o.s2 &&
-               power == o.power && atv == o.atv;
+               power == o.power && atv == o.atv && f64 == o.f64;
     }
 };
 
@@ -1418,7 +1504,7 @@ struct SpecKey {
 // caller alternating between shapes or scales rebuilds nothing), evicted
 // least recently used beyond kSpecEntries or 1/8 of the device's memory.
 struct SpecEntry {
-    SpecKey key{0, 0, 0, 0, 0, 0, 0, 0};
+    SpecKey key{0, 0, 0, 0, 0, 0, 0, 0, 0};
     int device = -1;
     void* buf = nullptr;  // twiddles (3 axes) then the octant spectra
     size_t bytes = 0;
@@ -1469,28 +1555,36 @@ static size_t spec_held(int dev) {
     return b;
 }
 
-static void twiddles(int L, float2* t) {
+template <class V>
+static void twiddles(int L, V* t) {
     for (int j = 0; j < L; j++) {
         const double a = -2.0 * M_PI * (double)j / (double)L;
-        t[j] = make_float2((float)std::cos(a), (float)std::sin(a));
+        t[j].x = (real_of<V>)std::cos(a);
+        t[j].y = (real_of<V>)std::sin(a);
     }
 }
 
-static size_t tw_bytes(int L) { return ((size_t)L * 8 + 255) & ~size_t(255); }
+template <class V = float2>
+static size_t tw_bytes(int L) {
+    return ((size_t)L * sizeof(V) + 255) & ~size_t(255);
+}
 
-// Kernel spectra for `key` (built and uploaded unless cached).
-static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, const float2** tw0,
-                       const float2** tw1, const float2** tw2, const float** kh) {
+// Kernel spectra and twiddles for `key` (built and uploaded unless cached), V
+// the complex type of its transforms.
+template <class V>
+static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, const V** tw0, const V** tw1,
+                       const V** tw2, const real_of<V>** kh) {
+    using T = real_of<V>;
     int dev = 0;
     TH_HIP(hipGetDevice(&dev));
-    const size_t tb = tw_bytes(key.L0) + tw_bytes(key.L1) + tw_bytes(key.L2);
-    const size_t kbytes = (size_t)6 * g.nf * g.ocs * 4;
+    const size_t tb0 = tw_bytes<V>(key.L0), tb1 = tw_bytes<V>(key.L1), tb = tb0 + tb1 + tw_bytes<V>(key.L2);
+    const size_t kbytes = (size_t)6 * g.nf * g.ocs * sizeof(T);
     auto set_ptrs = [&](const SpecEntry& x) {
         char* b = (char*)x.buf;
-        *tw0 = (const float2*)b;
-        *tw1 = (const float2*)(b + tw_bytes(key.L0));
-        *tw2 = (const float2*)(b + tw_bytes(key.L0) + tw_bytes(key.L1));
-        *kh = (const float*)(b + tb);
+        *tw0 = (const V*)b;
+        *tw1 = (const V*)(b + tb0);
+        *tw2 = (const V*)(b + tb0 + tb1);
+        *kh = (const T*)(b + tb);
     };
     g_spec.clock++;
     for (auto& x : g_spec.e)
@@ -1537,10 +1631,10 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
 
     // twiddles
     {
-        std::vector<float2> t(tb / 8);
+        std::vector<V> t(tb / sizeof(V));
         twiddles(key.L0, t.data());
-        twiddles(key.L1, t.data() + tw_bytes(key.L0) / 8);
-        twiddles(key.L2, t.data() + (tw_bytes(key.L0) + tw_bytes(key.L1)) / 8);
+        twiddles(key.L1, t.data() + tb0 / sizeof(V));
+        twiddles(key.L2, t.data() + (tb0 + tb1) / sizeof(V));
         TH_HIP(hipMemcpy(ent.buf, t.data(), tb, hipMemcpyHostToDevice));
     }
     // offset kernels (the stick's, or the ATV's e2 part, only: the plate part,
@@ -1607,7 +1701,7 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
         k_khat_x<<<grid(t1n), 256, 0, st>>>(dK, dtr[2], dpar, dT1, w, g.h2, nch);
         k_khat_y<<<grid(t2n), 256, 0, st>>>(dT1, dtr[1], dpar, dT2, w, g.h1, g.h2, nch);
         const double scale = 0.5 / ((double)g.L0 * g.L1 * g.L2);
-        k_khat_z<<<grid((size_t)nch * g.ocs), 256, 0, st>>>(dT2, dtr[0], dpar, (float*)*kh, w, g.h0, g.h1, g.h2,
+        k_khat_z<<<grid((size_t)nch * g.ocs), 256, 0, st>>>(dT2, dtr[0], dpar, const_cast<T*>(*kh), w, g.h0, g.h1, g.h2,
                                                            nch, scale);
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) rc = -2;
     } while (false);
@@ -1622,6 +1716,21 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
     return TIRA_OK;
 }
 
+// Column passes in FP64 (stop: nothing is done where *stop is set).
+static int launch_cols64(double2* data, const LineGeom& lg, const FftPlan& pl, const double2* tw, bool inv,
+                         const unsigned long long* stop, hipStream_t st) {
+    const size_t nblk = (size_t)lg.nab * lg.nb * lg.nchan;
+    if (nblk == 0) return TIRA_OK;
+    TH_ARG(nblk < (1ull << 31), "spectral vote: volume too large");
+    const size_t clds = ((size_t)lg.B * pl.L + pl.L) * sizeof(double2);
+    TH_ARG(clds <= kColsLds && lg.Bh >= 1 && lg.B % lg.Bh == 0 && (size_t)lg.Bh * pl.L <= (size_t)kFftBL64,
+           "spectral vote: column batch exceeds the staging");
+    if (inv) k_fft_cols<true, kFftBL64, 1><<<(unsigned)nblk, kFT, clds, st>>>(data, lg, pl, tw, stop);
+    else k_fft_cols<false, kFftBL64, 1><<<(unsigned)nblk, kFT, clds, st>>>(data, lg, pl, tw, stop);
+    TH_HIP(hipGetLastError());
+    return TIRA_OK;
+}
+
 static int launch_lines(float2* data, const LineGeom& lg, const FftPlan& pl, const float2* tw, bool inv, bool rows,
                         hipStream_t st) {
     const size_t nblk = (size_t)lg.nab * lg.nb * lg.nchan;
@@ -1633,12 +1742,12 @@ static int launch_lines(float2* data, const LineGeom& lg, const FftPlan& pl, con
            "spectral vote: column batch exceeds the staging");
     if (inv) {
         if (rows) k_fft_lines<true, true><<<grid, kFT, 0, st>>>(data, lg, pl, tw);
-        else if (lg.Bh >= 16) k_fft_cols<true, kFftBL, 6><<<grid, kFT, clds, st>>>(data, lg, pl, tw);
-        else k_fft_cols<true, kFftBL, 1><<<grid, kFT, clds, st>>>(data, lg, pl, tw);
+        else if (lg.Bh >= 16) k_fft_cols<true, kFftBL, 6><<<grid, kFT, clds, st>>>(data, lg, pl, tw, nullptr);
+        else k_fft_cols<true, kFftBL, 1><<<grid, kFT, clds, st>>>(data, lg, pl, tw, nullptr);
     } else {
         if (rows) k_fft_lines<false, true><<<grid, kFT, 0, st>>>(data, lg, pl, tw);
-        else if (lg.Bh >= 16) k_fft_cols<false, kFftBL, 6><<<grid, kFT, clds, st>>>(data, lg, pl, tw);
-        else k_fft_cols<false, kFftBL, 1><<<grid, kFT, clds, st>>>(data, lg, pl, tw);
+        else if (lg.Bh >= 16) k_fft_cols<false, kFftBL, 6><<<grid, kFT, clds, st>>>(data, lg, pl, tw, nullptr);
+        else k_fft_cols<false, kFftBL, 1><<<grid, kFT, clds, st>>>(data, lg, pl, tw, nullptr);
     }
     TH_HIP(hipGetLastError());
     return TIRA_OK;
@@ -1647,7 +1756,7 @@ static int launch_lines(float2* data, const LineGeom& lg, const FftPlan& pl, con
 // Lines of the axis with stride `estride` over a (n0 x n1 x n2)-indexed
 // stack: the batch dimension `a` is x (stride 1) for the y and z axes.
 static LineGeom strided_geom(size_t cs, int nchan, int L, size_t estride, int na, int nb, size_t bstride, int n_in,
-                             int n_out) {
+                             int n_out, size_t bytes = sizeof(float2)) {
     LineGeom g{};
     g.cstride = cs;
     g.bstride = bstride;
@@ -1656,13 +1765,14 @@ static LineGeom strided_geom(size_t cs, int nchan, int L, size_t estride, int na
     g.na = na;
     g.nb = nb;
     g.nchan = nchan;
-    // B: up to 16 adjacent lines (128-byte rows of complex values) within
+    // B: adjacent lines of up to 128 bytes a row (16 values of 8 bytes) within
     // kColsLds of staging; Bh: the largest group of them the middle stages
-    // take at once (Bh L <= kFftBL)
+    // take at once (Bh L <= kFftBL, or half of it in FP64)
+    const int most = (int)(128 / bytes), bl = bytes == sizeof(float2) ? kFftBL : kFftBL64;
     int B = 1, lb = 0;
-    while (2 * B <= 16 && ((size_t)2 * B * L + L) * sizeof(float2) <= kColsLds) { B *= 2; lb++; }
+    while (2 * B <= most && ((size_t)2 * B * L + L) * bytes <= kColsLds) { B *= 2; lb++; }
     int Bh = B;
-    while (Bh > 1 && Bh * L > kFftBL) Bh /= 2;
+    while (Bh > 1 && Bh * L > bl) Bh /= 2;
     g.B = B;
     g.lb = lb;
     g.Bh = Bh;
@@ -1684,18 +1794,21 @@ static bool spectral_serves(unsigned p, bool plate, unsigned samples) {
 // costs microseconds and the first call's spectra build would dominate), and
 // device memory for the spectra, their build and the feature volumes within
 // 80% of the device.
-// Above power 1 the features are more (28, 45, 66 for 15) and the line lies
-// where neither time nor error against 64 bits is worse than the gather's,
-// measured from 32^3 to 128^3: power 2 at w = 9 takes 69 us for 718 us (32^3)
-// and 555 for 2296 (128^3) at 5e-7 for 4.6e-7, power 3 931 for 2575 (128^3) at
-// 4.8e-7 for 5e-7; power 2 at w = 13 549 for 6598 us (128^3) at 5.2e-7 for
-// 6.3e-7, power 4 1329 for 7195 us at 7.3e-7 for 7.7e-7. At w = 7 the gather's
-// error is the smaller (3.3e-7 for 5e-7), at w = 5 its time too.
+// Above power 1 the features are more (28, 45, 66 for 15) and the transforms FP64
+// (spectral_run64); the line is one of time, with the error the smaller on its
+// whole side (3.3e-8 against 64 bits for the gather's 4.8e-7 at 40 x 45 x 50,
+// power 2, w = 9, and 6.0e-7 at 91 x 117 x 101, w = 13). Spectral for gather, in
+// us: power 2, w = 9: 95 for 713 (32^3), 217 for 748 (64^3), 1159 for 2108 (128^3),
+// 4687 for 8967 (200^3); power 3, w = 9: 119 for 731, 313 for 792, 1760 for 2248,
+// 7507 for 9828, and 665 for 770 at 30 x 30 x 512; power 4, w = 11: 155 for 1369,
+// 456 for 1435, 2595 for 4348. At w = 7 the gather takes a third to a half of its
+// time at 9.
 // With `atv`: analytical tensor voting, whose features come from the input
 // tensors in the x pass only.
 bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsigned power, bool stick, bool plate,
                         unsigned samples, bool atv) {
     const unsigned p = power < 1 || atv ? 1 : power;
+    const bool f64 = p > 1;
     if (!atv && !spectral_serves(p, plate, samples)) return false;
     if (w < (p == 1 ? 5u : p < 4 ? 9u : 11u) || (size_t)s0 * s1 * s2 < 32768) return false;
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);
@@ -1704,8 +1817,9 @@ bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsig
     const size_t W = 2 * (w / 2) + 1;
     const size_t h0 = L0 / 2 + 1, h1 = L1 / 2 + 1, h2 = L2 / 2 + 1;
     // payloads: of the field, above power 1 padded for the window gather
-    const size_t pay = p == 1 ? (size_t)s0 * s1 * s2 : vote3_payload_voxels(s0, s1, s2, (unsigned)W);
-    const size_t need = nz * (size_t)L0 * L1 * L2 * 8 + 6 * nf * h0 * h1 * h2 * 4 + 6 * nf * W * h1 * h2 * 8 + pay * 32;
+    const size_t pay = !f64 ? (size_t)s0 * s1 * s2 : vote3_payload_voxels(s0, s1, s2, (unsigned)W);
+    const size_t need = nz * (size_t)L0 * L1 * L2 * (f64 ? 16 : 8) + 6 * nf * h0 * h1 * h2 * (f64 ? 8 : 4) +
+                        6 * nf * W * h1 * h2 * 8 + pay * 32;
     size_t free_b = 0, total_b = 0;
     int dev = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
@@ -1719,12 +1833,129 @@ bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsig
 }
 
 static void launch_xfwd_pay(int power, unsigned grid, size_t lds, hipStream_t st, const SpecPayload& v,
-                            const SpecGeom& g, int B, int C, int FG, const FftPlan& pl, const float2* tw, float2* Z) {
+                            const SpecGeom& g, int B, int C, int FG, const FftPlan& pl, const double2* tw,
+                            double2* Z) {
     switch (power) {
-        case 2: k_spec_xfwd_pay<2><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z); break;
-        case 3: k_spec_xfwd_pay<3><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z); break;
-        default: k_spec_xfwd_pay<4><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z); break;
+        case 2: k_spec_xfwd_pay<2><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
+        case 3: k_spec_xfwd_pay<3><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
+        default: k_spec_xfwd_pay<4><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
     }
+}
+
+// How the forward x pass takes the rows of a field.
+struct XfwdPlan {
+    int B, C, FG;  // rows per block, channels per group, lines per transform
+    size_t lds;
+};
+static XfwdPlan xfwd_plan(const SpecGeom& g, const FftPlan& p2, size_t bytes) {
+    // Channels per group: all of them when the lines of one row fit 64 KB of
+    // LDS, so that each voxel's eigen-solve and features are computed once;
+    // else the fewest balanced groups that fit. The staged lines are
+    // transformed in groups of FG that fit every stage's register rounds (at
+    // L = 540 two channel groups had solved every voxel twice).
+    XfwdPlan x;
+    x.C = g.nz;
+    for (int ng = 1; ng <= g.nz; ng++) {
+        x.C = (g.nz + ng - 1) / ng;
+        if (((size_t)x.C * g.L2 + g.L2) * bytes <= 65536) break;
+    }
+    // Rows per block: among the counts that fit 64 KB of dynamic LDS (and,
+    // where one row's lines fit the stages' rounds, whose lines all do), the
+    // one whose voxels best fill whole passes of the block's threads in the
+    // eigen-solve (ties: more rows). 128-wide rows of 8 channels take 4 rows
+    // (512 voxels, 4320 values), not the 3 that fit 4096 values (384 voxels:
+    // half the threads solving twice).
+    const bool row_fits = lines_fit(p2, x.C);
+    x.B = 1;
+    double best = -1.0;
+    for (int b = 1; b <= 64; b++) {
+        if (((size_t)x.C * b * g.L2 + g.L2) * bytes > 65536 || (row_fits && !lines_fit(p2, x.C * b))) break;
+        const int vox = b * g.n2, passes = (vox + kFT - 1) / kFT;
+        const double fill = (double)vox / ((double)passes * kFT);
+        if (fill >= best) { best = fill; x.B = b; }
+        if (vox >= 4 * kFT) break;
+    }
+    x.FG = x.C * x.B;
+    for (int ng = 1; !lines_fit(p2, x.FG); ng++) x.FG = (x.C * x.B + ng) / (ng + 1);
+    x.lds = ((size_t)x.C * x.B * g.L2 + g.L2) * bytes;
+    return x;
+}
+
+// Rows per block of the inverse x pass, at most Bmax: the count whose grid best
+// fills whole rounds of the resident blocks (four per CU). 128^2 rows of L = 135
+// take 8 rows (2048 blocks, two full rounds), not 10 (1639 blocks: a second
+// round 60% full).
+static int xinv_rows(size_t nrows, int Bmax) {
+    const double slots = 4.0 * cu_count();
+    int B = Bmax;
+    double best = -1.0;
+    for (int b = Bmax; b >= std::max(1, Bmax / 2); b--) {
+        const double rounds = (double)ceil_div(nrows, (size_t)b) / slots;
+        const double fill = rounds / std::ceil(rounds);
+        if (fill > best + 0.02) { best = fill; B = b; }
+    }
+    return B;
+}
+
+// The vote in FP64 from the payloads `pay`: every value between the voters' FP32
+// payload and the FP32 result. The transforms of FP32 round by the norm of the
+// whole field, the window gather by that of a receiver's own window: beside
+// bright voters the votes of faint ones kept 3 digits where the gather kept 6
+// (7e-4 of a receiver's vote down to 1e-4 of the largest, gather 2e-6).
+static int spectral_run64(const SpecGeom& g, const FftPlan& p0, const FftPlan& p1, const FftPlan& p2, const SpecKey& key,
+                          const SpecPayload& pay, float* out, int out_layout, hipStream_t st) {
+    double2* Z = nullptr;
+    const double2 *tw0, *tw1, *tw2;
+    const double* kh;
+    int rc = ws_get(WS_SPEC0, (size_t)g.nz * g.cs * sizeof(double2), (void**)&Z);
+    if (rc == TIRA_OK) rc = spectra_for(key, g, st, &tw0, &tw1, &tw2, &kh);
+    if (rc == TIRA_ERR_OUT_OF_MEMORY) {
+        (void)hipGetLastError();
+        return kSpectralNotApplicable;
+    }
+    TH_TRY(rc);
+    const size_t row = (size_t)g.P2, plane = (size_t)g.L1 * row, nrows = (size_t)g.n0 * g.n1, cb = sizeof(double2);
+    {
+        ProfScope prof("spec_fwd_x", st);
+        const XfwdPlan x = xfwd_plan(g, p2, cb);
+        const unsigned grid = ceil_div(nrows, (size_t)x.B);
+        launch_xfwd_pay(g.power, grid, x.lds, st, pay, g, x.B, x.C, x.FG, p2, tw2, Z);
+        TH_HIP(hipGetLastError());
+    }
+    {
+        ProfScope prof("spec_fwd_y", st);
+        TH_TRY(launch_cols64(Z, strided_geom(g.cs, g.nz, g.L1, row, g.L2, g.n0, plane, g.n1, g.L1, cb), p1, tw1, false,
+                             pay.stop, st));
+    }
+    {
+        ProfScope prof("spec_fwd_z", st);
+        TH_TRY(launch_cols64(Z, strided_geom(g.cs, g.nz, g.L0, plane, g.L2, g.L1, row, g.n0, g.L0, cb), p0, tw0, false,
+                             pay.stop, st));
+    }
+    {
+        ProfScope prof("spec_mul", st);
+        k_spec_mul<<<(unsigned)ceil_div(g.ocs, 256), 256, 0, st>>>(Z, kh, g, pay.stop);
+        TH_HIP(hipGetLastError());
+    }
+    {
+        ProfScope prof("spec_inv_z", st);
+        TH_TRY(launch_cols64(Z, strided_geom(g.cs, 3, g.L0, plane, g.L2, g.L1, row, g.L0, g.n0, cb), p0, tw0, true,
+                             pay.stop, st));
+    }
+    {
+        ProfScope prof("spec_inv_y", st);
+        TH_TRY(launch_cols64(Z, strided_geom(g.cs, 3, g.L1, row, g.L2, g.n0, plane, g.L1, g.n1, cb), p1, tw1, true,
+                             pay.stop, st));
+    }
+    {
+        ProfScope prof("spec_inv_x", st);
+        // 64 KB of staged values and twiddles: one row of 1024 fits
+        const int B = xinv_rows(nrows, std::max(1, (65536 / (int)cb - g.L2) / (3 * g.L2)));
+        const size_t lds = ((size_t)3 * B * g.L2 + g.L2) * cb;
+        k_spec_xinv64<<<ceil_div(nrows, (size_t)B), kFT, lds, st>>>(Z, g, B, p2, tw2, out, out_layout, pay.stop);
+        TH_HIP(hipGetLastError());
+    }
+    return TIRA_OK;
 }
 
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
@@ -1772,40 +2003,13 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     g.ocs = (size_t)g.h0 * g.h1 * g.h2;
 
     const size_t nvox = (size_t)s0 * s1 * s2;
-    // Channels per group: all of them when the lines of one row fit 64 KB of
-    // LDS, so that each voxel's eigen-solve and features are computed once;
-    // else the fewest balanced groups that fit. The staged lines are
-    // transformed in groups of FG that fit every stage's register rounds (at
-    // L = 540 two channel groups had solved every voxel twice).
-    int C = g.nz;
-    for (int ng = 1; ng <= g.nz; ng++) {
-        C = (g.nz + ng - 1) / ng;
-        if (((size_t)C * g.L2 + g.L2) * 8 <= 65536) break;
-    }
-    // Rows per block: among the counts that fit 64 KB of dynamic LDS (and,
-    // where one row's lines fit the stages' rounds, whose lines all do), the
-    // one whose voxels best fill whole passes of the block's threads in the
-    // eigen-solve (ties: more rows). 128-wide rows of 8 channels take 4 rows
-    // (512 voxels, 4320 values), not the 3 that fit 4096 values (384 voxels:
-    // half the threads solving twice).
-    const bool row_fits = lines_fit(p2, C);
-    int B = 1;
-    {
-        double best = -1.0;
-        for (int b = 1; b <= 64; b++) {
-            if (((size_t)C * b * g.L2 + g.L2) * 8 > 65536 || (row_fits && !lines_fit(p2, C * b))) break;
-            const int vox = b * g.n2, passes = (vox + kFT - 1) / kFT;
-            const double fill = (double)vox / ((double)passes * kFT);
-            if (fill >= best) { best = fill; B = b; }
-            if (vox >= 4 * kFT) break;
-        }
-    }
-    int FG = C * B;
-    for (int ng = 1; !lines_fit(p2, FG); ng++) FG = (C * B + ng) / (ng + 1);
-    const size_t xlds = ((size_t)C * B * g.L2 + g.L2) * 8;
+    // the spectra are those of the stick part whatever the stick / plate selection
+    const SpecKey key{g.L0, g.L1, g.L2, (int)w, sigma1, sigma2, (int)p, atv ? 1 : 0, pay ? 1 : 0};
+    if (pay) return spectral_run64(g, p0, p1, p2, key, *pay, out, out_layout, st);
+    const XfwdPlan x = xfwd_plan(g, p2, sizeof(float2));
     // tensor input: the x pass decomposes the voxels itself, in every channel
     // group (no payload round trip); eigenpair input goes through the payload
-    const bool fused = pay || tensors != nullptr;
+    const bool fused = tensors != nullptr;
     float4 *ps = nullptr, *pp = nullptr;
     float2* Z = nullptr;
     // Out of device memory for the spectral buffers: clear the error and let
@@ -1821,8 +2025,6 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
         return rc == TIRA_ERR_OUT_OF_MEMORY ? kSpectralNotApplicable : rc;
     if ((rc = alloc(ws_get(WS_SPEC0, (size_t)g.nz * g.cs * 8, (void**)&Z))) != TIRA_OK)
         return rc == TIRA_ERR_OUT_OF_MEMORY ? kSpectralNotApplicable : rc;
-    // the spectra are those of the stick part whatever the stick / plate selection
-    const SpecKey key{g.L0, g.L1, g.L2, (int)w, sigma1, sigma2, (int)p, atv ? 1 : 0};
     const float2 *tw0, *tw1, *tw2;
     const float* kh;
     if ((rc = alloc(spectra_for(key, g, st, &tw0, &tw1, &tw2, &kh))) != TIRA_OK)
@@ -1836,14 +2038,13 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     {
         ProfScope prof("spec_fwd_x", st);
         const size_t nrows = (size_t)s0 * s1;
-        const size_t nblk = ceil_div(nrows, (size_t)B);
+        const size_t nblk = ceil_div(nrows, (size_t)x.B);
         TH_ARG(nblk < (1ull << 31), "spectral vote: volume too large");
-        if (pay)
-            launch_xfwd_pay(g.power, (unsigned)nblk, xlds, st, *pay, g, B, C, FG, p2, tw2, Z);
-        else if (fused)
-            k_spec_xfwd<true><<<(unsigned)nblk, kFT, xlds, st>>>(ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z);
+        const unsigned grid = (unsigned)nblk;
+        if (fused)
+            k_spec_xfwd<true><<<grid, kFT, x.lds, st>>>(ps, pp, tensors, in_layout, g, x.B, x.C, x.FG, p2, tw2, Z);
         else
-            k_spec_xfwd<false><<<(unsigned)nblk, kFT, xlds, st>>>(ps, pp, tensors, in_layout, g, B, C, FG, p2, tw2, Z);
+            k_spec_xfwd<false><<<grid, kFT, x.lds, st>>>(ps, pp, tensors, in_layout, g, x.B, x.C, x.FG, p2, tw2, Z);
         TH_HIP(hipGetLastError());
     }
     {
@@ -1858,7 +2059,7 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     }
     {
         ProfScope prof("spec_mul", st);
-        k_spec_mul<<<(unsigned)ceil_div(g.ocs, 256), 256, 0, st>>>(Z, kh, g);
+        k_spec_mul<<<(unsigned)ceil_div(g.ocs, 256), 256, 0, st>>>(Z, kh, g, nullptr);
         TH_HIP(hipGetLastError());
     }
     {
@@ -1873,22 +2074,8 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
     }
     {
         ProfScope prof("spec_inv_x", st);
-        // Rows per block: up to the staging's 4096 values, the count whose grid
-        // best fills whole rounds of the resident blocks (four per CU). 128^2
-        // rows of L = 135 take 8 rows (2048 blocks, two full rounds), not 10
-        // (1639 blocks: a second round 60% full).
         const size_t nrows = (size_t)s0 * s1;
-        const int Bmax = std::max(1, kFftBL / (3 * g.L2));
-        const double slots = 4.0 * cu_count();
-        int B = Bmax;
-        {
-            double best = -1.0;
-            for (int b = Bmax; b >= std::max(1, Bmax / 2); b--) {
-                const double rounds = (double)ceil_div(nrows, (size_t)b) / slots;
-                const double fill = rounds / std::ceil(rounds);
-                if (fill > best + 0.02) { best = fill; B = b; }
-            }
-        }
+        const int B = xinv_rows(nrows, std::max(1, kFftBL / (3 * g.L2)));  // within the staging's 4096 values
         k_spec_xinv<<<ceil_div(nrows, (size_t)B), kFT, 0, st>>>(Z, g, B, p2, tw2, out, out_layout,
                                                                 eig ? eig->evals : nullptr, eig ? eig->flags : 0u,
                                                                 eig ? eig->n_refined : nullptr);

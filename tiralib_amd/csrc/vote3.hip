@@ -1415,7 +1415,7 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     float2* dcs = nullptr;
     TH_TRY(table_for(key, P, st, &dtab, &dcs));
     if (spectral) {
-        const SpecPayload pay{ps, pp, g};
+        const SpecPayload pay{ps, pp, g, gate};
         const int rc = vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0, s1, s2, sigma1, sigma2,
                                           w, power, stick, plate, samples, false, st, nullptr, &pay);
         if (rc == kSpectralNotApplicable) gate = nullptr;  // no memory for it: the gather, as it stands
@@ -1664,7 +1664,7 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
         // sticks overwrites the spectral ones if any voter is such.
         bool spectral = false;
         if (stick && spectral_preferred(s0, s1, s2, w, m->power, true, false, 0)) {
-            const SpecPayload pay{ps, nullptr, g};
+            const SpecPayload pay{ps, nullptr, g, cnt + 1};
             const int rc = vote3_spectral_run(tensors, in_layout, nullptr, nullptr, nullptr, out, out_layout, s0, s1, s2,
                                               m->sigma1, m->sigma2, w, m->power, true, false, 0, false, st, nullptr,
                                               m->power > 1 ? &pay : nullptr);

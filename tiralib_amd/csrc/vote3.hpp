@@ -36,15 +36,17 @@ struct EigOut {
 };
 // Status of vote3_spectral_run when the request is outside the spectral method.
 constexpr int kSpectralNotApplicable = -1;
-// Voters of a spectral vote above power 1: the padded payloads of the window
-// gather, formed (and the voters looked over, see k_vote3_prep) before it.
+// Voters of a spectral vote in FP64: the padded payloads of the window gather,
+// formed (and the voters looked over, see k_vote3_prep) before it. stop (device):
+// set where the gather has to vote instead; the vote then leaves `out` alone.
 struct SpecPayload {
     const float4 *ps, *pp;
     VoteGeom g;
+    const unsigned long long* stop;
 };
 // Padded payload voxels of the window gather.
 size_t vote3_payload_voxels(unsigned s0, unsigned s1, unsigned s2, unsigned w);
-// pay: given above power 1 and only there.
+// pay: the vote in FP64; given above power 1 and only there.
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        float* out, int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1,
                        float sigma2, unsigned w, unsigned power, bool stick, bool plate, unsigned samples,
