@@ -12,9 +12,9 @@
 // quartic monomials q_x^a q_y^b q_z^c (a + b + c = 4), so
 //     V_c(x) = sum_f sum_d K_{c,f}(d) F_f(x + d),      c = xx, xy, xz, yy, yz, zz,
 // with offset kernels K_{c,f}(d) of the stick vote fitted in FP64 (on the device,
-// once per parameter set). The plate vote integrates the stick vote over the great circle
-// perpendicular to n, and averaging a quartic over that circle is a fixed
-// linear map on the 15 monomials (add_circle_average), so the plate kernels
+// once per parameter set). The plate vote integrates the stick vote over the
+// great circle perpendicular to n, and averaging a quartic over that circle is a
+// fixed linear map on the 15 monomials (add_circle_average), so the plate kernels
 // are the stick kernels times that map and both votes share them: the voter
 // features are F_f = s m_f(e2) + sticknorm3 t (circle average of m(e0))_f.
 // The whole field's vote is a 15-in / 6-out correlation with a w^3 window:
@@ -23,9 +23,10 @@
 // Powers 2 to 4 are the same with degree g = 2 p + 2 (eta has degree 2 p):
 // (g + 1)(g + 2) / 2 = 28, 45 or 66 monomials. Their circle averages are
 // evaluated as the mean over p + 2 equispaced directions of the half circle,
-// which is exact for a trigonometric polynomial of degree g. The window gather
-// serves every other request of these powers, so theirs runs in FP64 from the
-// gather's payloads (spectral_run64): no vote is further from 64 bits than it was.
+// which is exact for a trigonometric polynomial of degree g. These votes, and the
+// sticks of the learned vote, run in FP64 from the payloads of the window gather
+// that serves them otherwise (spectral_run64): its rounding is that of a
+// receiver's own window, the FP32 transforms' that of the whole field.
 //
 // Pipeline of one call (device buffers, zero padding to L >= n + w/2 per axis
 // so the circular convolution equals the reference's bounded window):
@@ -45,8 +46,9 @@
 //     the inverse x pass fused with the output write (either layout).
 // FFTs are Stockham autosort, mixed radix 2/3/4/5/7/8/9, one block per batch of
 // lines staged in LDS; the twiddle table is FP64-built and rounded once.
-// The kernel spectra depend on (L0, L1, L2, w, sigma1, sigma2, power) only: built on the device (separable FP64 cosine/sine transforms of the
-// offset kernels) and cached per host thread and device.
+// The kernel spectra depend on (L0, L1, L2, w, sigma1, sigma2, power) only: built
+// on the device (separable FP64 cosine/sine transforms of the offset kernels) and
+// cached per host thread and device.
 #include "common.hpp"
 #include "vote3.hpp"
 #include "voxel_payload.hpp"
@@ -1806,9 +1808,9 @@ static bool spectral_serves(unsigned p, bool plate, unsigned samples) {
 // With `atv`: analytical tensor voting, whose features come from the input
 // tensors in the x pass only.
 bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsigned power, bool stick, bool plate,
-                        unsigned samples, bool atv) {
+                        unsigned samples, bool atv, bool payload) {
     const unsigned p = power < 1 || atv ? 1 : power;
-    const bool f64 = p > 1;
+    const bool f64 = p > 1 || payload;
     if (!atv && !spectral_serves(p, plate, samples)) return false;
     if (w < (p == 1 ? 5u : p < 4 ? 9u : 11u) || (size_t)s0 * s1 * s2 < 32768) return false;
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);
@@ -1816,7 +1818,7 @@ bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsig
     const size_t nf = (size_t)mono_count((int)p), nz = (nf + 1) / 2;  // the combined features
     const size_t W = 2 * (w / 2) + 1;
     const size_t h0 = L0 / 2 + 1, h1 = L1 / 2 + 1, h2 = L2 / 2 + 1;
-    // payloads: of the field, above power 1 padded for the window gather
+    // payloads: of the field, in FP64 padded for the window gather
     const size_t pay = !f64 ? (size_t)s0 * s1 * s2 : vote3_payload_voxels(s0, s1, s2, (unsigned)W);
     const size_t need = nz * (size_t)L0 * L1 * L2 * (f64 ? 16 : 8) + 6 * nf * h0 * h1 * h2 * (f64 ? 8 : 4) +
                         6 * nf * W * h1 * h2 * 8 + pay * 32;
@@ -1836,6 +1838,7 @@ static void launch_xfwd_pay(int power, unsigned grid, size_t lds, hipStream_t st
                             const SpecGeom& g, int B, int C, int FG, const FftPlan& pl, const double2* tw,
                             double2* Z) {
     switch (power) {
+        case 1: k_spec_xfwd_pay<1><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
         case 2: k_spec_xfwd_pay<2><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
         case 3: k_spec_xfwd_pay<3><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
         default: k_spec_xfwd_pay<4><<<grid, kFT, lds, st>>>(v.ps, v.pp, v.g, g, B, C, FG, pl, tw, Z, v.stop); break;
@@ -1967,7 +1970,7 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
         stick = plate = true;
         sigma2 = 0.0f;
         if (!tensors) return kSpectralNotApplicable;
-    } else if (!spectral_serves(p, plate, samples) || (p > 1) != (pay != nullptr)) {
+    } else if (!spectral_serves(p, plate, samples) || (p > 1 && !pay)) {
         return kSpectralNotApplicable;
     }
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);

@@ -24,7 +24,7 @@ void plate_polys(int P, double c1, double c2, std::vector<double>& al, std::vect
 int vote3_payload_flat(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        unsigned s0, unsigned s1, unsigned s2, float4* ps, float4* pp, hipStream_t st);
 bool spectral_preferred(unsigned s0, unsigned s1, unsigned s2, unsigned w, unsigned power, bool stick, bool plate,
-                        unsigned samples, bool atv = false);
+                        unsigned samples, bool atv = false, bool payload = false);
 // Eigenvalues of the voted field requested with the vote: the spectral vote
 // writes them from its last pass and sets `done`; otherwise the caller runs
 // eig3 on the field.
@@ -36,9 +36,16 @@ struct EigOut {
 };
 // Status of vote3_spectral_run when the request is outside the spectral method.
 constexpr int kSpectralNotApplicable = -1;
-// Voters of a spectral vote in FP64: the padded payloads of the window gather,
-// formed (and the voters looked over, see k_vote3_prep) before it. stop (device):
-// set where the gather has to vote instead; the vote then leaves `out` alone.
+// What the payload pass finds out about the voters of a spectral vote in FP64,
+// on the device. stop: set where the window gather has to vote instead (k_vote_gate).
+struct VoterStat {
+    unsigned long long stop;
+    unsigned dense;      // receiver tiles that the window gather serves the plates of (learned vote)
+    unsigned pad;
+    unsigned hist[256];  // voting voxels by the binary exponent of their scale
+};
+// Voters of a spectral vote in FP64: the padded payloads of the window gather.
+// Where *stop is set the vote leaves `out` alone.
 struct SpecPayload {
     const float4 *ps, *pp;
     VoteGeom g;
@@ -46,7 +53,7 @@ struct SpecPayload {
 };
 // Padded payload voxels of the window gather.
 size_t vote3_payload_voxels(unsigned s0, unsigned s1, unsigned s2, unsigned w);
-// pay: the vote in FP64; given above power 1 and only there.
+// pay: the vote in FP64 from these payloads; always given above power 1.
 int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0,
                        float* out, int out_layout, unsigned s0, unsigned s1, unsigned s2, float sigma1,
                        float sigma2, unsigned w, unsigned power, bool stick, bool plate, unsigned samples,
