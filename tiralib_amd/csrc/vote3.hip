@@ -595,68 +595,23 @@ __device__ __forceinline__ void plate_basis(const float n[3], float u[3], float 
     v[2] = n[0] * u[1] - n[1] * u[0];
 }
 
-// Voters that a spectral vote would spread beyond their window: not finite (the
-// scale itself is tested: of features formed from it, all can be NaN), or a
-// caller's stick that is not of unit length, which the features take: a length
-// off by 5e-7 changes a vote by as much as the window gather rounds it.
+// Voters that a spectral vote would spread beyond their window: not finite, of
+// a scale whose sums in the transforms could overflow (the scale itself is
+// tested: of features formed from it, all can be NaN), or a caller's stick that
+// is not of unit length, which the features take.
+constexpr float kWildScale = 1e30f;
 __device__ __forceinline__ bool wild_stick(const float4 S) {
     const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
-    return !(fabsf(S.w) <= 3e38f) || !(q2 < 1e30f) || (S.w != 0.0f && !(fabsf(q2 - 1.0f) < 1e-6f));
+    if (S.w == 0.0f) return !(q2 < kWildScale);
+    return !(fabsf(S.w) < kWildScale) || !(fabsf(q2 - 1.0f) < 2e-6f);
 }
-__device__ __forceinline__ bool wild_plate(const float4 N) {
-    return !(fabsf(N.w) <= 3e38f) || !(fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z)) < 2.0f);
+// alpha: the factor of the plate's features (sticknorm3).
+__device__ __forceinline__ bool wild_plate(const float4 N, float alpha) {
+    return !(fabsf(N.w * alpha) < kWildScale) || !(fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z)) < 2.0f);
 }
-
-// The voters a block of a payload pass has seen, for a spectral vote.
-struct StatBlock {
-    unsigned* h;  // LDS: 256 counts
-    bool wild = false;
-    __device__ __forceinline__ void begin() {
-        for (int i = (int)threadIdx.x; i < 256; i += (int)blockDim.x) h[i] = 0;
-        __syncthreads();
-    }
-    __device__ __forceinline__ void voter(float scale) {
-        if (scale > 0.0f) atomicAdd(&h[min(__float_as_uint(scale) >> 23, 255u)], 1u);
-    }
-    __device__ __forceinline__ void end(VoterStat* st) {
-        __syncthreads();
-        for (int i = (int)threadIdx.x; i < 256; i += (int)blockDim.x)
-            if (h[i]) atomicAdd(&st->hist[i], h[i]);
-        if (__any(wild) && (threadIdx.x & 63) == 0) st->stop = 1ull;  // equal stores do not queue up
-    }
-};
-
-// Whether the window gather has to vote after all (one wave): a wild voter
-// (already flagged), a range of scales beyond FP64's reach, or (ntile > 0) too
-// many tiles of dense plates.
-// The transforms' error at a receiver is at most about 4 x 2^-53 of the 2-norm F of
-// all scales (3e-16 measured), wherever its votes come from. Voters below
-// 2^-27 F would get less than seven digits of their votes; with more than one
-// voting voxel in 256 of those the field goes to the gather, whose rounding is
-// each receiver's own. A field of 2^24 equally strong voters has the line at
-// 3e-5 of their scale, one with a single voter of 1e6 among ones at 7e-3.
-__global__ __launch_bounds__(64) void k_vote_gate(VoterStat* __restrict__ st, unsigned ntile) {
-    const int lane = (int)threadIdx.x;
-    unsigned c[4], total = 0;
-    int top = 0;
-    for (int k = 0; k < 4; k++) {
-        c[k] = st->hist[4 * lane + k];
-        total += c[k];
-        if (c[k]) top = 4 * lane + k;
-    }
-    for (int d = 32; d; d >>= 1) top = max(top, __shfl_xor(top, d));
-    double e = 0.0;  // of scales up to 2^(bin + 1), in units of 2^top
-    for (int k = 0; k < 4; k++) e += 4.0 * c[k] * exp2(2.0 * (4 * lane + k - top));
-    for (int d = 32; d; d >>= 1) e += __shfl_xor(e, d);
-    const double line = 7.45058059692383e-09 * sqrt(e);  // 2^-27 F
-    unsigned faint = 0;
-    for (int k = 0; k < 4; k++)
-        if (exp2((double)(4 * lane + k - top)) < line) faint += c[k];
-    for (int d = 32; d; d >>= 1) {
-        total += __shfl_xor((int)total, d);
-        faint += __shfl_xor((int)faint, d);
-    }
-    if (lane == 0 && (faint > total / 256 || (ntile && st->dense > ntile / 8))) st->stop = 1ull;
+// Raises *flag if any lane's voters were wild (equal stores do not queue up).
+__device__ __forceinline__ void raise_wild(bool wild, unsigned long long* flag) {
+    if (flag && __any(wild) && (threadIdx.x & 63) == 0) *flag = 1ull;
 }
 
 // Writes the voter payload for one voxel given its eigen-decomposition.
