@@ -91,3 +91,19 @@ def test_bad_voter_stays_in_its_window(hip, nets, bad):
         assert np.isfinite(got[~inside]).all()
         # the sticks come from the window gather then, and from the spectral vote without the bad voter
         assert np.abs(got[~inside].astype(np.float64) - ref[~inside]).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("bright", [1e6, 1e12])
+def test_faint_sticks_beside_a_bright_one(hip, nets, bright):
+    """Receivers outside the window of a bright stick keep the votes of the faint
+    ones; a range beyond FP64 sends the sticks to the window gather."""
+    shape, w, at = (36, 40, 44), 9, (5, 6, 7)
+    f = _plates(shape, 0.03, seed=12)
+    f[..., 0] += 0.2 * (np.random.default_rng(1).random(shape) < 0.1)  # sticks along x
+    f[at] = bright * np.array([1, 0, 0, 0, 0, 0], np.float32)
+    a, b = nets[1.5]
+    got, ref = _vote(hip, a, f, w, True, hip.LAYOUT_PACKED6), _vote(hip, b, f, w, True, hip.LAYOUT_PACKED6)
+    far = np.ones(shape, bool)
+    far[tuple(slice(0, c + w // 2 + 1) for c in at)] = False
+    d = got[far].astype(np.float64) - ref[far]
+    assert np.linalg.norm(d) <= 5.6e-6 * np.linalg.norm(ref[far].astype(np.float64))

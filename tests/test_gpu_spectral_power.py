@@ -240,3 +240,21 @@ def test_spectral_power_is_closer_to_64_bits_than_the_gather(hip, oracle, power)
            for mode in (_lib.PLATE_AUTO, _lib.PLATE_CLOSED)]
     # voters and result in FP32, all between in FP64: a few roundings of 6e-8, averaged over the voters
     assert err[0] <= min(err[1], 1.2e-7)
+
+
+@pytest.mark.parametrize("power,w", [(2, 9), (4, 11)])
+@pytest.mark.parametrize("bright", [1e10, 1e12, 1e30, 3e37])
+def test_range_beyond_fp64_is_voted_by_window(hip, power, w, bright):
+    """A voter so bright that even FP64 transforms would cost the others digits:
+    the whole field is the window gather's, bit for bit."""
+    shape, at = (33, 34, 35), (4, 5, 6)
+    f = _field(shape, seed=8)
+    f[at] = bright * np.diag([1.0, 0.25, 0.0]).astype(np.float32).ravel()
+    got, _ = _run(f, shape, _lib.PLATE_AUTO, 1.5, 0.0, w, power)
+    ref, _ = _run(f, shape, _lib.PLATE_CLOSED, 1.5, 0.0, w, power)
+    np.testing.assert_array_equal(got, ref)
+    # scales all as large are no range: the spectral vote, and close to the gather
+    g = (_field(shape, seed=8) * np.float32(bright / 1e3)).astype(np.float32)
+    got, _ = _run(g, shape, _lib.PLATE_AUTO, 1.5, 0.0, w, power)
+    ref, _ = _run(g, shape, _lib.PLATE_CLOSED, 1.5, 0.0, w, power)
+    assert not np.array_equal(got, ref) and _rel(got, ref) <= 2e-6

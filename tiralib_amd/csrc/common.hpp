@@ -50,7 +50,7 @@ enum Slot {
     WS_NB2,  // the 2D neighbour table of the last stick/plate vote (kept while unchanged)
     WS_TABLE4,  // offset table of the tabulated-network vote
     WS_TABLE5,  // offset tables of the listed plate gather
-    WS_WILD,    // flag of a spectral vote that has to be voted by window
+    WS_WILD,    // voter statistics of a spectral vote in FP64
     WS_LIST,    // the listed gather's voter list, segment starts and tile flags
     WS_NSLOTS
 };

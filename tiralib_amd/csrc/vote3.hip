@@ -595,32 +595,85 @@ __device__ __forceinline__ void plate_basis(const float n[3], float u[3], float 
     v[2] = n[0] * u[1] - n[1] * u[0];
 }
 
-// Voters that a spectral vote would spread beyond their window: not finite, of
-// a scale whose sums in the transforms could overflow (the scale itself is
-// tested: of features formed from it, all can be NaN), or a caller's stick that
-// is not of unit length, which the features take.
-constexpr float kWildScale = 1e30f;
+// Voters that a spectral vote would spread beyond their window: not finite (the
+// scale itself is tested: of features formed from it, all can be NaN), or a
+// caller's stick that is not of unit length, which the features take: a length
+// off by 5e-7 changes a vote by as much as the window gather rounds it.
 __device__ __forceinline__ bool wild_stick(const float4 S) {
     const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
-    if (S.w == 0.0f) return !(q2 < kWildScale);
-    return !(fabsf(S.w) < kWildScale) || !(fabsf(q2 - 1.0f) < 2e-6f);
+    return !(fabsf(S.w) <= 3e38f) || !(q2 < 1e30f) || (S.w != 0.0f && !(fabsf(q2 - 1.0f) < 1e-6f));
 }
-// alpha: the factor of the plate's features (sticknorm3).
-__device__ __forceinline__ bool wild_plate(const float4 N, float alpha) {
-    return !(fabsf(N.w * alpha) < kWildScale) || !(fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z)) < 2.0f);
+__device__ __forceinline__ bool wild_plate(const float4 N) {
+    return !(fabsf(N.w) <= 3e38f) || !(fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z)) < 2.0f);
 }
-// Raises *flag if any lane's voters were wild (equal stores do not queue up).
-__device__ __forceinline__ void raise_wild(bool wild, unsigned long long* flag) {
-    if (flag && __any(wild) && (threadIdx.x & 63) == 0) *flag = 1ull;
+
+// The voters a block of a payload pass has seen, for a spectral vote.
+struct StatBlock {
+    unsigned* h;  // LDS: 256 counts
+    bool wild = false;
+    __device__ __forceinline__ void begin() {
+        for (int i = (int)threadIdx.x; i < 256; i += (int)blockDim.x) h[i] = 0;
+        __syncthreads();
+    }
+    // A voxel of eigenvalues up to `lam` that votes with `scale`; a scale that is
+    // rounding of its eigenvalues (an isotropic tensor) is no voter.
+    __device__ __forceinline__ void voter(float scale, float lam) {
+        if (scale > 1e-6f * lam) atomicAdd(&h[min(__float_as_uint(scale) >> 23, 255u)], 1u);
+    }
+    __device__ __forceinline__ void end(VoterStat* st) {
+        __syncthreads();
+        for (int i = (int)threadIdx.x; i < 256; i += (int)blockDim.x)
+            if (h[i]) atomicAdd(&st->hist[i], h[i]);
+        if (__any(wild) && (threadIdx.x & 63) == 0) st->stop = 1ull;  // equal stores do not queue up
+    }
+};
+
+// Whether the window gather has to vote after all (one wave): a wild voter
+// (already flagged), a range of scales beyond FP64's reach, or (ntile > 0) too
+// many tiles of dense plates.
+// The transforms' error at a receiver goes with the 2-norm F of all scales,
+// wherever they are: at most 8e-17 F of the largest vote of a unit voter (powers
+// 2 to 4, windows 9 to 21, 40 x 44 x 48 and 128 x 120 x 100). A voter of 2^-30 F
+// has 9e-8 of its votes there, no more than the window gather's rounding. Where
+// more than one voting voxel in 256 is fainter, the field goes to the gather.
+// A field of 2^24 equally strong voters has the line at 4e-6 of their scale, one
+// with a single voter of 1e6 among ones at 1e-3.
+__global__ __launch_bounds__(64) void k_vote_gate(VoterStat* __restrict__ st, unsigned ntile) {
+    const int lane = (int)threadIdx.x;
+    unsigned c[4], total = 0;
+    int top = 0;
+    for (int k = 0; k < 4; k++) {
+        c[k] = st->hist[4 * lane + k];
+        total += c[k];
+        if (c[k]) top = 4 * lane + k;
+    }
+    for (int d = 32; d; d >>= 1) top = max(top, __shfl_xor(top, d));
+    double e = 0.0;  // of scales up to 2^(bin + 1), in units of 2^top
+    for (int k = 0; k < 4; k++) e += 4.0 * c[k] * exp2(2.0 * (4 * lane + k - top));
+    for (int d = 32; d; d >>= 1) e += __shfl_xor(e, d);
+    const double line = 9.31322574615479e-10 * sqrt(e);  // 2^-30 F
+    unsigned faint = 0;
+    for (int k = 0; k < 4; k++)
+        if (exp2((double)(4 * lane + k - top)) < line) faint += c[k];
+    for (int d = 32; d; d >>= 1) {
+        total += __shfl_xor((int)total, d);
+        faint += __shfl_xor((int)faint, d);
+    }
+    if (lane == 0 && (faint > total / 256 || (ntile && st->dense > ntile / 8))) st->stop = 1ull;
 }
 
 // Writes the voter payload for one voxel given its eigen-decomposition.
 __device__ __forceinline__ void write_payload(const VoteGeom& g, size_t pidx, float l0, float l1, float l2,
                                               const float* e0, const float* e2, float4* pay_s, float4* pay_p,
-                                              float4* pay_v, float sum_inv_n, float alpha, bool& wild) {
+                                              float4* pay_v, float sum_inv_n, float alpha, VoterStat* stat,
+                                              StatBlock& sb) {
     float4 S, N;
     stick_plate_payload(l0, l1, l2, e0, e2, S, N);
-    wild = wild || (pay_s && wild_stick(S)) || (pay_p && wild_plate(N, alpha));
+    if (stat) {
+        sb.wild = sb.wild || (pay_s && wild_stick(S)) || (pay_p && wild_plate(N));
+        sb.voter(fmaxf(pay_s ? fabsf(S.w) : 0.0f, pay_p ? fminf(fabsf(N.w) * alpha, 3e38f) : 0.0f),
+                 fmaxf(fabsf(l2), fmaxf(fabsf(l1), fabsf(l0))));
+    }
     if (pay_s) pay_s[pidx] = S;
     if (pay_p) {
         if (!pay_v) {
@@ -636,13 +689,15 @@ __device__ __forceinline__ void write_payload(const VoteGeom& g, size_t pidx, fl
 }
 
 // Grid-stride over the padded payload volume: voxels outside the field get a
-// zero payload. wild (optional): raised if a voter is such that a spectral vote
-// cannot serve (wild_stick, wild_plate).
+// zero payload. stat (optional): what a spectral vote has to know of the voters;
+// alpha: the factor of its plates (sticknorm3).
 __global__ __launch_bounds__(256) void k_vote3_prep(const float* __restrict__ in, int layout, VoteGeom g,
                                                     float4* __restrict__ pay_s, float4* __restrict__ pay_p,
                                                     float4* __restrict__ pay_v, float sum_inv_n,
-                                                    float alpha, unsigned long long* __restrict__ wild) {
-    bool odd = false;
+                                                    float alpha, VoterStat* __restrict__ stat) {
+    __shared__ unsigned s_hist[256];
+    StatBlock sb{s_hist};
+    if (stat) sb.begin();
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
@@ -657,9 +712,10 @@ __global__ __launch_bounds__(256) void k_vote3_prep(const float* __restrict__ in
         const size_t v = ((size_t)z * g.s1 + y) * g.s2 + x;
         float l0, l1, l2, e0[3], e2[3];
         voxel_eig(in, layout, v, l0, l1, l2, e0, e2);
-        write_payload(g, p, l0, l1, l2, e0, e2, pay_s, pay_p, pay_v, sum_inv_n, alpha, odd);
+        write_payload(g, p, l0, l1, l2, e0, e2, pay_s, pay_p, pay_v, sum_inv_n, alpha, stat,
+                      sb);
     }
-    raise_wild(odd, wild);
+    if (stat) sb.end(stat);
 }
 
 // Payload from caller eigenpairs (_tensorvote3_tk inputs).
@@ -667,8 +723,10 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
                                                        const float* __restrict__ ev0, VoteGeom g,
                                                        float4* __restrict__ pay_s, float4* __restrict__ pay_p,
                                                        float4* __restrict__ pay_v, float sum_inv_n,
-                                                       float alpha, unsigned long long* __restrict__ wild) {
-    bool odd = false;
+                                                       float alpha, VoterStat* __restrict__ stat) {
+    __shared__ unsigned s_hist[256];
+    StatBlock sb{s_hist};
+    if (stat) sb.begin();
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
@@ -684,9 +742,10 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
         const float z3[3] = {0, 0, 0};
         const float* e2 = ev2 ? ev2 + v * 3 : z3;
         const float* e0 = ev0 ? ev0 + v * 3 : z3;
-        write_payload(g, p, lam[v * 3], lam[v * 3 + 1], lam[v * 3 + 2], e0, e2, pay_s, pay_p, pay_v, sum_inv_n, alpha, odd);
+        write_payload(g, p, lam[v * 3], lam[v * 3 + 1], lam[v * 3 + 2], e0, e2, pay_s, pay_p, pay_v, sum_inv_n, alpha, stat,
+                      sb);
     }
-    raise_wild(odd, wild);
+    if (stat) sb.end(stat);
 }
 
 // ---------------------------------------------------------------- learned plate (MLP)
@@ -696,18 +755,20 @@ __global__ __launch_bounds__(256) void k_vote3_prep_tk(const float* __restrict__
 // surrogate's error check -- their plate votes come from the integrator (the
 // closed form of the N-sample sum). Without pay_u (the tabulated network)
 // a flagged voter gets plate scale 0 in pay_n and its (n, scale) in pay_f,
-// which is zero for every other voter. wild (optional): raised if there is a
-// stick that a spectral vote cannot serve (wild_stick).
+// which is zero for every other voter. stat (optional): what a spectral vote of
+// the sticks has to know of them.
 __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict__ in, int layout, VoteGeom g,
                                                         float4* __restrict__ pay_s, float4* __restrict__ pay_n,
                                                         float4* __restrict__ pay_u, float4* __restrict__ pay_f,
                                                         const float* __restrict__ bin_err, float tol,
                                                         unsigned long long* __restrict__ n_fallback,
-                                                        unsigned long long* __restrict__ wild) {
+                                                        VoterStat* __restrict__ stat) {
+    __shared__ unsigned s_hist[256];
+    StatBlock sb{s_hist};
+    if (stat) sb.begin();
     const size_t total = (size_t)g.P0 * g.P1 * g.P2;
     const float4 zero = make_float4(0, 0, 0, 0);
     unsigned nf = 0;
-    bool odd = false;
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < total; p += (size_t)gridDim.x * blockDim.x) {
         const int px = (int)(p % g.P2), py = (int)((p / g.P2) % g.P1), pz = (int)(p / ((size_t)g.P1 * g.P2));
         const int x = px - g.r, y = py - g.r, z = pz - g.r;
@@ -724,7 +785,11 @@ __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict_
         const float ss = copysignf(fabsf(l2) - fabsf(l1), l2);
         const float4 S = make_float4(e2[0], e2[1], e2[2], ss);
         if (pay_s) pay_s[p] = S;
-        odd = odd || wild_stick(S);
+        if (stat) {
+            sb.wild = sb.wild || wild_stick(S);
+            // (the plate counts as well: what a stick far below it adds is no digit of their votes)
+            sb.voter(fmaxf(fabsf(ss), fabsf(fabsf(l1) - fabsf(l0))), fmaxf(fabsf(l2), fmaxf(fabsf(l1), fabsf(l0))));
+        }
         float n[3] = {e0[0], e0[1], e0[2]};
         const float nn = n[0] * n[0] + n[1] * n[1] + n[2] * n[2];
         float sp = copysignf(fabsf(l1) - fabsf(l0), l1);
@@ -745,7 +810,7 @@ __global__ __launch_bounds__(256) void k_vote3_prep_mlp(const float* __restrict_
         }
     }
     if (n_fallback && nf) atomicAdd(n_fallback, (unsigned long long)nf);
-    raise_wild(odd, wild);
+    if (stat) sb.end(stat);
 }
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -1343,6 +1408,19 @@ static void launch_closed(bool stick, bool plate, unsigned grid, hipStream_t st,
     else k_vote3_closed_lds<P, false, true, kBZ><<<grid, kThreads, sh, st>>>(ps, pp, tab, g, out, layout);
 }
 
+// Zeroed voter statistics of a spectral vote.
+static int voter_stat(VoterStat** stat, hipStream_t st) {
+    TH_TRY(ws_get(WS_WILD, sizeof(VoterStat), (void**)stat));
+    k_fill_zero<<<1, 256, 0, st>>>((float*)*stat, sizeof(VoterStat) / 4);
+    TH_HIP(hipGetLastError());
+    return TIRA_OK;
+}
+// Blocks of a payload pass over n voxels: one voxel per thread, or (with
+// statistics, which every block adds to the device's) eight blocks per CU.
+static unsigned prep_grid(size_t n, bool stat) {
+    return (unsigned)std::min<size_t>(ceil_div(n, 256), stat ? (size_t)8 * cu_count() : 65536);
+}
+
 // Runs the vote on device buffers. `eig_in`: tensors (layout) or NULL when
 // lam/ev2/ev0 eigenpairs are given.
 int vote3_run(const float* tensors, int in_layout, const float* lam, const float* ev2, const float* ev0, float* out,
@@ -1391,18 +1469,14 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     const unsigned nsamp = samples == 0 ? p + 2 : samples;  // samples == 0 (analytic) equals the exact integral
     if (sum) TH_TRY(ws_get(WS_SCRATCH0, ptotal * 16, (void**)&pv));
     const float inv_n = sum ? 1.0f / (float)nsamp : 1.0f;
-    unsigned long long* gate = nullptr;
-    float alpha = 1.0f;
-    if (spectral) {
-        TH_TRY(ws_get(WS_WILD, 8, (void**)&gate));
-        k_fill_zero<<<1, 64, 0, st>>>((float*)gate, 2);
-        alpha = sticknorm3_host(sigma1, sigma2, p);
-    }
-    const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), 65536);
+    VoterStat* stat = nullptr;
+    if (spectral) TH_TRY(voter_stat(&stat, st));
+    const float alpha = spectral ? sticknorm3_host(sigma1, sigma2, p) : 1.0f;
+    const unsigned pgrid = prep_grid(ptotal, stat != nullptr);
     {
         ProfScope prof("vote3_prep", st);
-        if (tensors) k_vote3_prep<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, pv, inv_n, alpha, gate);
-        else k_vote3_prep_tk<<<pgrid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, pv, inv_n, alpha, gate);
+        if (tensors) k_vote3_prep<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pp, pv, inv_n, alpha, stat);
+        else k_vote3_prep_tk<<<pgrid, 256, 0, st>>>(lam, ev2, ev0, g, ps, pp, pv, inv_n, alpha, stat);
     }
     TH_HIP(hipGetLastError());
 
@@ -1414,7 +1488,10 @@ int vote3_run(const float* tensors, int in_layout, const float* lam, const float
     char* dtab = nullptr;
     float2* dcs = nullptr;
     TH_TRY(table_for(key, P, st, &dtab, &dcs));
+    const unsigned long long* gate = nullptr;
     if (spectral) {
+        gate = &stat->stop;
+        k_vote_gate<<<1, 64, 0, st>>>(stat, 0u);
         const SpecPayload pay{ps, pp, g, gate};
         const int rc = vote3_spectral_run(tensors, in_layout, lam, ev2, ev0, out, out_layout, s0, s1, s2, sigma1, sigma2,
                                           w, power, stick, plate, samples, false, st, nullptr, &pay);
@@ -1632,17 +1709,23 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
     if (stick) TH_TRY(ws_get(WS_PAY0, ptotal * 16, (void**)&ps));
     TH_TRY(ws_get(WS_PAY1, ptotal * 16, (void**)&pn));
     TH_TRY(ws_get(WS_PAY2, ptotal * 16, table ? (void**)&pf : (void**)&pu));
-    unsigned long long* cnt = nullptr;  // voters of the fallback, voters whose stick must stay local
+    unsigned long long* cnt = nullptr;  // voters of the fallback
     if (n_fallback || table) {
-        TH_TRY(ws_get(WS_COUNTER, 16, (void**)&cnt));
-        k_fill_zero<<<1, 64, 0, st>>>((float*)cnt, 4);
+        TH_TRY(ws_get(WS_COUNTER, 8, (void**)&cnt));
+        k_fill_zero<<<1, 64, 0, st>>>((float*)cnt, 2);
     }
-    const unsigned pgrid = (unsigned)std::min<size_t>(ceil_div(ptotal, 256), 65536);
+    // The sticks as a spectral vote (spectral_run64), where it serves them. It
+    // leaves the window gather 36 of its 57 VALU instructions per pair, and the
+    // plates can take the listed gather; both add to its output.
+    bool spectral = table && stick &&
+                    spectral_preferred(s0, s1, s2, w, m->power, true, false, 0, false, true);
+    VoterStat* stat = nullptr;
+    if (spectral) TH_TRY(voter_stat(&stat, st));
+    const unsigned pgrid = prep_grid(ptotal, stat != nullptr);
     {
         ProfScope prof("vote3_prep_mlp", st);
         k_vote3_prep_mlp<<<pgrid, 256, 0, st>>>(tensors, in_layout, g, ps, pn, pu, pf,
-                                                table ? m->bin_err + kMlpBins : m->bin_err, tol, cnt,
-                                                table ? cnt + 1 : nullptr);
+                                                table ? m->bin_err + kMlpBins : m->bin_err, tol, cnt, stat);
     }
     TH_HIP(hipGetLastError());
     const TableKey key{0, (int)w, m->sigma1, m->sigma2, m->power, 0u};
@@ -1657,14 +1740,9 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
         const size_t lds = (size_t)(w / 2 + 1) * 2 * kMlpTabPad * sizeof(float4);
         const float4* vt = m->vtab;
         const int nr = m->vtab_rows;
-        // The sticks, where the spectral vote serves them: they leave the
-        // window gather 36 of its 57 VALU instructions per pair, and the plates
-        // can then take the listed gather. Both add to the spectral output, which is
-        // FP64 up to there (spectral_run64). A stick that is not finite stays within
-        // its window: the gather votes the sticks if any voter is such.
-        bool spectral = false;
-        if (stick && spectral_preferred(s0, s1, s2, w, m->power, true, false, 0, false, true)) {
-            const SpecPayload pay{ps, nullptr, g, cnt + 1};
+        if (spectral) {
+            k_vote_gate<<<1, 64, 0, st>>>(stat, 0u);
+            const SpecPayload pay{ps, nullptr, g, &stat->stop};
             const int rc = vote3_spectral_run(tensors, in_layout, nullptr, nullptr, nullptr, out, out_layout, s0, s1, s2,
                                               m->sigma1, m->sigma2, w, m->power, true, false, 0, false, st, nullptr,
                                               &pay);
@@ -1674,10 +1752,10 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
         if (spectral) {
             ProfScope prof("vote3_mlp_wild", st);
             switch (P) {
-                case 1: k_vote3_closed<1, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
-                case 2: k_vote3_closed<2, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
-                case 3: k_vote3_closed<3, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
-                default: k_vote3_closed<4, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, cnt + 1, 0); break;
+                case 1: k_vote3_closed<1, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
+                case 2: k_vote3_closed<2, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
+                case 3: k_vote3_closed<3, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
+                default: k_vote3_closed<4, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
             }
             TH_HIP(hipGetLastError());
         }

@@ -36,9 +36,16 @@ struct EigOut {
 };
 // Status of vote3_spectral_run when the request is outside the spectral method.
 constexpr int kSpectralNotApplicable = -1;
-// Voters of a spectral vote in FP64: the padded payloads of the window gather,
-// formed (and the voters looked over, see k_vote3_prep) before it. stop (device):
-// set where the gather has to vote instead; the vote then leaves `out` alone.
+// What the payload pass finds out about the voters of a spectral vote in FP64,
+// on the device. stop: set where the window gather has to vote instead (k_vote_gate).
+struct VoterStat {
+    unsigned long long stop;
+    unsigned dense;      // receiver tiles that the window gather serves the plates of (learned vote)
+    unsigned pad;
+    unsigned hist[256];  // voting voxels by the binary exponent of their scale
+};
+// Voters of a spectral vote in FP64: the padded payloads of the window gather.
+// Where *stop is set the vote leaves `out` alone.
 struct SpecPayload {
     const float4 *ps, *pp;
     VoteGeom g;
