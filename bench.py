@@ -382,7 +382,7 @@ def bench_config4(steps, warmup, cpu_seconds=None, log=None):
     st.synchronize()
     call("tira_hip_profile_end")
     prof = _lib.profile_get
-    stages = {k: prof(k)[0] for k in ("vote3_prep_mlp", *SPECTRAL_KERNELS, "vote3_mlp_wild", "plate_sparse",
+    stages = {k: prof(k)[0] for k in ("vote3_prep_mlp", *SPECTRAL_KERNELS, "vote3_mlp_wild", "plate_list", "plate_sparse",
                                       "vote3_mlptab", "vote3_mlp_fallback")}
     nfall = net.vote(vol, outs["mlp"], shape, w, stick=True, tol=tol, in_layout=_lib.LAYOUT_PACKED6,
                      count_fallback=True)
@@ -476,7 +476,7 @@ def bench_pipeline(net=None, log=None):
         if mode == _lib.VOTE_SPECTRAL:
             vote_stages = list(SPECTRAL_KERNELS)
         elif mode == _lib.PLATE_MLP:
-            vote_stages = [*SPECTRAL_KERNELS, "vote3_mlp_wild", "plate_sparse", "vote3_mlptab", "vote3_mlp_fallback"]
+            vote_stages = [*SPECTRAL_KERNELS, "vote3_mlp_wild", "plate_list", "plate_sparse", "vote3_mlptab", "vote3_mlp_fallback"]
         else:
             vote_stages = ["vote3_closed"]
         prep_name = "vote3_prep_mlp" if mode == _lib.PLATE_MLP else "vote3_prep"

@@ -93,10 +93,31 @@ def test_bad_voter_stays_in_its_window(hip, nets, bad):
         assert np.abs(got[~inside].astype(np.float64) - ref[~inside]).max() <= 1e-5 * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("w,density", [(9, 1.0), (9, 0.05), (13, 1.0), (7, 0.05)])
+def test_sticks_of_the_learned_vote(hip, nets, w, density):
+    """Sticks and plates of fields that the density and the window send to the spectral
+    vote with listed or windowed plates (w >= 13, or few plates) or to one window
+    gather (bit for bit the caller's table's, which never lists): the same votes."""
+    shape = (34, 40, 70)
+    f = _plates(shape, density, seed=3)
+    rng = np.random.default_rng(4)
+    q = rng.normal(size=shape + (3,))
+    q /= np.linalg.norm(q, axis=-1, keepdims=True)
+    on = (rng.random(shape) < 0.1)[..., None]
+    x, y, z = q[..., 0], q[..., 1], q[..., 2]
+    f = f + np.where(on, np.stack([x * x, x * y, x * z, y * y, y * z, z * z], -1), 0).astype(np.float32)
+    a, b = nets[2.0 if w == 13 else 1.5]
+    got, ref = _vote(hip, a, f, w, True, hip.LAYOUT_PACKED6), _vote(hip, b, f, w, True, hip.LAYOUT_PACKED6)
+    if w < 9 or (w < 13 and density == 1.0):
+        np.testing.assert_array_equal(got, ref)
+    # w^3 FP32 terms in either order, as test_listed_plates_equal_window_gather
+    assert np.linalg.norm(got.astype(np.float64) - ref) <= 5.6e-6 * np.linalg.norm(ref.astype(np.float64))
+
+
 @pytest.mark.parametrize("bright", [1e6, 1e12])
 def test_faint_sticks_beside_a_bright_one(hip, nets, bright):
     """Receivers outside the window of a bright stick keep the votes of the faint
-    ones; a range beyond FP64 sends the sticks to the window gather."""
+    ones; a range beyond FP64 sends sticks and plates to the window gather."""
     shape, w, at = (36, 40, 44), 9, (5, 6, 7)
     f = _plates(shape, 0.03, seed=12)
     f[..., 0] += 0.2 * (np.random.default_rng(1).random(shape) < 0.1)  # sticks along x
@@ -107,3 +128,5 @@ def test_faint_sticks_beside_a_bright_one(hip, nets, bright):
     far[tuple(slice(0, c + w // 2 + 1) for c in at)] = False
     d = got[far].astype(np.float64) - ref[far]
     assert np.linalg.norm(d) <= 5.6e-6 * np.linalg.norm(ref[far].astype(np.float64))
+    if bright == 1e12:
+        np.testing.assert_array_equal(got, ref)

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void k_plate_list(const float4* __restrict__ p
 // a window pair.
 __global__ __launch_bounds__(256) void k_plate_tiles(VoteGeom g, int bz, const unsigned* __restrict__ cnt,
                                                      const unsigned* __restrict__ tot, float ratio,
-                                                     unsigned char* __restrict__ sparse) {
+                                                     unsigned char* __restrict__ sparse, unsigned* __restrict__ dense) {
     const unsigned t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     const unsigned nt = g.nbx * g.nby * g.nbz;
     if (t >= nt) return;
@@ -97,7 +97,9 @@ __global__ __launch_bounds__(256) void k_plate_tiles(VoteGeom g, int bz, const u
     if (lane == 0) {
         const float box = (float)(xhi - xlo + 1) * 64.0f * (float)(4 + 2 * g.r) * (float)(bz + 2 * g.r);
         const float wc = (float)(2 * g.r + kCube), ww = (float)(2 * g.r + 1);
-        sparse[t] = (float)c * wc * wc * wc * ratio < box * ww * ww * ww ? 1 : 0;
+        const bool few = (float)c * wc * wc * wc * ratio < box * ww * ww * ww;
+        sparse[t] = few ? 1 : 0;
+        if (dense && !few) atomicAdd(dense, 1u);
     }
 }
 
@@ -159,7 +161,8 @@ __global__ __launch_bounds__(kSparseThreads) void k_plate_sparse(
     const unsigned* __restrict__ tot, const float4* __restrict__ ent, const int* __restrict__ entrow,
     const float4* __restrict__ vtab, const int* __restrict__ rows, int nrows, VoteGeom g, int bz,
     const unsigned char* __restrict__ sparse, unsigned* __restrict__ next, float* __restrict__ out, int layout,
-    int accumulate) {
+    int accumulate, const unsigned long long* __restrict__ stop) {
+    if (stop && *stop) return;
     extern __shared__ float4 s_tab[];
     for (int i = (int)threadIdx.x; i < nrows * kSparseCells; i += kSparseThreads) {
         const int slot = i / kSparseCells, p = i - slot * kSparseCells;
@@ -318,47 +321,52 @@ static int sparse_tables(int w, float s1, int vtab_rows, hipStream_t st, float4*
 // at w = 13 (0.47).
 constexpr float kSparseRatio = 1.45f;
 
-int plate_sparse_run(const float4* pay, const float4* vtab, int vtab_rows, float sigma1, const VoteGeom& g, int bz,
-                     float* out, int layout, bool accumulate, hipStream_t st, const unsigned char** tiles) {
-    *tiles = nullptr;
+int plate_list_build(const float4* pay, int vtab_rows, float sigma1, const VoteGeom& g, int bz, unsigned* dense,
+                     hipStream_t st, PlateList* list, bool* ok) {
+    *ok = false;
     const size_t n = (size_t)g.s0 * g.s1 * g.s2;
     if (n >= (size_t)1 << 31 || g.s1 > 65535 || g.s2 > 65535) return TIRA_OK;
-    const int w = 2 * g.r + 1;
-    float4* ent = nullptr;
-    int *entrow = nullptr, *rows = nullptr, nrows = 0;
-    TH_TRY(sparse_tables(w, sigma1, vtab_rows, st, &ent, &entrow, &rows, &nrows));
-    if (nrows > (int)plate_sparse_max_rows()) return TIRA_OK;
     const unsigned nseg = g.nbx * (unsigned)g.s0 * (unsigned)g.s1, ntile = g.nbx * g.nby * g.nbz;
     const unsigned nscan = (nseg + 1 + kScanSegs - 1) / kScanSegs;
     const size_t lv_b = n * 16, lp_b = n * 8, cnt_b = ((size_t)nseg + 1) * 4, tot_b = (size_t)nscan * 4;
     auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
     char* buf = nullptr;
-    const int rc = ws_get(WS_LIST, up(lv_b) + up(lp_b) + up(cnt_b) + up(tot_b) + 256 + ntile, (void**)&buf);
-    if (rc == TIRA_ERR_OUT_OF_MEMORY) {  // the window gather needs no list
+    PlateList& L = *list;
+    int rc = sparse_tables(2 * g.r + 1, sigma1, vtab_rows, st, &L.ent, &L.entrow, &L.rows, &L.nrows);
+    if (rc == TIRA_OK && L.nrows > (int)plate_sparse_max_rows()) return TIRA_OK;
+    if (rc == TIRA_OK) rc = ws_get(WS_LIST, up(lv_b) + up(lp_b) + up(cnt_b) + up(tot_b) + 256 + ntile, (void**)&buf);
+    if (rc == TIRA_ERR_OUT_OF_MEMORY) {  // the window gather needs neither
         (void)hipGetLastError();
         return TIRA_OK;
     }
     TH_TRY(rc);
-    float4* lv = (float4*)buf;
-    uint2* lp = (uint2*)(buf + up(lv_b));
-    unsigned* cnt = (unsigned*)(buf + up(lv_b) + up(lp_b));
-    unsigned* tot = (unsigned*)((char*)cnt + up(cnt_b));
-    unsigned* next = (unsigned*)((char*)tot + up(tot_b));
-    unsigned char* flags = (unsigned char*)next + 256;
+    L.lv = (float4*)buf;
+    L.lp = (uint2*)(buf + up(lv_b));
+    L.cnt = (unsigned*)(buf + up(lv_b) + up(lp_b));
+    L.tot = (unsigned*)((char*)L.cnt + up(cnt_b));
+    L.next = (unsigned*)((char*)L.tot + up(tot_b));
+    L.sparse = (unsigned char*)L.next + 256;
+    ProfScope prof("plate_list", st);
+    k_plate_count<<<nseg / 4 + 1, 256, 0, st>>>(pay, g, nseg, L.cnt);
+    k_seg_scan<<<nscan, 256, 0, st>>>(L.cnt, nseg + 1, L.tot);
+    k_seg_scan_top<<<1, 1024, 0, st>>>(L.tot, nscan, L.next);
+    k_plate_list<<<ceil_div(nseg, 4), 256, 0, st>>>(pay, g, nseg, L.cnt, L.tot, L.lv, L.lp);
+    k_plate_tiles<<<ceil_div(ntile, 4), 256, 0, st>>>(g, bz, L.cnt, L.tot, kSparseRatio, L.sparse, dense);
+    TH_HIP(hipGetLastError());
+    *ok = true;
+    return TIRA_OK;
+}
+
+int plate_sparse_gather(const PlateList& L, const float4* vtab, const VoteGeom& g, int bz, float* out, int layout,
+                        bool accumulate, const unsigned long long* stop, hipStream_t st) {
     ProfScope prof("plate_sparse", st);
-    k_plate_count<<<nseg / 4 + 1, 256, 0, st>>>(pay, g, nseg, cnt);
-    k_seg_scan<<<nscan, 256, 0, st>>>(cnt, nseg + 1, tot);
-    k_seg_scan_top<<<1, 1024, 0, st>>>(tot, nscan, next);
-    k_plate_list<<<ceil_div(nseg, 4), 256, 0, st>>>(pay, g, nseg, cnt, tot, lv, lp);
-    k_plate_tiles<<<ceil_div(ntile, 4), 256, 0, st>>>(g, bz, cnt, tot, kSparseRatio, flags);
-    const size_t lds = (size_t)nrows * kSparseCells * sizeof(float4);
+    const size_t lds = (size_t)L.nrows * kSparseCells * sizeof(float4);
     TH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_plate_sparse), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)kSparseLds));
-    k_plate_sparse<<<(unsigned)cu_count(), kSparseThreads, lds, st>>>(lv, lp, cnt, tot, ent, entrow, vtab, rows, nrows,
-                                                                      g, bz, flags, next, out, layout,
-                                                                      accumulate ? 1 : 0);
+    k_plate_sparse<<<(unsigned)cu_count(), kSparseThreads, lds, st>>>(L.lv, L.lp, L.cnt, L.tot, L.ent, L.entrow, vtab,
+                                                                      L.rows, L.nrows, g, bz, L.sparse, L.next, out,
+                                                                      layout, accumulate ? 1 : 0, stop);
     TH_HIP(hipGetLastError());
-    *tiles = flags;
     return TIRA_OK;
 }
 

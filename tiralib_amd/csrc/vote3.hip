@@ -1040,14 +1040,17 @@ __global__ __launch_bounds__(kThreads) void k_vote3_mlp(const float4* __restrict
 // kMlpTabStride floats per offset (build_mlptab_table). Voters flagged by the
 // error check carry plate scale 0 here; their plates come from the
 // integrator's pass. listed (optional): tiles with a nonzero flag are left to
-// the listed gather (plate_sparse.hip); accumulate: add the votes to `out`.
+// the listed gather (plate_sparse.hip); accumulate: add the votes to `out`; gate
+// (optional): the launch votes where *gate is set (gate_on) or where it is not.
 template <int P, bool STICK, int BZ>
 __global__ __launch_bounds__(kThreads) void k_vote3_mlptab(const float4* __restrict__ pay_s,
                                                            const float4* __restrict__ pay_p,
                                                            const float* __restrict__ tab,
                                                            const float4* __restrict__ vtab, int nrows,
                                                            VoteGeom g, float* __restrict__ out, int out_layout,
-                                                           const unsigned char* __restrict__ listed, int accumulate) {
+                                                           const unsigned char* __restrict__ listed, int accumulate,
+                                                           const unsigned long long* __restrict__ gate, int gate_on) {
+    if (gate && (*gate != 0ull) != (gate_on != 0)) return;
     constexpr int STRIDE = kMlpTabStride;
     constexpr int C1PI = 8, ROW = 9;
     constexpr int CELLS2 = 2 * kMlpTabPad;  // float4 per staged row
@@ -1672,17 +1675,28 @@ static int mlptab_lds_attr(size_t lds) {
 template <int P>
 static int launch_mlptab(bool stick, unsigned grid, size_t lds, hipStream_t st, const float4* ps, const float4* pn,
                          const float* t, const float4* vt, int nrows, const VoteGeom& g, float* out, int layout,
-                         const unsigned char* listed, bool accumulate) {
-    const int acc = accumulate ? 1 : 0;
+                         const unsigned char* listed, bool accumulate, const unsigned long long* gate, bool gate_on) {
+    const int acc = accumulate ? 1 : 0, on = gate_on ? 1 : 0;
     if (stick) {
         TH_TRY((mlptab_lds_attr<P, true>(lds)));
-        k_vote3_mlptab<P, true, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout, listed, acc);
+        k_vote3_mlptab<P, true, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout, listed, acc, gate, on);
     } else {
         TH_TRY((mlptab_lds_attr<P, false>(lds)));
-        k_vote3_mlptab<P, false, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout, listed, acc);
+        k_vote3_mlptab<P, false, kBZMlp><<<grid, kThreads, lds, st>>>(ps, pn, t, vt, nrows, g, out, layout, listed, acc, gate, on);
     }
     return TIRA_OK;
 }
+
+// Windows from which the sticks go through the spectral vote: at w = 9 it takes
+// 341 us for the window gather's 1548 (32^3 curved sheets), 1378 for 2223 (128^3);
+// at w = 7 1009 for 774 at 64^3 and 1317 for 1159 at 128^3.
+constexpr unsigned kMlpSpectralW = 9;
+// Windows from which it does so whatever the plates: fields whose plates are too
+// dense for the list (128^3 random plates) take 6.3 ms for the window gather of
+// stick and plate's 7.1 at w = 13 and 39.7 for 46.8 at w = 25, but 4.5 for 4.2 at
+// w = 11 and 3.1 for 2.3 at w = 9. Below, such fields (more than an eighth of the
+// tiles) stay with the window gather.
+constexpr unsigned kMlpDenseW = 13;
 
 // Stick + learned plate vote on device buffers with the network `m` (trained
 // for its sigma1, sigma2 and power). Voters whose orientation bin's error
@@ -1717,7 +1731,7 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
     // The sticks as a spectral vote (spectral_run64), where it serves them. It
     // leaves the window gather 36 of its 57 VALU instructions per pair, and the
     // plates can take the listed gather; both add to its output.
-    bool spectral = table && stick &&
+    bool spectral = table && stick && w >= kMlpSpectralW &&
                     spectral_preferred(s0, s1, s2, w, m->power, true, false, 0, false, true);
     VoterStat* stat = nullptr;
     if (spectral) TH_TRY(voter_stat(&stat, st));
@@ -1740,36 +1754,41 @@ int vote3_mlp_run(PlateMlp* m, const float* tensors, int in_layout, float* out, 
         const size_t lds = (size_t)(w / 2 + 1) * 2 * kMlpTabPad * sizeof(float4);
         const float4* vt = m->vtab;
         const int nr = m->vtab_rows;
+        // the plates' voters as a list, where it serves them (a caller's table: never)
+        PlateList list;
+        bool listed = false;
+        if ((!stick || spectral) && !m->vtab_custom)
+            TH_TRY(plate_list_build(pn, nr, m->sigma1, g, kBZMlp, stat ? &stat->dense : nullptr, st, &list, &listed));
+        const unsigned long long* gate = nullptr;
+        if (spectral && !listed && w < kMlpDenseW) spectral = false;
         if (spectral) {
-            k_vote_gate<<<1, 64, 0, st>>>(stat, 0u);
+            k_vote_gate<<<1, 64, 0, st>>>(stat, w < kMlpDenseW ? g.nbx * g.nby * g.nbz : 0u);
             const SpecPayload pay{ps, nullptr, g, &stat->stop};
             const int rc = vote3_spectral_run(tensors, in_layout, nullptr, nullptr, nullptr, out, out_layout, s0, s1, s2,
                                               m->sigma1, m->sigma2, w, m->power, true, false, 0, false, st, nullptr,
                                               &pay);
             if (rc != TIRA_OK && rc != kSpectralNotApplicable) return rc;
             spectral = rc == TIRA_OK;
+            if (spectral) gate = &stat->stop;
         }
-        if (spectral) {
-            ProfScope prof("vote3_mlp_wild", st);
+        if (stick && !spectral) listed = false;
+        if (listed)
+            TH_TRY(plate_sparse_gather(list, vt, g, kBZMlp, out, out_layout, spectral, gate, st));
+        const unsigned char* tiles = listed ? list.sparse : nullptr;
+        // the window gather: sticks and plates of all tiles, or (after a spectral
+        // vote) the plates of the tiles that are not listed, and sticks and plates
+        // of all where that vote stood back
+        for (int full = 0; full < 2; full++) {
+            const bool fs = full != 0;  // sticks too
+            if (fs ? !stick : stick && !spectral) continue;
+            const unsigned char* tl = fs ? nullptr : tiles;
+            const bool add = !fs && spectral;
+            ProfScope prof(fs && spectral ? "vote3_mlp_wild" : "vote3_mlptab", st);
             switch (P) {
-                case 1: k_vote3_closed<1, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
-                case 2: k_vote3_closed<2, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
-                case 3: k_vote3_closed<3, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
-                default: k_vote3_closed<4, true, false, kBZMlp><<<grid, kThreads, 0, st>>>(ps, nullptr, ct, g, out, out_layout, &stat->stop, 0); break;
-            }
-            TH_HIP(hipGetLastError());
-        }
-        const bool gather_stick = stick && !spectral;
-        const unsigned char* listed = nullptr;
-        if (!gather_stick && !m->vtab_custom)
-            TH_TRY(plate_sparse_run(pn, vt, nr, m->sigma1, g, kBZMlp, out, out_layout, spectral, st, &listed));
-        {
-            ProfScope prof("vote3_mlptab", st);
-            switch (P) {
-                case 1: TH_TRY(launch_mlptab<1>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
-                case 2: TH_TRY(launch_mlptab<2>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
-                case 3: TH_TRY(launch_mlptab<3>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
-                default: TH_TRY(launch_mlptab<4>(gather_stick, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, listed, spectral)); break;
+                case 1: TH_TRY(launch_mlptab<1>(fs, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, tl, add, gate, fs)); break;
+                case 2: TH_TRY(launch_mlptab<2>(fs, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, tl, add, gate, fs)); break;
+                case 3: TH_TRY(launch_mlptab<3>(fs, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, tl, add, gate, fs)); break;
+                default: TH_TRY(launch_mlptab<4>(fs, grid, lds, st, ps, pn, mt, vt, nr, g, out, out_layout, tl, add, gate, fs)); break;
             }
         }
         TH_HIP(hipGetLastError());
