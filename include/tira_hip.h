@@ -267,7 +267,9 @@ int tira_tensorvote3_atv_method_async(const float* input_field, int in_layout, f
  * normal e0 (when plate)) such that the pair vote of tensorvote.h:1183-1213 /
  * 1651-1695 (normalised by sticknorm3 and pi, plate exact) at offset d equals
  * sum_f K[c,f](d) * scale * monomial_f. Host computation, FP64, no GPU; out
- * holds 6 * nf * (2(w/2)+1)^3 doubles; *nf_out receives nf. power must be 1. */
+ * holds 6 * nf * (2(w/2)+1)^3 doubles; *nf_out receives nf. power must be 1. The
+ * stick features come from the fit that the votes run on the device; the plate's
+ * by themselves serve the test of the map that folds them into the stick's. */
 int tira_spectral_offset_kernels(unsigned w, float sigma1, float sigma2, unsigned power, int stick, int plate,
                                  double* out, unsigned* nf_out);
 /* The same for analytical tensor voting (tensorvote.h:688-760, attenuation

@@ -1387,10 +1387,39 @@ __host__ __device__ static inline void atv_vote64(const double e0[3], const doub
     sym_add(V, 2.0 * K2, v, e2);
 }
 
-// The offset kernels of the combined features on the device: coefficients of
-// the stick vote (ATV: of its e2 part) of every offset, K[c nf + f][dw][dv][du],
-// from its values at the fit points Q by the projector P (nf x npts). One
-// thread per (offset, feature); the votes are evaluated again by each feature,
+// Fit points of a power's monomials.
+static int fit_count(int power) { return std::max(32, 3 * mono_count(power)); }
+
+// Direction d, distance rho (1, or 0 at the voter itself) and attenuations of an offset.
+__host__ __device__ static inline void offset_geometry64(int du, int dv, int dw, double s1, double s2, double d[3],
+                                                         double& rho, double& c1, double& c2) {
+    const double l2 = (double)du * du + (double)dv * dv + (double)dw * dw;
+    d[0] = d[1] = d[2] = 0.0;
+    if (l2 > 0) { const double L = sqrt(l2); d[0] = du / L; d[1] = dv / L; d[2] = dw / L; }
+    rho = l2 > 0 ? 1.0 : 0.0;
+    c1 = s1 > 0 ? exp(-l2 / (s1 * s1)) : (l2 > 0 ? 0.0 : 1.0);
+    c2 = s2 > 0 ? exp(-l2 / (s2 * s2)) : (l2 > 0 ? 0.0 : 1.0);
+}
+
+// Coefficients (six components) of one feature of the stick vote (ATV: of its e2
+// part) at one offset: the vote at the npts fit points Q, projected by the
+// feature's row P.
+__host__ __device__ static inline void fit_offset(int du, int dv, int dw, double s1, double s2, int power, bool atv,
+                                                  double sn, const double* Q, const double* P, int npts, double acc[6]) {
+    const double zero[3] = {0.0, 0.0, 0.0};
+    double d[3], rho, c1, c2;
+    offset_geometry64(du, dv, dw, s1, s2, d, rho, c1, c2);
+    for (int c = 0; c < 6; c++) acc[c] = 0.0;
+    for (int k = 0; k < npts; k++) {
+        double V[6];
+        if (atv) atv_vote64(zero, Q + 3 * k, d, rho, c1, 1.0, 0.0, 0.0, V);
+        else stick_vote64(Q + 3 * k, d, c1, c2, sn, V, power);
+        for (int c = 0; c < 6; c++) acc[c] = fma(P[k], V[c], acc[c]);
+    }
+}
+
+// The offset kernels of the combined features on the device, K[c nf + f][dw][dv][du].
+// One thread per (offset, feature); the votes are evaluated again by each feature,
 // which costs less than keeping them. 2197 offsets of the 15 quartic features:
 // 18 us, 29 us for the 28 of power 2 (the same sums are 1.7e8 FMA for the 66 of
 // power 4 at w = 13, 1.2e9 at w = 25: seconds on the host).
@@ -1403,26 +1432,15 @@ __global__ __launch_bounds__(256) void k_offset_kernels(int r, double s1, double
     const int f = (int)(i / noff);
     const size_t o = i - (size_t)f * noff;
     const int du = (int)(o % W) - r, dv = (int)((o / W) % W) - r, dw = (int)(o / ((size_t)W * W)) - r;
-    const double l2 = (double)du * du + (double)dv * dv + (double)dw * dw;
-    double d[3] = {0.0, 0.0, 0.0};
-    if (l2 > 0) { const double L = sqrt(l2); d[0] = du / L; d[1] = dv / L; d[2] = dw / L; }
-    const double c1 = s1 > 0 ? exp(-l2 / (s1 * s1)) : (l2 > 0 ? 0.0 : 1.0);
-    const double c2 = s2 > 0 ? exp(-l2 / (s2 * s2)) : (l2 > 0 ? 0.0 : 1.0);
-    const double zero[3] = {0.0, 0.0, 0.0};
-    double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = 0; k < npts; k++) {
-        double V[6];
-        if (atv) atv_vote64(zero, Q + 3 * k, d, l2 > 0 ? 1.0 : 0.0, c1, 1.0, 0.0, 0.0, V);
-        else stick_vote64(Q + 3 * k, d, c1, c2, sn, V, power);
-        const double p = P[(size_t)f * npts + k];
-        for (int c = 0; c < 6; c++) acc[c] = fma(p, V[c], acc[c]);
-    }
+    double acc[6];
+    fit_offset(du, dv, dw, s1, s2, power, atv != 0, sn, Q, P + (size_t)f * npts, npts, acc);
     for (int c = 0; c < 6; c++) K[((size_t)c * nf + f) * noff + o] = acc[c];
 }
 
-// K[ch][dw][dv][du], ch = c * nf + f (see tira_spectral_offset_kernels), on the host. With
-// `atv`, the features are s1 m(e2) (15), s2 m(e0) (15) and s3 (1), the window
-// half-width w / 2 and the attenuation exp(-|d|^2 / s1^2) of ATV.
+// K[ch][dw][dv][du] of power 1, ch = c * nf + f (see tira_spectral_offset_kernels),
+// on the host, for tests: the stick features (ATV: s1 m(e2), 15) from fit_offset,
+// as every vote has them, and beside them the plate's (ATV: s2 m(e0), 15, and s3,
+// 1) by themselves, which the votes fold into the first.
 static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate, bool atv, std::vector<double>& K,
                           int& nf) {
     const int r = (int)(w / 2), W = 2 * r + 1;
@@ -1431,7 +1449,7 @@ static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate
         s2 = 0.0f;
     }
     nf = (stick ? kMono : 0) + (plate ? kMono : 0) + (atv ? 1 : 0);
-    const int npts = 32;
+    const int npts = fit_count(1);
     std::vector<double> Q, P;
     fit_points(Q, npts);
     if (!fit_projector(Q, npts, P)) {
@@ -1441,18 +1459,23 @@ static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate
     const double sn = 1.0 / (double)sticknorm3_host(s1, s2, 1);
     const size_t noff = (size_t)W * W * W;
     K.assign((size_t)6 * nf * noff, 0.0);
-    std::vector<double> al, be, ga, de, Vs((size_t)npts * 6), Vp((size_t)npts * 6);
+    std::vector<double> al, be, ga, de, Vp((size_t)npts * 6);
     size_t o = 0;
     for (int dw = -r; dw <= r; dw++)
         for (int dv = -r; dv <= r; dv++)
             for (int du = -r; du <= r; du++, o++) {
-                const double l2 = (double)du * du + (double)dv * dv + (double)dw * dw;
-                double d[3] = {0.0, 0.0, 0.0};
-                if (l2 > 0) { const double L = std::sqrt(l2); d[0] = du / L; d[1] = dv / L; d[2] = dw / L; }
-                const double c1 = s1 > 0 ? std::exp(-l2 / ((double)s1 * s1)) : (l2 > 0 ? 0.0 : 1.0);
-                const double c2 = s2 > 0 ? std::exp(-l2 / ((double)s2 * s2)) : (l2 > 0 ? 0.0 : 1.0);
-                if (plate && !atv) {
-                    if (l2 == 0) {
+                if (stick)
+                    for (int m = 0; m < kMono; m++) {
+                        double acc[6];
+                        fit_offset(du, dv, dw, s1, s2, 1, atv, sn, Q.data(), &P[(size_t)m * npts], npts, acc);
+                        for (int c = 0; c < 6; c++) K[((size_t)c * nf + m) * noff + o] = acc[c];
+                    }
+                if (!plate) continue;
+                double d[3], rho, c1, c2;
+                offset_geometry64(du, dv, dw, s1, s2, d, rho, c1, c2);
+                const double zero[3] = {0.0, 0.0, 0.0};
+                if (!atv) {
+                    if (rho == 0.0) {
                         al.assign(2, 0.0); be.assign(2, 0.0); ga.assign(2, 0.0); de.assign(3, 0.0);
                         al[0] = 0.5 * M_PI * c1;
                         be[0] = -0.5 * M_PI * c1;
@@ -1460,33 +1483,22 @@ static int offset_kernels(unsigned w, float s1, float s2, bool stick, bool plate
                         plate_polys(1, c1, c2, al, be, ga, de);
                     }
                 }
-                const double zero[3] = {0.0, 0.0, 0.0};
-                const double rho = l2 > 0 ? 1.0 : 0.0;
                 for (int i = 0; i < npts; i++) {
-                    if (atv) {
-                        atv_vote64(zero, &Q[i * 3], d, rho, c1, 1.0, 0.0, 0.0, &Vs[(size_t)i * 6]);
-                        atv_vote64(&Q[i * 3], zero, d, rho, c1, 0.0, 1.0, 0.0, &Vp[(size_t)i * 6]);
-                        continue;
-                    }
-                    if (stick) stick_vote64(&Q[i * 3], d, c1, c2, sn, &Vs[(size_t)i * 6]);
-                    if (plate) plate_vote64(&Q[i * 3], d, l2 == 0, al, be, ga, de, &Vp[(size_t)i * 6]);
+                    if (atv) atv_vote64(&Q[i * 3], zero, d, rho, c1, 0.0, 1.0, 0.0, &Vp[(size_t)i * 6]);
+                    else plate_vote64(&Q[i * 3], d, rho == 0.0, al, be, ga, de, &Vp[(size_t)i * 6]);
                 }
                 if (atv) {  // the ball weight s3: a constant kernel
                     double V3[6];
                     atv_vote64(zero, zero, d, rho, c1, 0.0, 0.0, 1.0, V3);
                     for (int c = 0; c < 6; c++) K[((size_t)c * nf + 2 * kMono) * noff + o] = V3[c];
                 }
-                for (int kind = 0; kind < 2; kind++) {
-                    if ((kind == 0 && !stick) || (kind == 1 && !plate)) continue;
-                    const std::vector<double>& V = kind == 0 ? Vs : Vp;
-                    const int f0 = (kind == 1 && stick) ? kMono : 0;
-                    for (int m = 0; m < kMono; m++)
-                        for (int c = 0; c < 6; c++) {
-                            double acc = 0.0;
-                            for (int i = 0; i < npts; i++) acc += P[(size_t)m * npts + i] * V[(size_t)i * 6 + c];
-                            K[((size_t)c * nf + f0 + m) * noff + o] = acc;
-                        }
-                }
+                const int f0 = stick ? kMono : 0;
+                for (int m = 0; m < kMono; m++)
+                    for (int c = 0; c < 6; c++) {
+                        double acc = 0.0;
+                        for (int i = 0; i < npts; i++) acc += P[(size_t)m * npts + i] * Vp[(size_t)i * 6 + c];
+                        K[((size_t)c * nf + f0 + m) * noff + o] = acc;
+                    }
             }
     return TIRA_OK;
 }
@@ -1643,7 +1655,7 @@ static int spectra_for(const SpecKey& key, const SpecGeom& g, hipStream_t st, co
     // and the ATV's e0 and constant parts, are linear maps of it and fold into
     // the features), parities and trig tables
     const int w = 2 * (key.w / 2) + 1, r = key.w / 2, nf = g.nf;
-    const int nch = 6 * nf, npts = std::max(32, 3 * nf);
+    const int nch = 6 * nf, npts = fit_count(key.power);
     std::vector<double> Q, P;
     fit_points(Q, npts);
     if (!fit_projector(Q, npts, P, key.power)) {
@@ -2097,7 +2109,7 @@ extern "C" {
 int tira_spectral_offset_kernels(unsigned w, float sigma1, float sigma2, unsigned power, int stick, int plate,
                                  double* out, unsigned* nf_out) {
     TH_ARG(out, "NULL pointer");
-    TH_ARG(power == 1, "the spectral vote serves power 1 only");
+    TH_ARG(power == 1, "the offset kernels are exported for power 1 only");
     TH_ARG(stick || plate, "neither stick nor plate");
     TH_ARG(sigma1 >= 0.0f && sigma2 >= 0.0f, "sigmas must be >= 0");
     std::vector<double> K;
