@@ -119,3 +119,21 @@ def test_vote_scale_at_high_powers(hip, oracle, share, s1, s2, p):
         for got in (s.tensorvote_tk(s1, s2, p, w=w, plate=False), tvk.tensorvote_tk(f, s1, s2, p, w=w, plate=False)):
             scale = ((got.astype(np.float64) - ref) * ref).sum() / (ref * ref).sum()
             assert abs(scale) <= (1.3e-7 if s2 == 0.0 else 2.5e-7), scale
+
+
+@pytest.mark.parametrize("share", [0.19, 0.21, 0.39, 0.41])
+def test_share_and_window_pick_the_gather(hip, share):
+    """Around the shares and the window at which a session changes over: narrow and
+    wide windows in turn on one session, against the module's window gather; where
+    the window gather serves them too, to an ulp of a vote with its table."""
+    f = _field((90, 110), share, 21)
+    with tvk.Session(f) as s:
+        for k, (s1, s2, p) in enumerate([(3.0, 0.0, 1), (4.0, 0.0, 2), (3.5, 1.0, 3), (3.0, 0.0, 1), (8.0, 2.0, 4)]):
+            w = 2 * int(3 * max(s1, s2)) + 1
+            got, ref = s.tensorvote_tk(s1, s2, p), tvk.tensorvote_tk(f, s1, s2, p)
+            _close(got, ref, w * w)
+            if share > 0.4 or (share > 0.2 and w < 25):
+                nb = api.build_neighbors2d(w, s1, s2, p, 20)
+                one = s.tensorvote_tk_prebuilt(nb.tobytes(), nb.size, w, s1, s2, p)
+                # the device's table may differ from the host's by an ulp in c1, c2
+                assert np.abs(got - one).max() <= 1.2e-7 * np.abs(one).max()

@@ -790,6 +790,16 @@ struct SessionTable {
     unsigned long long used = 0;
 };
 
+// Shares of the pixels up to which a vote takes the listed gather: windows from
+// kListedWideW on, and smaller ones, whose few pairs the window gather reads along
+// rows. Listed over window gather, random voters, device time: at 640 x 640
+// 0.65, 0.72, 0.92, 1.17, 1.38 for shares 0.05, 0.1, 0.2, 0.3, 0.39 at w = 7;
+// 0.41, 0.53, 0.76, 1.01, 1.25 at w = 13; 0.28, 0.40, 0.64, 0.88, 1.11 at w = 19;
+// 0.12 .. 0.73 at w = 49, 0.08 .. 0.56 at w = 151. Smaller images lie below that
+// (0.90 at most at 256 x 256, w = 7; 0.96 at w = 19; 0.81 at w = 49).
+constexpr double kListedShare = 0.4, kListedShareNarrow = 0.2;
+constexpr int kListedWideW = 25;
+
 // One graph of the session: its nodes take new arguments before each launch.
 struct SessionGraph {
     hipGraph_t graph = nullptr;
@@ -810,6 +820,7 @@ struct Vote2Session {
     size_t part_cap = 0;
     SessionGraph dense, listed;  // the window gather; the listed gather of a field of few voters
     char* list = nullptr;        // its voter list (NULL: the window gather serves every vote)
+    bool few = false;            // few enough voters for the listed gather at any window
     float4* lv = nullptr;
     unsigned *lp = nullptr, *lcnt = nullptr, *ltot = nullptr;
     unsigned long long clock = 0, replays = 0, table_hits = 0, table_builds = 0;
@@ -869,7 +880,7 @@ static int session_table(Vote2Session& s, const Nb2* nb, int nbc, int w, float s
         t.grid = nullptr;
     }
     t.used = 0;
-    if (built && nbc > 0 && s.list) {  // the listed gather reads its table as a grid
+    if (built && nbc > 0 && s.list && (s.few || w >= kListedWideW)) {  // the listed gather reads its table as a grid
         const size_t cells = (size_t)grid2_edge(w) * grid2_edge(w);
         TH_HIP(hipMalloc((void**)&t.grid, 2 * cells * sizeof(float4)));
         k_build_grid2<<<ceil_div(cells, 256), 256, 0, stream()>>>(w, s1, s2, power, samples, stick ? 1 : 0, plate ? 1 : 0,
@@ -967,13 +978,6 @@ static int session_build_graph(Vote2Session& s, SessionGraph& g, SessionArgs& a,
     return TIRA_OK;
 }
 
-// Share of the pixels up to which the listed gather is the cheaper: with 40% of
-// 256 x 256 pixels voting it takes 1.21 ms for the window gather's 2.09 at
-// (sigma1, sigma2, power) = (25, 8, 30), 0.59 for 0.91 at (17, 5, 15), 0.16 for
-// 0.20 at (8, 2, 3) and 0.067 for 0.062 at (3, 0, 1); all voting 2.45 for 2.14,
-// 1.07 for 0.92, 0.26 for 0.20 and 0.083 for 0.062.
-constexpr double kListedShare = 0.4;
-
 // Lists the field's voters when they are few: payload of unit stick norm,
 // counts, the total (read back), then the list. Leaves s.list NULL otherwise.
 static int session_list(Vote2Session& s) {
@@ -1001,7 +1005,9 @@ static int session_list(Vote2Session& s) {
     TH_HIP(hipMemcpyAsync(&end[0], s.lcnt + nseg, 4, hipMemcpyDeviceToHost, st));
     TH_HIP(hipMemcpyAsync(&end[1], s.ltot + nseg / kScanSegs, 4, hipMemcpyDeviceToHost, st));
     TH_HIP(hipStreamSynchronize(st));
-    if ((size_t)end[0] + end[1] > most) {
+    const size_t voters = (size_t)end[0] + end[1];
+    s.few = voters <= (size_t)(kListedShareNarrow * (double)s.n);
+    if (voters > most) {
         TH_HIP(hipFree(s.list));
         s.list = nullptr;
         return TIRA_OK;
