@@ -978,7 +978,8 @@ __global__ __launch_bounds__(kFT, 4) void k_spec_xfwd(const float4* __restrict__
 
 // The same in FP64 from the padded voter payloads of the window gather (vg):
 // they are formed before this vote, with the FP64 re-solve of close pairs, and
-// serve the gather too where it has to vote instead (*stop is set).
+// serve the gather too where it has to vote instead (*stop is set). Power 1 has
+// sticks only (the learned vote's).
 template <int P>
 __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restrict__ ps, const float4* __restrict__ pp,
                                                           VoteGeom vg, SpecGeom g, int B, int C, int FG, FftPlan pl,
@@ -1010,9 +1011,9 @@ __global__ __launch_bounds__(kFT, 2) void k_spec_xfwd_pay(const float4* __restri
             const int row = row0 + b, z = fdiv(row, g.n1, rn1), y = row - z * g.n1;
             const size_t v = ((size_t)(z + vg.r) * vg.P1 + y + vg.r) * vg.P2 + e + vg.r;
             const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const float4 S = g.stick ? ps[v] : zero, N = g.plate ? pp[v] : zero;
+            const float4 S = g.stick ? ps[v] : zero, N = P > 1 && g.plate ? pp[v] : zero;
             double A[(NF + 2) & ~1];
-            voter_features<P>(S, N, (double)g.alpha, g.stick != 0, g.plate != 0, A);
+            voter_features<P>(S, N, (double)g.alpha, g.stick != 0, P > 1 && g.plate != 0, A);
             if (NF & 1) A[NF] = 0.0;
 #pragma unroll
             for (int j = 0; j < (NF + 1) / 2; j++)
@@ -1916,7 +1917,13 @@ static int xinv_rows(size_t nrows, int Bmax) {
 // payload and the FP32 result. The transforms of FP32 round by the norm of the
 // whole field, the window gather by that of a receiver's own window: beside
 // bright voters the votes of faint ones kept 3 digits where the gather kept 6
-// (7e-4 of a receiver's vote down to 1e-4 of the largest, gather 2e-6).
+// (7e-4 of a receiver's vote down to 1e-4 of the largest, gather 2e-6; 2e-7 here).
+// Twice the bytes of FP32: at 91 x 117 x 101, power 2, w = 13 the forward y and z
+// passes take 146 us each (3.9 TB/s), the product 134 (4.5 TB/s), the inverse ones
+// 33 each, the whole vote 690 (FP32 390, window gather 4830). The x passes have two
+// waves per SIMD (248 VGPRs, of the radix-27 stage: without it, or bound to three
+// waves, they were 10 to 20% slower) and are bound by their LDS stages: 123 us
+// forward (2.5 TB/s), 32 inverse; the learned vote's sticks at 256^3 1.2 and 0.6 ms.
 static int spectral_run64(const SpecGeom& g, const FftPlan& p0, const FftPlan& p1, const FftPlan& p2, const SpecKey& key,
                           const SpecPayload& pay, float* out, int out_layout, hipStream_t st) {
     double2* Z = nullptr;
@@ -1982,7 +1989,7 @@ int vote3_spectral_run(const float* tensors, int in_layout, const float* lam, co
         stick = plate = true;
         sigma2 = 0.0f;
         if (!tensors) return kSpectralNotApplicable;
-    } else if (!spectral_serves(p, plate, samples) || (p > 1 && !pay)) {
+    } else if (!spectral_serves(p, plate, samples) || (p > 1 && !pay) || (p == 1 && pay && plate)) {
         return kSpectralNotApplicable;
     }
     const unsigned L0 = spectral_length(s0, w), L1 = spectral_length(s1, w), L2 = spectral_length(s2, w);
