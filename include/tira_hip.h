@@ -56,9 +56,10 @@ typedef enum tira_status {
 #define TIRA_PLATE_SUM     1   /* literal N-sample Riemann sum, the reference's algorithm, any N */
 #define TIRA_PLATE_CLOSED  2   /* closed form of the same integral (exact for N >= p+2 and for samples == 0) */
 #define TIRA_PLATE_MLP     3   /* learned surrogate with per-voxel integrator fallback: served by tira_tensorvote3_mlp */
-#define TIRA_VOTE_SPECTRAL 4   /* stick + exact (closed-form) plate vote as an FFT convolution (above power 1
-                                  where TIRA_PLATE_AUTO takes it): power 1 and
-                                  samples == 0 or >= 3; other requests take the direct gather (AUTO) */
+#define TIRA_VOTE_SPECTRAL 4   /* stick + exact (closed-form) plate vote as an FFT convolution: power 1 with
+                                  samples == 0 or >= 3 (FP32; rounding relative to the norm of the field),
+                                  powers 2 to 4 where TIRA_PLATE_AUTO takes it (FP64); other requests take
+                                  the direct gather (AUTO) */
 
 /* eig3 flags */
 #define TIRA_EIG_REFINE_FP64   1u  /* FP64 re-solve of voxels with relative eigengap < 1e-4 */

@@ -150,12 +150,12 @@ __device__ __forceinline__ void listed_pair(Acc& a, float3& hd, float nx, float 
 // The listed gather. Persistent blocks, one per CU: 130 KB of LDS hold the
 // rows of the network table (values at x_j; a lookup interpolates between two
 // neighbouring cells), every wave takes cubes from a counter until none is
-// left. VALU-bound: 57 instructions per (cube, voter), 85% of the issue slots
+// left. VALU-bound: 58 instructions per (cube, voter), 84% of the issue slots
 // in use, 71% of the lanes inside the window at w = 25 (a 4 x 4 x 8 box on two
 // receivers per lane would have 62%). 256^3 curved sheets with 2% plate noise,
 // w = 25: 27 ms (30 ms with the entry addresses in vector arithmetic and the
 // prefetched entry copied), where the window gather of stick and plate took
-// 285 ms; the sticks take 3.2 ms as a spectral vote.
+// 285 ms; the sticks take 5.9 ms as a spectral vote in FP64.
 __global__ __launch_bounds__(kSparseThreads) void k_plate_sparse(
     const float4* __restrict__ lv, const uint2* __restrict__ lp, const unsigned* __restrict__ cnt,
     const unsigned* __restrict__ tot, const float4* __restrict__ ent, const int* __restrict__ entrow,
