@@ -31,6 +31,11 @@ ARCH = "gfx950"
 # -amdgpu-mfma-vgpr-form: MFMA results in VGPRs, so the BF16 network's
 # activations feed the next layer without v_accvgpr_read copies.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form"]
+# Host functions and loops start on a cache line, so that their speed does not
+# hang on the size of what the linker puts before them: creating and freeing a
+# network (host generator of its weights) took 0.47 or 0.73 ms from one build
+# to the next with the same source; aligned 0.47 ms in four link orders.
+HOST_FLAGS = ["-Xarch_host", "-falign-functions=64", "-Xarch_host", "-falign-loops=64"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", f"-I{INCLUDE}", f"-I{CSRC}",
           "-Wall", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-unknown-pragmas",
           "-Wno-unused-command-line-argument"]
@@ -47,9 +52,9 @@ def _run(cmd):
 
 def _compile(src):
     obj = os.path.join(BUILD_DIR, os.path.basename(src) + ".o")
-    cmd = [HIPCC, *COMMON, *DEVICE_FLAGS, "-c", src, "-o", obj]
+    cmd = [HIPCC, *COMMON, *HOST_FLAGS, *DEVICE_FLAGS, "-c", src, "-o", obj]
     if src.endswith(".cpp"):
-        cmd = [HIPCC, *COMMON, "-x", "hip", *DEVICE_FLAGS, "-c", src, "-o", obj]
+        cmd = [HIPCC, *COMMON, "-x", "hip", *HOST_FLAGS, *DEVICE_FLAGS, "-c", src, "-o", obj]
     return obj, _run(cmd)
 
 
