@@ -170,6 +170,26 @@ def test_wild_eigenvalue_is_voted_by_window(hip, power, bad):
         assert np.abs(got[~inside].astype(np.float64) - clean[~inside]).max() <= 1e-5 * np.abs(clean[~inside]).max()
 
 
+@pytest.mark.parametrize("power", [2, 3, 4])
+@pytest.mark.parametrize("length", [1e20, 3e38, 1e-7])
+def test_plate_of_a_normal_beyond_range(hip, power, length):
+    """A caller's normal whose squared length leaves FP32 becomes the zero vector, which
+    has no circle of directions to vote along: its plate stays within its window."""
+    shape, w, at = (32, 34, 36), 11, (15, 16, 17)
+    n, i = int(np.prod(shape)), np.ravel_multi_index(at, shape)
+    rng = np.random.default_rng(power)
+    e0 = np.ascontiguousarray(np.linalg.qr(rng.normal(size=(n, 3, 3)))[0][:, :, 1], np.float32)
+    lam = np.sort(rng.random((n, 3)), axis=1).astype(np.float32)
+    lam[i] = 0
+    inside = np.zeros(shape, bool)
+    inside[tuple(slice(c - w // 2, c + w // 2 + 1) for c in at)] = True
+    clean = api.tensorvote3_tk(lam, None, e0, shape, 1.5, 0.0, power, w, False, True, 20).reshape(shape + (9,))
+    lam[i], e0[i] = (0.0, 1.0, 1.0), (0.0, length, 0.0)
+    got = api.tensorvote3_tk(lam, None, e0, shape, 1.5, 0.0, power, w, False, True, 20).reshape(shape + (9,))
+    assert np.isfinite(got[~inside]).all()
+    assert np.abs(got[~inside].astype(np.float64) - clean[~inside]).max() <= 1e-5 * np.abs(clean[~inside]).max()
+
+
 @pytest.mark.parametrize("wild", [False, True])
 @pytest.mark.parametrize("power", [2, 4])
 def test_input_may_lie_in_the_output(hip, power, wild):

@@ -598,13 +598,16 @@ __device__ __forceinline__ void plate_basis(const float n[3], float u[3], float 
 // Voters that a spectral vote would spread beyond their window: not finite (the
 // scale itself is tested: of features formed from it, all can be NaN), or a
 // caller's stick that is not of unit length, which the features take: a length
-// off by 5e-7 changes a vote by as much as the window gather rounds it.
+// off by 5e-7 changes a vote by as much as the window gather rounds it. A plate's
+// normal is of unit length or, where a caller's left the range of FP32 squared,
+// zero or not finite: such a plate has no circle of directions.
 __device__ __forceinline__ bool wild_stick(const float4 S) {
     const float q2 = fmaf(S.x, S.x, fmaf(S.y, S.y, S.z * S.z));
     return !(fabsf(S.w) <= 3e38f) || !(q2 < 1e30f) || (S.w != 0.0f && !(fabsf(q2 - 1.0f) < 1e-6f));
 }
 __device__ __forceinline__ bool wild_plate(const float4 N) {
-    return !(fabsf(N.w) <= 3e38f) || !(fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z)) < 2.0f);
+    const float q2 = fmaf(N.x, N.x, fmaf(N.y, N.y, N.z * N.z));
+    return !(fabsf(N.w) <= 3e38f) || !(q2 < 2.0f) || (N.w != 0.0f && !(q2 > 0.5f));
 }
 
 // The voters a block of a payload pass has seen, for a spectral vote.
